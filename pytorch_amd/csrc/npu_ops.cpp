@@ -434,6 +434,14 @@ Tensor as_matrix(const Tensor &t)
     return (row_major || col_major) ? t : t.contiguous();
 }
 
+// Rows of a K that is a multiple of 16 which start off a 16-byte boundary (a view cut out of a wider tensor): copied once, since
+// the matrix kernels load 16 bytes at a time.  (Any other K is padded inside the C ABI.)
+Tensor aligned_rows(const Tensor &t, int64_t K)
+{
+    const bool off = (t.stride(0) & 15) != 0 || (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) != 0;
+    return off && (K & 15) == 0 && K >= 128 ? t.clone(at::MemoryFormat::Contiguous) : t;
+}
+
 // int32 words of eight int4 values along the last dimension -> int8 of eight times that last dimension
 // (contiguous result; the input is made contiguous first if its rows are not)
 Tensor unpack_int4_rows(const Tensor &t)
@@ -506,7 +514,9 @@ Tensor quant_matmul_hip(const Tensor &x1, const Tensor &x2, const Tensor &scale,
     int64_t row0 = 0;
     for (auto &job : jobs) {
         Tensor a = job.first.stride(1) == 1 && job.first.stride(0) >= p.K ? job.first : job.first.contiguous();
+        a = aligned_rows(a, p.K);
         Tensor w = as_matrix(job.second);
+        if (w.stride(0) == 1) w = aligned_rows(w.t(), p.K).t();
         const int64_t m = a.size(0);
         Tensor ws;
         const size_t ws_bytes = mi355_quant_matmul_workspace(m, p.N, p.K, w.stride(0), w.stride(1));

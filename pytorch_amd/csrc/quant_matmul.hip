@@ -146,8 +146,13 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     // roles (one refills activations, one weights): wn = 0, 1, 0, 1, 1, 0, 1, 0 for wavefronts 0 .. 7.
     const int wm = LOOP == 1 || LOOP == 2 ? ((wave & 3) >> 1) + 2 * (wave >> 2) : wave / WGN;
     const int wn = LOOP == 1 || LOOP == 2 ? ((wave >> 2) ^ wave) & 1 : wave % WGN;
-    const int kt0 = (int)((int64_t)(p.K / BK) * chunk / p.S);            // first K step of this workgroup
-    const int KT = (int)((int64_t)(p.K / BK) * (chunk + 1) / p.S) - kt0;  // its number of K steps
+    // K steps of this workgroup.  A K that is not a multiple of 128 ends in a partial step: the activations of the missing
+    // bytes are loaded as zeros (kbytes below), so what the weight rows hold there (the next row, or padding) does not
+    // matter.  The wide loop, whose loads take scalar offsets only, runs the whole steps and leaves the partial one to tail_step.
+    const int ksteps = WIDE ? p.K / BK : (p.K + BK - 1) / BK;
+    const int kt0 = (int)((int64_t)ksteps * chunk / p.S);                 // first K step of this workgroup
+    const int KT = (int)((int64_t)ksteps * (chunk + 1) / p.S) - kt0;      // its number of K steps
+    const int kbytes = min(KT * BK, p.K - kt0 * BK);                      // bytes of K in them
 
     // Global -> LDS addressing.  Lane l of a unit fills LDS slot l (16 B): row l/8, chunk slot l%8,
     // which must hold global chunk (l%8) ^ (l/8) of that row (XOR swizzle).
@@ -166,9 +171,9 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
 
     // Loads are never skipped, so that the number of outstanding loads at every point of the loop is a
     // compile-time constant; a K step past the end gets an out-of-range lane offset instead (no memory traffic).
-    auto issue_a = [&](int kt, int KT) {
+    auto issue_a = [&](int kt) {
         char *slot = lds + (kt % NSA) * A_BYTES;
-        const uint32_t vo = kt < KT ? voff_a : kOutOfRange;
+        const uint32_t vo = kt * BK + gchunk < kbytes ? voff_a : kOutOfRange;
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             const int u = i * NW + wave;
@@ -254,6 +259,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             st.sbase = (uint32_t)u0 * unit_stride_a + (uint32_t)kt0 * BK;
             st.dst0 = (uint32_t)u0 * 1024u;
             wide::k_loop<WTN, 0, LOOP - 1>(acc, lds, st);
+            if (p.K % BK != 0 && chunk == p.S - 1) wide::tail_step<WTN, 0>(acc, lds, st, p.K % BK, lane);
         } else {
             const int u0 = wm * G::LBW;                                   // a quarter of the weight rows
             st.rsrc = rsrc_b;
@@ -263,6 +269,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             st.sbase = (uint32_t)u0 * unit_stride_b + (uint32_t)kt0 * BK;
             st.dst0 = (uint32_t)u0 * 1024u;
             wide::k_loop<WTN, 1, LOOP - 1>(acc, lds, st);
+            if (p.K % BK != 0 && chunk == p.S - 1) wide::tail_step<WTN, 1>(acc, lds, st, p.K % BK, lane);
         }
         MI355_TS(2)
         __syncthreads();
@@ -307,15 +314,16 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
         const int st_row = lane & 15, st_g = lane >> 4;
         auto stage = [&](int ch) {
             char *buf = lds + (ch & 1) * XBUF;
+            const bool last = (ch + 1) * CH * BK > kbytes;                   // reaches past the end of K: a scalar test per chunk
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int combo = wave * 4 + j;                              // (group of 16 rows, group of 4 pieces)
                 const int mt = combo % WTM, qg = combo / WTM;                // pieces 4 qg .. 4 qg + 3: step qg / 2, half qg % 2
                 const int row = mt * 16 + st_row, q = qg * 4 + st_g;
-                const bool ok = ch * CH + (q >> 3) < KT;
+                uint32_t vo = (uint32_t)(row * (int)p.lda + q * 16);
+                if (last && ch * CH * BK + q * 16 >= kbytes) vo = kOutOfRange;
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_void *)(buf + (((qg >> 1) * WTM + mt) * 2 + (qg & 1)) * 1024), 16,
-                                                         ok ? (uint32_t)(row * (int)p.lda + q * 16) : kOutOfRange,
-                                                         (uint32_t)(kt0 + ch * CH) * BK, 0, 0);
+                                                         vo, (uint32_t)(kt0 + ch * CH) * BK, 0, 0);
             }
         };
         // a chunk has landed: at most the `younger` loads issued behind its four are outstanding; and every wavefront is
@@ -419,15 +427,15 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     // are requested NS steps ahead: NS-1 stages in flight per CU instead of one is what a weight stream from HBM
     // needs when no second workgroup shares the CU.)
     static_assert(NS >= 2 && NS <= 4 && (NS < 4 || WTM * WTN <= 16), "weight slots");
-    issue_a(0, KT);
+    issue_a(0);
     issue_b(0, KT);
-    issue_a(1, KT);
+    issue_a(1);
     issue_b(1, KT);
     if constexpr (NS == 3 && !WHOLE) issue_b(2, KT);
     if constexpr (WHOLE) {
 #pragma unroll
         for (int st = 2; st < NS; st++) {
-            issue_a(st, KT);
+            issue_a(st);
             issue_b(st, KT);
         }
         wait_vmcnt<(NS - 1) * (LA + LB)>();                            // stage 0 has landed
@@ -446,7 +454,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             wait_vmcnt_lgkm0<LB>();            // stage kt+1 has landed and this wavefront is done reading stage kt
             __syncthreads();
             MI355_READ_FRAGS(af0, bf0, kt + 1, 0)
-            issue_a(kt + 2, KT);
+            issue_a(kt + 2);
             issue_b(kt + NS, KT);
             MI355_MFMA_BLOCK(af1, bf1)
             MI355_INTERLEAVE(LA + LB, 1)
@@ -461,7 +469,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             if constexpr (WHOLE) wait_vmcnt_lgkm0<(NS - 2) * (LA + LB)>();     // stage kt+1 has landed, NS-2 more may be in flight
             else wait_vmcnt_lgkm0<(NS - 2) * LB>();
             __syncthreads();
-            issue_a(kt + NSA, KT);
+            issue_a(kt + NSA);
             issue_b(kt + NS, KT);
             MI355_READ_FRAGS(af0, bf0, kt + 1, 0)
             __builtin_amdgcn_sched_barrier(0);
@@ -819,7 +827,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
 }
 
 // Correct for every shape, stride and alignment; used when the tiled kernel's preconditions
-// (K multiple of 128, 16-byte aligned rows) do not hold.  One thread per output element.
+// (K at least 128, 16-byte aligned rows or a K whose rows are copied into padded ones) do not hold.  One thread per output element.
 __global__ __launch_bounds__(256) void qmm_generic_kernel(const int8_t *__restrict__ a, const int8_t *__restrict__ b,
                                                           const float *__restrict__ pertoken,
                                                           const float *__restrict__ scale, int scale_len,
@@ -852,9 +860,29 @@ __global__ __launch_bounds__(256) void qmm_generic_kernel(const int8_t *__restri
     static_cast<uint16_t *>(out)[(int64_t)m * ldc + n] = (uint16_t)(out_f16 ? pack_f16x2(v, 0.0f) : pack_bf16x2(v, 0.0f));
 }
 
-// [K,N] contiguous -> [N,K] contiguous, 64x64 byte tiles through LDS.
+// Rows of K bytes (any K, pitch and alignment) -> rows of `pitch` bytes (K rounded up to a multiple of 16) with zeros past K:
+// what makes an operand whose rows are not a multiple of 16 bytes fit for 16-byte loads.  One 16-byte chunk per thread.
+__global__ __launch_bounds__(256) void pad_rows_i8_kernel(const int8_t *__restrict__ src, int64_t ld, int8_t *__restrict__ dst, int pitch,
+                                                          int rows, int K)
+{
+    const int chunks = pitch / 16;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < (int64_t)rows * chunks; i += (int64_t)gridDim.x * 256) {
+        const int64_t row = i / chunks;
+        const int k = (int)(i - row * chunks) * 16;
+        const int8_t *s = src + row * ld + k;
+        u32x4 v{0u, 0u, 0u, 0u};
+        if (k + 16 <= K) {
+            __builtin_memcpy(&v, s, 16);
+        } else {
+            for (int b = 0; k + b < K; b++) v[b >> 2] |= (uint32_t)(uint8_t)s[b] << (8 * (b & 3));
+        }
+        *reinterpret_cast<u32x4 *>(dst + row * pitch + k) = v;
+    }
+}
+
+// [K,N] contiguous -> [N,K] with rows of `pitch` bytes, 64x64 byte tiles through LDS.
 __global__ __launch_bounds__(256) void transpose_i8_kernel(const int8_t *__restrict__ src, int8_t *__restrict__ dst,
-                                                           int K, int N, int64_t ld_src)
+                                                           int K, int N, int64_t ld_src, int pitch)
 {
     __shared__ int8_t tile[64][64 + 4];
     const int k0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
@@ -866,7 +894,7 @@ __global__ __launch_bounds__(256) void transpose_i8_kernel(const int8_t *__restr
     __syncthreads();
     for (int r = ty; r < 64; r += 4) {
         const int n = n0 + r, k = k0 + tx;
-        if (n < N && k < K) dst[(int64_t)n * K + k] = tile[tx][r];
+        if (n < N && k < pitch) dst[(int64_t)n * pitch + k] = tile[tx][r];   // zeros past K
     }
 }
 
@@ -952,11 +980,12 @@ constexpr TileChoice kTiles[] = {{256, 256, 256, 58.0, 59.0, 0}, {256, 224, 256,
                                  {128, 128, 512, 40.0, 43.3, 0}, {64, 256, 512, 40.0, 52.6, 0},  {64, 128, 512, 24.0, 30.0, 0},
                                  {128, 192, 256, 32.0, 32.0, 1}, {128, 128, 256, 24.0, 24.8, 1}};
 
-// Workspace layout: [arrival counters | split-K partial sums | transposed weight].
+// Workspace layout: [arrival counters | split-K partial sums | transposed weight | padded operands].
 struct QmmPlan {
     TileChoice tile;
     int S;                       // K chunks per tile
-    size_t counter_bytes, partial_bytes, transpose_bytes;
+    size_t counter_bytes, partial_bytes, transpose_bytes, pad_bytes;
+    size_t workspace() const { return counter_bytes + partial_bytes + transpose_bytes + pad_bytes; }
 };
 
 // Pick the tile shape and the split of K with the smallest estimated time.  The table above gives a launch at K = 4096
@@ -980,7 +1009,7 @@ void choose_tile_and_split(int64_t M, int64_t N, int64_t K, bool may_split, size
 {
     const int forced_tile = knob(kKnobQmmTile);             // debugging aids: bm * 1000 + bn, and the split
     const int forced_split = knob(kKnobQmmSplit);
-    const int64_t kt = K / BK;
+    const int64_t kt = (K + BK - 1) / BK;
     double best_cost = 1e300;
     *tile = kTiles[0];
     *split = 1;
@@ -1035,18 +1064,21 @@ QmmPlan make_qmm_plan(int64_t M, int64_t N, int64_t K, int64_t ldb_k, int64_t ld
                       size_t scratch_cap = ~(size_t)0)
 {
     QmmPlan pl{};
-    const bool tiled_shape = K >= BK && K % BK == 0;
+    const bool tiled_shape = K >= BK;
+    const int64_t Kp = (K + 15) / 16 * 16;
     // the decode kernel splits K inside its workgroups (it is not used while a tile or a split is forced)
-    const bool decode = qmm_decode_shape(M, N, K) && knob(kKnobQmmSplit) == 0 && knob(kKnobQmmTile) == 0;
+    const bool decode = qmm_decode_shape(M, N, Kp) && knob(kKnobQmmSplit) == 0 && knob(kKnobQmmTile) == 0;
     // a contiguous [K,N] weight is transposed into the workspace
-    pl.transpose_bytes = tiled_shape && ldb_k != 1 && ldb_n == 1 ? (size_t)N * (size_t)K : 0;
-    const size_t fixed = zero_area + pl.transpose_bytes;
-    choose_tile_and_split(M, N, K, tiled_shape && !decode, scratch_cap > fixed ? scratch_cap - fixed : 0, &pl.tile, &pl.S);
+    pl.transpose_bytes = tiled_shape && ldb_k != 1 && ldb_n == 1 ? (size_t)N * (size_t)Kp : 0;
+    // rows that are not a multiple of 16 bytes are copied into padded ones
+    if (tiled_shape && Kp != K) pl.pad_bytes = ((size_t)M + (ldb_k == 1 ? (size_t)N : 0)) * (size_t)Kp;
+    const size_t fixed = zero_area + pl.transpose_bytes + pl.pad_bytes;
+    choose_tile_and_split(M, N, Kp, tiled_shape && !decode, scratch_cap > fixed ? scratch_cap - fixed : 0, &pl.tile, &pl.S);
     if (tiled_shape && pl.S > 1) {
         const int64_t tiles = ((M + pl.tile.bm - 1) / pl.tile.bm) * ((N + pl.tile.bn - 1) / pl.tile.bn);
         pl.partial_bytes = (size_t)tiles * pl.S * pl.tile.bm * pl.tile.bn * 4;   // tiles <= 128 counters
     }
-    pl.counter_bytes = pl.partial_bytes + pl.transpose_bytes > 0 ? zero_area : 0;
+    pl.counter_bytes = pl.workspace() > 0 ? zero_area : 0;
     return pl;
 }
 
@@ -1058,7 +1090,7 @@ extern "C" size_t mi355_quant_matmul_workspace(int64_t M, int64_t N, int64_t K, 
     using namespace mi355;
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff) return 0;
     const QmmPlan pl = make_qmm_plan(M, N, K, ldb_k, ldb_n);
-    return pl.counter_bytes + pl.partial_bytes + pl.transpose_bytes;
+    return pl.workspace();
 }
 
 namespace mi355 {
@@ -1112,15 +1144,18 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
 
     const int8_t *bt = b;
     int64_t ldbt = ldb_n;
+    const int64_t Kp = (K + 15) / 16 * 16;
+    const bool pad = Kp != K;                              // both operands get rows of Kp bytes in the workspace
     // the tiled kernel addresses a tile's rows with 32-bit buffer offsets: 256 rows of either operand must stay below 2^31
-    const bool offsets_fit = (uint64_t)256 * (uint64_t)lda + (uint64_t)K < (1ull << 31) &&
-                             (uint64_t)256 * (uint64_t)(ldb_k != 1 ? K : ldb_n) + (uint64_t)K < (1ull << 31);
-    bool tiled = K >= BK && K % BK == 0 && (lda & 15) == 0 && aligned(a, 16) && offsets_fit;
+    const bool offsets_fit = (uint64_t)256 * (uint64_t)(pad ? Kp : lda) + (uint64_t)Kp < (1ull << 31) &&
+                             (uint64_t)256 * (uint64_t)(ldb_k != 1 || pad ? Kp : ldb_n) + (uint64_t)Kp < (1ull << 31);
+    bool tiled = K >= BK && (pad || ((lda & 15) == 0 && aligned(a, 16))) && offsets_fit;
     const QmmPlan pl = make_qmm_plan(M, N, K, ldb_k, ldb_n, zero_area, scratch_cap);
     char *ws = static_cast<char *>(workspace);
-    if (tiled && pl.counter_bytes + pl.partial_bytes + pl.transpose_bytes > 0) {
-        if (!ws || workspace_bytes < pl.counter_bytes + pl.partial_bytes + pl.transpose_bytes) return MI355_ERR_WORKSPACE;
-        if (!aligned(ws, 16)) return MI355_ERR_ALIGNMENT;
+    if (tiled && pl.workspace() > 0 && (!ws || workspace_bytes < pl.workspace() || !aligned(ws, 16))) {
+        // a K of whole steps needs its workspace; any other K also runs without one, on the generic kernel
+        if (K % BK == 0) return !ws || workspace_bytes < pl.workspace() ? MI355_ERR_WORKSPACE : MI355_ERR_ALIGNMENT;
+        tiled = false;
     }
     if (tiled && ldb_k != 1) {
         // contiguous [K,N]: transpose once into the workspace
@@ -1130,11 +1165,32 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
                                dim3(256), 0, s, b, dst, (int)K, (int)N, ldb_k);
         else
             hipLaunchKernelGGL(transpose_i8_kernel, dim3((unsigned)((N + 63) / 64), (unsigned)((K + 63) / 64)), dim3(256), 0,
-                               s, b, dst, (int)K, (int)N, ldb_k);
+                               s, b, dst, (int)K, (int)N, ldb_k, (int)Kp);
         bt = dst;
-        ldbt = K;
+        ldbt = Kp;
+    }
+    if (tiled && pad) {
+        // a zero-padded copy of the operands, then a product over Kp: 2 bytes of traffic per operand byte (a 45 MB weight: about
+        // 20 us) where the generic kernel takes tens of milliseconds
+        int8_t *dst = reinterpret_cast<int8_t *>(ws + pl.counter_bytes + pl.partial_bytes + pl.transpose_bytes);
+        const auto copy = [&](const int8_t *src, int64_t ld, int64_t rows) {
+            const int64_t blocks = (rows * (Kp / 16) + 255) / 256;
+            hipLaunchKernelGGL(pad_rows_i8_kernel, dim3((unsigned)(blocks < 16384 ? blocks : 16384)), dim3(256), 0, s, src, ld, dst, (int)Kp,
+                               (int)rows, (int)K);
+            int8_t *at = dst;
+            dst += rows * Kp;
+            return at;
+        };
+        a = copy(a, lda, M);
+        lda = Kp;
+        if (ldb_k == 1) {
+            bt = copy(b, ldb_n, N);
+            ldbt = Kp;
+        }
     }
     tiled = tiled && (ldbt & 15) == 0 && aligned(bt, 16);
+    const int64_t K_in = K;
+    if (tiled) K = Kp;
     if (tiled && knob(kKnobQmmSplit) == 0 && knob(kKnobQmmTile) == 0) {
         // at most 64 rows: the barrier-free kernel that splits K inside the workgroup (quant_matmul_decode.hip)
         QmmDecodeArgs d;
@@ -1162,7 +1218,7 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
     if (!tiled) {
         hipLaunchKernelGGL(qmm_generic_kernel, dim3((unsigned)((N + 15) / 16), (unsigned)((M + 15) / 16)), dim3(256), 0, s,
                            a, b, pertoken_scale, scale, (int)scale_len, bias, bias_dtype, out_dtype == MI355_OUT_FP16 ? 1 : 0, out,
-                           out_i32, qparam, out_i8, (int)M, (int)N, (int)K, lda, ldb_k, ldb_n, ldc);
+                           out_i32, qparam, out_i8, (int)M, (int)N, (int)K_in, lda, ldb_k, ldb_n, ldc);
         return check_launch();
     }
 
@@ -1363,15 +1419,16 @@ extern "C" int mi355_quant_matmul_noalloc(const int8_t *a, const int8_t *b, cons
                                 ldb_k, ldb_n, ldc, nullptr, 0, stream);
     // the scratch array is private to this operator: the arrival counters are followed directly by the partial sums
     const QmmPlan pl = make_qmm_plan(M, N, K, ldb_k, ldb_n, kWorkspaceCounterCapacity, kStaticScratchBytes);
-    const size_t need = pl.counter_bytes + pl.partial_bytes + pl.transpose_bytes;
-    if (need > kStaticScratchBytes) return MI355_ERR_WORKSPACE;      // beyond the fixed scratch: use mi355_quant_matmul
-    void *ws = nullptr;
-    if (need > 0) {
+    const size_t need = pl.workspace();
+    const bool fits = need <= kStaticScratchBytes;
+    if (!fits && K % BK == 0) return MI355_ERR_WORKSPACE;            // beyond the fixed scratch: use mi355_quant_matmul
+    void *ws = nullptr;                                              // (any other K runs without a workspace)
+    if (need > 0 && fits) {
         const int st = scratch_of_current_device(&ws, static_cast<hipStream_t>(stream));
         if (st != MI355_OK) return st;
     }
     return run_quant_matmul(a, b, pertoken_scale, scale, nullptr, scale_len, bias, bias_dtype, out, out_dtype, M, N, K, lda,
-                            ldb_k, ldb_n, ldc, ws, need > 0 ? kStaticScratchBytes : 0, stream, kWorkspaceCounterCapacity, kStaticScratchBytes);
+                            ldb_k, ldb_n, ldc, ws, ws ? kStaticScratchBytes : 0, stream, kWorkspaceCounterCapacity, kStaticScratchBytes);
 }
 
 // One-time weight pre-layout for npu_quant_matmul: a contiguous [K,N] int8 weight is rewritten K-major ([N,K] storage),
@@ -1389,6 +1446,6 @@ extern "C" int mi355_transpose_int8(const int8_t *src, int8_t *dst, int64_t K, i
                            src, dst, (int)K, (int)N, ld_src);
     else
         hipLaunchKernelGGL(transpose_i8_kernel, dim3((unsigned)((N + 63) / 64), (unsigned)((K + 63) / 64)), dim3(256), 0, s, src, dst,
-                           (int)K, (int)N, ld_src);
+                           (int)K, (int)N, ld_src, (int)K);
     return check_launch();
 }

@@ -45,7 +45,7 @@ __global__ __launch_bounds__(512) void qmm_decode_kernel(const QmmDecodeArgs p)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    const int KT = p.K / kStep;
+    const int KT = (p.K + kStep - 1) / kStep;                             // the last step may be partial: zeros from x past K
     const int s0 = KT * wave / 8, ns = KT * (wave + 1) / 8 - s0;          // this wavefront's steps (at most NS)
     const int strips = (p.N + 15) / 16;
     const int my_strips = (strips - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;   // strips b, b + grid, ...
@@ -60,11 +60,13 @@ __global__ __launch_bounds__(512) void qmm_decode_kernel(const QmmDecodeArgs p)
     // lane l of half h loads row 8 h + l / 8, and the 16-byte piece that belongs in slot l % 8 of that row's swizzled
     // LDS image: piece (l % 8) ^ ((row / 2) % 8).  Weight rows past N lie beyond the descriptor's range.
     uint32_t voff_w[2], voff_x[MT][2];
+    int kpos[2];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         const int rl = 8 * h + (lane >> 3);
         const int piece = ((lane & 7) ^ ((rl >> 1) & 7)) * 16;
         voff_w[h] = (uint32_t)(rl * (int)p.ldbt + piece);
+        kpos[h] = p.K - piece;
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) voff_x[mt][h] = mt * 16 + rl < p.M ? (uint32_t)((mt * 16 + rl) * (int)p.lda + piece) : kOutOfRange;
     }
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(512) void qmm_decode_kernel(const QmmDecodeArgs p)
 #pragma unroll
             for (int h = 0; h < 2; h++)
                 xf[j][mt][h] = __builtin_bit_cast(i32x4v, __builtin_amdgcn_raw_buffer_load_b128(
-                    rsrc_x, j < ns ? voff_x[mt][h] : kOutOfRange, (uint32_t)(s0 + j) * kStep, 0));
+                    rsrc_x, j < ns && (s0 + j) * kStep < kpos[h] ? voff_x[mt][h] : kOutOfRange, (uint32_t)(s0 + j) * kStep, 0));
 
     // weights: flat step f = strip index * NS + step; ring slot f % PF, LDS buffer f % 2
     i32x4v wr[PF][2];
@@ -225,11 +227,11 @@ int launch(const QmmDecodeArgs &p, hipStream_t s)
 
 bool qmm_decode_shape(int64_t M, int64_t N, int64_t K)
 {
-    if (knob(kKnobQmmDecodeOff) == 1 || M < 1 || M > 64 || K % kStep != 0 || K < 8 * kStep || N < 2048) return false;
+    if (knob(kKnobQmmDecodeOff) == 1 || M < 1 || M > 64 || K % 16 != 0 || K < 8 * kStep || N < 2048) return false;
     // The activations of a wavefront's eighth of K stay in registers: up to 16 steps with one tile of 16 rows, 8 with two,
     // 4 with four.  With four tiles and more than 1024 strips the tiled kernel's streaming loop is faster (measured at
     // K = 4096: N = 6144 11.8 against 15.1 us, N = 28672 27.7 against 25.8).
-    const int64_t steps = (K / kStep + 7) / 8;
+    const int64_t steps = ((K + kStep - 1) / kStep + 7) / 8;
     if (M <= 16) return steps <= 16;
     if (M <= 32) return steps <= 8;
     return steps <= 4 && N <= 16384;
@@ -247,7 +249,7 @@ int launch_qmm_decode(const QmmDecodeArgs &p, hipStream_t s)
     // 32-bit buffer offsets over the whole weight and all activation rows
     if ((uint64_t)(p.N + 16) * (uint64_t)p.ldbt + (uint64_t)p.K >= (1ull << 31) || (uint64_t)p.M * (uint64_t)p.lda + (uint64_t)p.K >= (1ull << 31))
         return MI355_ERR_UNSUPPORTED;
-    const int ns = (p.K / kStep + 7) / 8;                                 // steps of the busiest wavefront
+    const int ns = ((p.K + kStep - 1) / kStep + 7) / 8;                                 // steps of the busiest wavefront
     if (p.M <= 16) return ns <= 4 ? launch<1, 4, 4>(p, s) : ns <= 8 ? launch<1, 8, 4>(p, s) : launch<1, 16, 4>(p, s);
     if (p.M <= 32) return ns <= 4 ? launch<2, 4, 4>(p, s) : launch<2, 8, 4>(p, s);
     return launch<4, 4, 4>(p, s);

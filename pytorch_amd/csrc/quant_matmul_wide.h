@@ -334,6 +334,39 @@ __device__ __forceinline__ void k_loop(i32x4v (&acc)[4][WTN], char *lds, const L
     wait_vmcnt_only<0>();                    // the refills past the end must not land in the epilogue's LDS
 }
 
+// The partial step behind the loop when K is not a multiple of 128 (`tail` bytes, a multiple of 16): the activation chunks
+// past K are loaded as zeros.  It stands outside the pipelined loop, whose refills have scalar offsets only, so that the loop
+// pays neither registers nor instructions for it; its loads are exposed instead (1.5 us against a launch of 40 and more).
+template <int WTN, int ROLE>
+__device__ __forceinline__ void tail_step(i32x4v (&acc)[4][WTN], char *lds, LoopState st, int tail, int lane)
+{
+    using G = Geometry<WTN>;
+    constexpr int NL = ROLE == 0 ? LAW : G::LBW;
+    __builtin_amdgcn_s_barrier();            // every wavefront is done with the slots
+    if constexpr (ROLE == 0) {
+        // lane l of unit u holds chunk (l % 8) ^ (4 * (u & 1) + l / 16) of its row; u0 is even
+        const int c0 = (lane & 7) ^ (lane >> 4);
+        if (c0 * 16 >= tail) st.voff0 = kPastEnd;
+        if ((c0 ^ 4) * 16 >= tail) st.voff1 = kPastEnd;
+    }
+    issue_units<NL>(st, lds, (ROLE == 0 ? 0 : G::B_BASE) + st.dst0, st.sbase + (uint32_t)st.KT * BK);
+    wait_vmcnt_only<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        i32x4v a[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[i] = *reinterpret_cast<const i32x4v *>(lds + (h ? st.va1 : st.va0) + i * 2048);
+#pragma unroll
+        for (int j = 0; j < WTN; j++) {
+            const i32x4v b = *reinterpret_cast<const i32x4v *>(lds + (h ? st.vb1 : st.vb0) + j * 2048);
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b, a[i], acc[i][j], 0, 0, 0);
+        }
+    }
+}
+
 
 // ---------------------------------------------------------------------------------------------------------------
 // Epilogue for the common cases: per-token scales or none, one float32 scale per column or one for all, optional bf16 bias,

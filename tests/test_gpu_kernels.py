@@ -555,6 +555,34 @@ def test_quant_matmul_decode_kernel(capi, golden, M, K, N):
         capi.set_tuning("MI355_QMM_DECODE_OFF", 0)
 
 
+@pytest.mark.parametrize("weight_nk", [True, False])
+@pytest.mark.parametrize("M,K,N", [(5, 1040, 2052), (20, 2160, 2048), (40, 1936, 2064),       # decode kernel, partial last step
+                                   (64, 144, 260), (100, 4112, 520), (128, 1264, 2000),         # streaming loop, small tiles, split K
+                                   (300, 240, 1000), (513, 2224, 1544), (3, 129, 40), (50, 1001, 2048), (257, 1025, 500)])
+def test_quant_matmul_partial_last_step(capi, golden, M, K, N, weight_nk):
+    """K that is not a multiple of 128 (a partial last step: the activations past K count as zeros) or not even of 16 (operands
+    copied into padded rows).  Accumulators and the bf16 epilogue bit-identical to the oracle on whatever the planner picks, and
+    the accumulators again on every tile with both loops of the 256-row ones, unsplit and split."""
+    d = workloads.quant_matmul_inputs(seed=M + K, M=M, K=K, N=N, weight_nk=weight_nk, bias=True)
+    x1, x2 = d["x1"].cuda(), d["x2"].cuda()
+    acc = golden.int8_gemm(d["x1"].numpy(), d["x2"].numpy())
+    assert np.array_equal(capi.quant_matmul(x1, x2, None, out_dtype=torch.int32).cpu().numpy(), acc)
+    out = capi.quant_matmul(x1, x2, d["scale"].cuda(), d["pertoken_scale"].cuda(), d["bias"].cuda())
+    want, _ = golden.quant_matmul(d["x1"].numpy(), d["x2"].numpy(), d["scale"].numpy(), d["pertoken_scale"].numpy(), _bits(d["bias"]))
+    assert np.array_equal(_bits(out), want)
+    try:
+        for tile in (256256, 256224, 256192, 128320, 128256, 128192, 128128, 64256, 64128):
+            capi.set_tuning("MI355_QMM_TILE", tile)
+            for loop in (0, 1, 2, 4):
+                capi.set_tuning("MI355_QMM_LOOP", loop)
+                for split in (0, 2):
+                    capi.set_tuning("MI355_QMM_SPLIT", split)
+                    assert np.array_equal(capi.quant_matmul(x1, x2, None, out_dtype=torch.int32).cpu().numpy(), acc), (tile, loop, split)
+    finally:
+        for k in ("MI355_QMM_TILE", "MI355_QMM_SPLIT", "MI355_QMM_LOOP"):
+            capi.set_tuning(k, 0)
+
+
 QMM_MID_ROWS = [33, 64, 65, 128, 192, 256]
 QMM_MID_PROJECTIONS = [(4096, 6144), (4096, 11008), (11008, 4096)]
 
