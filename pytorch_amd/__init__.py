@@ -20,12 +20,18 @@ _CSRC = _os.path.join(_os.path.dirname(_os.path.abspath(__file__)), "csrc")
 KERNEL_LIBRARY = _os.path.join(_CSRC, "libmi355_quant.so")
 OPS_LIBRARY = _os.path.join(_CSRC, "libmi355_npu_ops.so")
 
-for _p in (KERNEL_LIBRARY, OPS_LIBRARY):
+CALL_LIBRARY = _os.path.join(_os.path.dirname(_CSRC), "_op_call.so")
+
+for _p in (KERNEL_LIBRARY, OPS_LIBRARY, CALL_LIBRARY):
     if not _os.path.exists(_p):
         raise ImportError(f"{_p} is missing: build the native libraries first with `python pytorch_amd/build.py` "
                           "(hipcc, --offload-arch=gfx950)")
 
 _torch.ops.load_library(OPS_LIBRARY)
+
+from . import _op_call  # noqa: E402
+
+_op_call.install(_torch.ops.npu, _torch.nn.Parameter)          # calls of torch.ops.npu.* go straight to the dispatcher (csrc/op_call.cpp)
 
 __all__ = []
 

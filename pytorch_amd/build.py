@@ -2,6 +2,7 @@
 
 * ``csrc/libmi355_quant.so``  - the HIP kernels behind the C ABI of ``include/mi355_quant.h``
 * ``csrc/libmi355_npu_ops.so`` - the torch operator library registering ``torch.ops.npu.*``
+* ``_op_call.so``              - Python extension: the operators' direct call path (``csrc/op_call.cpp``)
 
 Usage: ``python pytorch_amd/build.py`` (compiles every time it is called; run it as a script, because
 importing the package requires the libraries this builds).
@@ -17,6 +18,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 KERNEL_LIB = os.path.join(CSRC, "libmi355_quant.so")
 OPS_LIB = os.path.join(CSRC, "libmi355_npu_ops.so")
+CALL_LIB = os.path.join(HERE, "_op_call.so")
 KERNEL_SOURCES = ["dynamic_quant.hip", "dynamic_quant_asym.hip", "quant_matmul.hip", "quant_matmul_decode.hip", "weight_quant_matmul.hip", "weight_quant_gemm.hip", "weight_quant_kpacked.hip", "weight_quant_kpacked_decode.hip", "weight_quant_kmajor_decode.hip", "weight_quant_decode.hip", "weight_quant_gemm4.hip", "weight_quant_repack.hip", "swiglu.hip", "anti_quant.hip", "unpack_int4.hip", "quantize.hip", "tuning.hip", "device_probe.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -65,8 +67,7 @@ def build_kernels(verbose: bool = False) -> str:
     return KERNEL_LIB
 
 
-def build_ops(verbose: bool = False) -> str:
-    """torch operator library: host-only C++ against libtorch + the C ABI."""
+def _torch_command(source: str, target: str, *more: str) -> list:
     import torch
     from torch.utils import cpp_extension as ce
 
@@ -74,15 +75,21 @@ def build_ops(verbose: bool = False) -> str:
     for p in ce.include_paths(device_type="cuda"):
         inc += ["-I", p]
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    cmd = [HIPCC, "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-Wno-unused-command-line-argument",
-           "-I", os.path.join(HERE, "..", "include"), *inc,
-           os.path.join(CSRC, "npu_ops.cpp"), "-o", OPS_LIB,
-           "-L", torch_lib, "-L", CSRC, "-lc10", "-ltorch_cpu", "-ltorch", "-lc10_hip", "-ltorch_hip", "-lmi355_quant",
-           "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + torch_lib]
-    out = _run(cmd)
-    if verbose and out.strip():
-        print(out)
+    return [HIPCC, "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-Wno-unused-command-line-argument",
+            "-I", os.path.join(HERE, "..", "include"), *inc, os.path.join(CSRC, source), "-o", target,
+            "-L", torch_lib, "-lc10", "-ltorch_cpu", "-ltorch", "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + torch_lib, *more]
+
+
+def build_ops(verbose: bool = False) -> str:
+    """torch operator library: host-only C++ against libtorch + the C ABI; and the operators' direct call path."""
+    import sysconfig
+
+    for cmd in (_torch_command("npu_ops.cpp", OPS_LIB, "-L", CSRC, "-lc10_hip", "-ltorch_hip", "-lmi355_quant"),
+                _torch_command("op_call.cpp", CALL_LIB, "-I", sysconfig.get_paths()["include"], "-ltorch_python")):
+        out = _run(cmd)
+        if verbose and out.strip():
+            print(out)
     return OPS_LIB
 
 

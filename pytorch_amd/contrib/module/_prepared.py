@@ -22,3 +22,10 @@ class PreparedCopiesMixin:
     def _load_from_state_dict(self, *args, **kwargs):
         self._drop_prepared()
         return super()._load_from_state_dict(*args, **kwargs)
+
+
+def parameter(module, name):
+    """``getattr(module, name)`` of a registered parameter (or ``None`` in its place) without the attribute protocol of
+    ``nn.Module``, which takes a Python call per access; anything else (a parametrized weight, say) goes through it."""
+    table = module._parameters
+    return table[name] if name in table else getattr(module, name)

@@ -13,7 +13,8 @@ import warnings
 import torch
 from torch import nn
 
-from ._prepared import PreparedCopiesMixin
+from ... import _op_call
+from ._prepared import PreparedCopiesMixin, parameter
 
 __all__ = ["LinearQuant", "LinearA8W8Quant"]
 
@@ -84,25 +85,31 @@ class _QuantLinearBase(PreparedCopiesMixin, nn.Module):
         return self
 
     def forward(self, linear_quant_input: torch.Tensor) -> torch.Tensor:
-        self._check_dtypes(linear_quant_input)
-        weight = self.weight
-        prepared = getattr(self, "_prepared_i8", None)
-        if prepared is not None and linear_quant_input.dtype == torch.int32:
+        x = linear_quant_input
+        weight, scale, offset = parameter(self, "weight"), parameter(self, "scale"), parameter(self, "offset")
+        pertoken_scale, bias = parameter(self, "pertoken_scale"), parameter(self, "bias")
+        if self._validate_dtypes or x.dtype != torch.int8 or weight.dtype != torch.int8:
+            self._check_dtypes(x)
+        prepared = self.__dict__.get("_prepared_i8")
+        if prepared is not None and x.dtype == torch.int32:
             from ... import _capi
-            x = linear_quant_input
             words = x.shape[-1]
-            linear_quant_input = _capi.unpack_int4(x.reshape(-1, words).contiguous()).view(*x.shape[:-1], words * 8)
+            x = _capi.unpack_int4(x.reshape(-1, words).contiguous()).view(*x.shape[:-1], words * 8)
             weight = prepared
-        elif prepared is not None and linear_quant_input.dtype == torch.int8 and self.weight.dtype == torch.int8:
+        elif prepared is not None and x.dtype == torch.int8 and weight.dtype == torch.int8:
             weight = prepared
-        scale = self.scale
         # a float32 scale is packed with npu_trans_quant_param when there is no pertoken_scale and the output is int8
         # (output_dtype None) or float16 (linear_quant.py:104-108)
-        if (self.pertoken_scale is None and scale.dtype == torch.float32
-                and self.output_dtype not in (torch.bfloat16, torch.int32)):
-            scale = torch.ops.npu.npu_trans_quant_param(scale, self.offset)
-        return torch.ops.npu.npu_quant_matmul(linear_quant_input, weight.transpose(-2, -1), scale,
-                                              offset=self.offset, pertoken_scale=self.pertoken_scale, bias=self.bias,
+        packs = pertoken_scale is None and scale.dtype == torch.float32 and self.output_dtype not in (torch.bfloat16, torch.int32)
+        if not (packs and scale.dim() != 1) and not torch.compiler.is_compiling():
+            # on the GPU: one native call.  The packed word of a float16 output holds the bits of the scale and nothing else that
+            # the product uses, so the scale vector goes as it is; for an int8 output the operator packs scale and offset itself.
+            out = _op_call.linear_quant(x, weight, scale, offset, pertoken_scale, bias, self.output_dtype)
+            if out is not NotImplemented:
+                return out
+        if packs:
+            scale = torch.ops.npu.npu_trans_quant_param(scale, offset)
+        return torch.ops.npu.npu_quant_matmul(x, weight.transpose(-2, -1), scale, offset=offset, pertoken_scale=pertoken_scale, bias=bias,
                                               output_dtype=self.output_dtype)
 
 

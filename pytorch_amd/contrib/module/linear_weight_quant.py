@@ -14,7 +14,8 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from ._prepared import PreparedCopiesMixin
+from ... import _op_call
+from ._prepared import PreparedCopiesMixin, parameter
 
 __all__ = ["LinearWeightQuant"]
 
@@ -74,8 +75,10 @@ class LinearWeightQuant(PreparedCopiesMixin, nn.Module):
         return param.transpose(-1, -2) if param is not None and param.dim() == 2 else param
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        prepared = getattr(self, "_prepared", None)
-        if prepared is not None and self.weight.dtype == torch.int32 and self.antiquant_group_size == 128:
+        prepared = self.__dict__.get("_prepared")
+        weight = parameter(self, "weight")
+        quant_scale, quant_offset, bias = parameter(self, "quant_scale"), parameter(self, "quant_offset"), parameter(self, "bias")
+        if prepared is not None and weight.dtype == torch.int32 and self.antiquant_group_size == 128:
             # 2 to 32 rows: the decode kernel for the module's own storage (words along K) is the faster one
             # (int4 [14336, 4096/8], 8 / 32 rows: 9.8 / 15.4 us against 10.3 / 17.2 on the repacked copy)
             rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
@@ -83,10 +86,15 @@ class LinearWeightQuant(PreparedCopiesMixin, nn.Module):
                 prepared = None
         if prepared is not None:
             weight, scale, offset = prepared
-            return torch.ops.npu.npu_weight_quant_batchmatmul(x, weight, scale, offset, self.quant_scale, self.quant_offset,
-                                                              self.bias, self.antiquant_group_size, self.inner_precise,
+            return torch.ops.npu.npu_weight_quant_batchmatmul(x, weight, scale, offset, quant_scale, quant_offset, bias,
+                                                              self.antiquant_group_size, self.inner_precise,
                                                               weight_dtype=self.weight_dtype)
+        scale, offset = parameter(self, "antiquant_scale"), parameter(self, "antiquant_offset")
+        if self.weight_dtype is None and not torch.compiler.is_compiling():
+            out = _op_call.linear_weight_quant(x, weight, scale, offset, quant_scale, quant_offset, bias, self.antiquant_group_size,
+                                               self.inner_precise)
+            if out is not NotImplemented:
+                return out
         return torch.ops.npu.npu_weight_quant_batchmatmul(
-            x, self.weight.transpose(-1, -2), self._as_group_major(self.antiquant_scale),
-            self._as_group_major(self.antiquant_offset), self.quant_scale, self.quant_offset, self.bias,
+            x, weight.transpose(-1, -2), self._as_group_major(scale), self._as_group_major(offset), quant_scale, quant_offset, bias,
             self.antiquant_group_size, self.inner_precise, weight_dtype=self.weight_dtype)

@@ -11,7 +11,9 @@
 // inference for FakeTensor).  There is deliberately no CPU kernel: calling these ops with CPU
 // tensors fails in the dispatcher.
 #include <ATen/ATen.h>
+#include <ATen/DimVector.h>
 #include <ATen/ExpandUtils.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <hip/hip_runtime_api.h>
@@ -57,6 +59,19 @@ void *stream_of(const Tensor &t)
     return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
 }
 
+// An uninitialised contiguous tensor beside `like`: through the dispatcher for shape inference (kMeta), and straight from the
+// caching allocator for a launch (kLaunch), where the dispatcher and the option parsing would be a tenth of an operator's host
+// time at decode sizes for each output.
+enum Alloc { kMeta, kLaunch };
+Tensor new_empty(Alloc how, const Tensor &like, at::IntArrayRef sizes, at::ScalarType dtype)
+{
+    if (how == kLaunch) return Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), c10::nullopt));
+    return at::empty(sizes, like.options().dtype(dtype));
+}
+
+// (at::contiguous dispatches even when there is nothing to do)
+Tensor packed(const Tensor &t) { return t.is_contiguous() ? t : t.contiguous(); }
+
 // ---------------------------------------------------------------- npu_dynamic_quant
 
 // Per-expert smooth scales: smooth_scales [E, H] with group_index [E], the running totals of the rows of each expert.
@@ -90,21 +105,19 @@ void dynamic_quant_check(const Tensor &input, const optional<Tensor> &smooth_sca
 }
 
 // int4: an int32 result whose last dimension is an eighth of the input's
-std::tuple<Tensor, Tensor> dynamic_quant_alloc(const Tensor &input, bool int4 = false)
+std::tuple<Tensor, Tensor> dynamic_quant_alloc(Alloc how, const Tensor &input, bool int4 = false)
 {
-    auto scale_shape = input.sizes().vec();
-    scale_shape.pop_back();
-    auto y_shape = input.sizes().vec();
+    at::DimVector y_shape(input.sizes());
     if (int4) y_shape.back() /= 8;
-    return {at::empty(y_shape, input.options().dtype(int4 ? at::kInt : at::kChar)),
-            at::empty(scale_shape, input.options().dtype(at::kFloat))};
+    return {new_empty(how, input, y_shape, int4 ? at::kInt : at::kChar),
+            new_empty(how, input, input.sizes().slice(0, input.dim() - 1), at::kFloat)};
 }
 
 std::tuple<Tensor, Tensor> dynamic_quant_meta(const Tensor &input, const optional<Tensor> &smooth_scales,
                                               const optional<Tensor> &group_index, optional<at::ScalarType> dst_type)
 {
     dynamic_quant_check(input, smooth_scales, group_index, dst_type, true);
-    return dynamic_quant_alloc(input, dst_type.has_value() && *dst_type == at::kQUInt4x2);
+    return dynamic_quant_alloc(kMeta, input, dst_type.has_value() && *dst_type == at::kQUInt4x2);
 }
 
 std::tuple<Tensor, Tensor> dynamic_quant_hip(const Tensor &input, const optional<Tensor> &smooth_scales,
@@ -114,7 +127,7 @@ std::tuple<Tensor, Tensor> dynamic_quant_hip(const Tensor &input, const optional
     check_same_device("npu_dynamic_quant", {&input, opt(smooth_scales), opt(group_index)});
     c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
     const bool int4 = dst_type.has_value() && *dst_type == at::kQUInt4x2;
-    auto [y, scale] = dynamic_quant_alloc(input, int4);
+    auto [y, scale] = dynamic_quant_alloc(kLaunch, input, int4);
     const int64_t cols = input.size(-1);
     const int64_t rows = cols ? input.numel() / cols : 0;
     if (rows == 0 || cols == 0) {
@@ -130,7 +143,7 @@ std::tuple<Tensor, Tensor> dynamic_quant_hip(const Tensor &input, const optional
         x = x.contiguous();
     }
     Tensor smooth;
-    if (const Tensor *s = opt(smooth_scales)) smooth = s->contiguous();
+    if (const Tensor *s = opt(smooth_scales)) smooth = packed(*s);
     Tensor gi;                                             // a handful of totals: int64 ones are narrowed on the device
     if (const Tensor *g = opt(group_index)) gi = g->to(at::kInt).contiguous();
     if (int4) {
@@ -154,10 +167,10 @@ std::tuple<Tensor, Tensor> dynamic_quant_hip(const Tensor &input, const optional
 // torch_npu.npu_dynamic_quant_asymmetric(input, *, smooth_scales=None, group_index=None, dst_type=None)
 // -> (y int8, scale float32, offset float32)   (test/test_fake_tensor.py:1689-1709, test/torch_npu_schema.json:2147-2149)
 
-std::tuple<Tensor, Tensor, Tensor> dynamic_quant_asym_alloc(const Tensor &input)
+std::tuple<Tensor, Tensor, Tensor> dynamic_quant_asym_alloc(Alloc how, const Tensor &input)
 {
-    auto [y, scale] = dynamic_quant_alloc(input);
-    return {y, scale, at::empty_like(scale)};
+    auto [y, scale] = dynamic_quant_alloc(how, input);
+    return {y, scale, new_empty(how, input, scale.sizes(), at::kFloat)};
 }
 
 std::tuple<Tensor, Tensor, Tensor> dynamic_quant_asym_meta(const Tensor &input, const optional<Tensor> &smooth_scales,
@@ -165,7 +178,7 @@ std::tuple<Tensor, Tensor, Tensor> dynamic_quant_asym_meta(const Tensor &input, 
                                                            optional<at::ScalarType> dst_type)
 {
     dynamic_quant_check(input, smooth_scales, group_index, dst_type);
-    return dynamic_quant_asym_alloc(input);
+    return dynamic_quant_asym_alloc(kMeta, input);
 }
 
 std::tuple<Tensor, Tensor, Tensor> dynamic_quant_asym_hip(const Tensor &input, const optional<Tensor> &smooth_scales,
@@ -175,7 +188,7 @@ std::tuple<Tensor, Tensor, Tensor> dynamic_quant_asym_hip(const Tensor &input, c
     dynamic_quant_check(input, smooth_scales, group_index, dst_type);
     check_same_device("npu_dynamic_quant_asymmetric", {&input, opt(smooth_scales), opt(group_index)});
     c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    auto [y, scale, offset] = dynamic_quant_asym_alloc(input);
+    auto [y, scale, offset] = dynamic_quant_asym_alloc(kLaunch, input);
     const int64_t cols = input.size(-1);
     const int64_t rows = cols ? input.numel() / cols : 0;
     if (rows == 0 || cols == 0) {
@@ -191,7 +204,7 @@ std::tuple<Tensor, Tensor, Tensor> dynamic_quant_asym_hip(const Tensor &input, c
         x = x.contiguous();
     }
     Tensor smooth;
-    if (const Tensor *s = opt(smooth_scales)) smooth = s->contiguous();
+    if (const Tensor *s = opt(smooth_scales)) smooth = packed(*s);
     Tensor gi;
     if (const Tensor *g = opt(group_index)) gi = g->to(at::kInt).contiguous();
     check_status(mi355_dynamic_quant_asymmetric_grouped(x.data_ptr(),
@@ -286,32 +299,32 @@ Tensor zeroed_workspace(const Tensor &like, size_t bytes)
 // torch_npu.npu_trans_quant_param(scale, offset=None) (linear_quant.py:104-108; shapes test/test_fake_tensor.py:1929-1943:
 // the result is int64 and takes the shape of whichever argument has more elements)
 
-std::vector<int64_t> trans_quant_param_shape(const Tensor &scale, const optional<Tensor> &offset)
+at::IntArrayRef trans_quant_param_shape(const Tensor &scale, const optional<Tensor> &offset)
 {
     TORCH_CHECK(scale.scalar_type() == at::kFloat, "npu_trans_quant_param: scale must be float32, got ", scale.scalar_type());
     TORCH_CHECK(scale.dim() >= 1 && scale.dim() <= 2, "npu_trans_quant_param: scale must have 1 or 2 dimensions");
     const Tensor *o = opt(offset);
-    if (!o) return scale.sizes().vec();
+    if (!o) return scale.sizes();
     TORCH_CHECK(o->scalar_type() == at::kFloat, "npu_trans_quant_param: offset must be float32, got ", o->scalar_type());
     TORCH_CHECK(o->dim() >= 1 && o->dim() <= 2, "npu_trans_quant_param: offset must have 1 or 2 dimensions");
     TORCH_CHECK(scale.numel() == o->numel() || scale.numel() == 1 || o->numel() == 1,
                 "npu_trans_quant_param: scale and offset must have the same number of elements, or one of them a single one");
-    return (o->numel() > scale.numel() ? *o : scale).sizes().vec();
+    return (o->numel() > scale.numel() ? *o : scale).sizes();
 }
 
 Tensor trans_quant_param_meta(const Tensor &scale, const optional<Tensor> &offset)
 {
-    return at::empty(trans_quant_param_shape(scale, offset), scale.options().dtype(at::kLong));
+    return new_empty(kMeta, scale, trans_quant_param_shape(scale, offset), at::kLong);
 }
 
 Tensor trans_quant_param_hip(const Tensor &scale, const optional<Tensor> &offset)
 {
     check_same_device("npu_trans_quant_param", {&scale, opt(offset)});
-    Tensor out = trans_quant_param_meta(scale, offset);
+    Tensor out = new_empty(kLaunch, scale, trans_quant_param_shape(scale, offset), at::kLong);
     if (out.numel() == 0) return out;
     c10::hip::HIPGuardMasqueradingAsCUDA guard(scale.device());
-    Tensor sc = scale.contiguous();
-    Tensor of = opt(offset) ? opt(offset)->contiguous() : Tensor();
+    Tensor sc = packed(scale);
+    Tensor of = opt(offset) ? packed(*opt(offset)) : Tensor();
     check_status(mi355_trans_quant_param(sc.data_ptr<float>(), sc.numel(), of.defined() ? of.data_ptr<float>() : nullptr,
                                          of.defined() ? of.numel() : 0, reinterpret_cast<uint64_t *>(out.data_ptr<int64_t>()),
                                          out.numel(), stream_of(scale)),
@@ -322,8 +335,8 @@ Tensor trans_quant_param_hip(const Tensor &scale, const optional<Tensor> &offset
 // ---------------------------------------------------------------- npu_quant_matmul
 
 struct QmmPlan {
-    std::vector<int64_t> out_shape;
-    std::vector<int64_t> batch;      // broadcast batch shape
+    at::DimVector out_shape;
+    at::DimVector batch;             // broadcast batch shape
     int64_t M, N, K;
     at::ScalarType out_dtype;
     bool a4w4;                       // both inputs int32 words of eight int4 values
@@ -411,7 +424,7 @@ QmmPlan quant_matmul_plan(const Tensor &x1, const Tensor &x2, const Tensor &scal
         TORCH_CHECK(!opt(pertoken_scale), "npu_quant_matmul: pertoken_scale is not applicable to int32 output");
     }
     auto b1 = x1.sizes().slice(0, x1.dim() - 2), b2 = x2.sizes().slice(0, x2.dim() - 2);
-    p.batch = at::infer_size(b1, b2);
+    if (!b1.empty() || !b2.empty()) p.batch = at::infer_size_dimvector(b1, b2);
     p.out_shape = p.batch;
     p.out_shape.push_back(p.M);
     p.out_shape.push_back(p.N);
@@ -423,7 +436,7 @@ Tensor quant_matmul_meta(const Tensor &x1, const Tensor &x2, const Tensor &scale
                          optional<at::ScalarType> output_dtype)
 {
     QmmPlan p = quant_matmul_plan(x1, x2, scale, offset, pertoken_scale, bias, output_dtype);
-    return at::empty(p.out_shape, x1.options().dtype(p.out_dtype));
+    return new_empty(kMeta, x1, p.out_shape, p.out_dtype);
 }
 
 // A 2-D int8 matrix the kernel can address: one of its strides is 1 and the other covers a row.
@@ -436,10 +449,10 @@ Tensor as_matrix(const Tensor &t)
 
 // Rows of a K that is a multiple of 16 which start off a 16-byte boundary (a view cut out of a wider tensor): copied once, since
 // the matrix kernels load 16 bytes at a time.  (Any other K is padded inside the C ABI.)
+bool rows_aligned(const Tensor &t, int64_t pitch) { return (pitch & 15) == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
 Tensor aligned_rows(const Tensor &t, int64_t K)
 {
-    const bool off = (t.stride(0) & 15) != 0 || (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) != 0;
-    return off && (K & 15) == 0 && K >= 128 ? t.clone(at::MemoryFormat::Contiguous) : t;
+    return !rows_aligned(t, t.stride(0)) && (K & 15) == 0 && K >= 128 ? t.clone(at::MemoryFormat::Contiguous) : t;
 }
 
 // int32 words of eight int4 values along the last dimension -> int8 of eight times that last dimension
@@ -464,7 +477,7 @@ Tensor quant_matmul_hip(const Tensor &x1, const Tensor &x2, const Tensor &scale,
     QmmPlan p = quant_matmul_plan(x1, x2, scale, offset, pertoken_scale, bias, output_dtype);
     check_same_device("npu_quant_matmul", {&x1, &x2, &scale, opt(pertoken_scale), opt(bias)});
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x1.device());
-    Tensor out = at::empty(p.out_shape, x1.options().dtype(p.out_dtype));
+    Tensor out = new_empty(kLaunch, x1, p.out_shape, p.out_dtype);
     if (out.numel() == 0) return out;
     Tensor xa = x1, xb = x2;
     if (p.a4w4) {
@@ -476,72 +489,67 @@ Tensor quant_matmul_hip(const Tensor &x1, const Tensor &x2, const Tensor &scale,
     const bool bf16 = p.out_dtype != at::kInt && !i8;     // a floating-point (dequantised) output
     Tensor scale_f, ps, b, qp;
     if (p.packed_scale) {
-        qp = scale.reshape({-1}).contiguous();            // an int64 scale carries its offset (any `offset` repeats it)
+        qp = packed(scale);                             // an int64 scale carries its offset (any `offset` repeats it)
     } else if (i8) {
         // float32 scale with int8 output: packed here the way the reference's module does it with
         // npu_trans_quant_param (linear_quant.py:104-108)
         qp = trans_quant_param_hip(scale, offset).reshape({-1});
     } else if (bf16) {
-        scale_f = scale.to(at::kFloat).contiguous();
-        if (const Tensor *t = opt(pertoken_scale)) ps = t->contiguous();
+        scale_f = packed(scale.scalar_type() == at::kFloat ? scale : scale.to(at::kFloat));
+        if (const Tensor *t = opt(pertoken_scale)) ps = packed(*t);
     }
-    if (const Tensor *t = opt(bias)) b = t->reshape({p.N}).contiguous();
+    if (const Tensor *t = opt(bias)) b = packed(*t);
     const int bias_dtype = !b.defined() ? MI355_BIAS_NONE
                            : b.scalar_type() == at::kInt ? MI355_BIAS_INT32
                            : b.scalar_type() == at::kFloat ? MI355_BIAS_FP32 : MI355_BIAS_BF16;
     const int out_dtype = i8 ? MI355_OUT_INT8
                           : p.out_dtype == at::kInt ? MI355_OUT_INT32 : p.out_dtype == at::kHalf ? MI355_OUT_FP16 : MI355_OUT_BF16;
+    const auto ptr = [](const Tensor &t) -> void * { return t.defined() ? t.data_ptr() : nullptr; };
+    // one product: `a_in` [m, K], `b_in` [K, N] into rows row0 .. row0 + m - 1 of the output
+    const auto product = [&](const Tensor &a_in, const Tensor &b_in, int64_t row0) {
+        Tensor a = aligned_rows(a_in.stride(1) == 1 && a_in.stride(0) >= p.K ? a_in : a_in.contiguous(), p.K);
+        Tensor w = as_matrix(b_in);
+        if (w.stride(0) == 1 && !rows_aligned(w, w.stride(1))) w = aligned_rows(w.t(), p.K).t();
+        const int64_t m = a.size(0);
+        const size_t ws_bytes = mi355_quant_matmul_workspace(m, p.N, p.K, w.stride(0), w.stride(1));
+        const Tensor ws = ws_bytes ? zeroed_workspace(xa, ws_bytes) : Tensor();
+        void *o = static_cast<char *>(out.data_ptr()) + row0 * p.N * (int64_t)out.element_size();
+        const int st = qp.defined()
+            ? mi355_quant_matmul_qparam(static_cast<int8_t *>(a.data_ptr()), static_cast<int8_t *>(w.data_ptr()), static_cast<uint64_t *>(qp.data_ptr()),
+                                        qp.numel(), ptr(b), bias_dtype, o, out_dtype, m, p.N, p.K, a.stride(0), w.stride(0), w.stride(1),
+                                        p.N, ptr(ws), ws_bytes, stream_of(x1))
+            : mi355_quant_matmul(static_cast<int8_t *>(a.data_ptr()), static_cast<int8_t *>(w.data_ptr()), static_cast<float *>(ptr(ps)),
+                                 static_cast<float *>(ptr(scale_f)), bf16 ? scale_f.numel() : 0, ptr(b), bias_dtype, o, out_dtype, m, p.N, p.K,
+                                 a.stride(0), w.stride(0), w.stride(1), p.N, ptr(ws), ws_bytes, stream_of(x1));
+        check_status(st, "npu_quant_matmul");
+    };
+    if (xa.dim() == 2 && xb.dim() == 2) {
+        product(xa, xb, 0);
+        return out;
+    }
     int64_t nb = 1;
     for (auto d : p.batch) nb *= d;
     // x1 with batch dimensions against a single weight matrix is one tall matmul
     bool x2_single = true;
     for (int64_t d = 0; d < xb.dim() - 2; d++) x2_single = x2_single && xb.size(d) == 1;
-    std::vector<std::pair<Tensor, Tensor>> jobs; // (a [m,K], b [K,N]) pairs writing consecutive rows of out
-    Tensor out2d = out.view({-1, p.N});
     if (x2_single) {
-        Tensor w2 = xb.dim() == 2 ? xb : xb.as_strided({p.K, p.N}, {xb.stride(-2), xb.stride(-1)});
-        jobs.emplace_back(xa.reshape({-1, p.K}), w2);
+        const Tensor a = xa.reshape({-1, p.K});
         // the [M] per-token scales apply to every matrix of the batch: one copy per matrix of the tall matmul
-        if (ps.defined() && p.M > 0 && jobs.back().first.size(0) != p.M) ps = ps.repeat({jobs.back().first.size(0) / p.M});
-    } else {
-        auto x1s = p.batch, x2s = p.batch;
-        x1s.push_back(p.M), x1s.push_back(p.K), x2s.push_back(p.K), x2s.push_back(p.N);
-        Tensor x1e = xa.expand(x1s).reshape({nb, p.M, p.K});
-        Tensor x2e = xb.expand(x2s);
-        x2e = x2e.reshape({nb, p.K, p.N});
-        for (int64_t i = 0; i < nb; i++) jobs.emplace_back(x1e[i], x2e[i]);
+        if (ps.defined() && p.M > 0 && a.size(0) != p.M) ps = ps.repeat({a.size(0) / p.M});
+        product(a, xb.dim() == 2 ? xb : xb.as_strided({p.K, p.N}, {xb.stride(-2), xb.stride(-1)}), 0);
+        return out;
     }
-    int64_t row0 = 0;
-    for (auto &job : jobs) {
-        Tensor a = job.first.stride(1) == 1 && job.first.stride(0) >= p.K ? job.first : job.first.contiguous();
-        a = aligned_rows(a, p.K);
-        Tensor w = as_matrix(job.second);
-        if (w.stride(0) == 1) w = aligned_rows(w.t(), p.K).t();
-        const int64_t m = a.size(0);
-        Tensor ws;
-        const size_t ws_bytes = mi355_quant_matmul_workspace(m, p.N, p.K, w.stride(0), w.stride(1));
-        if (ws_bytes) ws = zeroed_workspace(xa, ws_bytes);
-        Tensor o = out2d.narrow(0, row0, m);
-        const int st = qp.defined()
-            ? mi355_quant_matmul_qparam(a.data_ptr<int8_t>(), w.data_ptr<int8_t>(), reinterpret_cast<const uint64_t *>(qp.data_ptr<int64_t>()),
-                                        qp.numel(), b.defined() ? b.data_ptr() : nullptr, bias_dtype, o.data_ptr(), out_dtype, m, p.N,
-                                        p.K, a.stride(0), w.stride(0), w.stride(1), o.stride(0),
-                                        ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, stream_of(x1))
-            : mi355_quant_matmul(a.data_ptr<int8_t>(), w.data_ptr<int8_t>(), ps.defined() ? ps.data_ptr<float>() : nullptr,
-                                 bf16 ? scale_f.data_ptr<float>() : nullptr, bf16 ? scale_f.numel() : 0,
-                                 b.defined() ? b.data_ptr() : nullptr, bias_dtype, o.data_ptr(), out_dtype, m, p.N, p.K,
-                                 a.stride(0), w.stride(0), w.stride(1), o.stride(0), ws.defined() ? ws.data_ptr() : nullptr,
-                                 ws_bytes, stream_of(x1));
-        check_status(st, "npu_quant_matmul");
-        row0 += m;
-    }
+    at::DimVector x1s(p.batch), x2s(p.batch);
+    x1s.push_back(p.M), x1s.push_back(p.K), x2s.push_back(p.K), x2s.push_back(p.N);
+    const Tensor x1e = xa.expand(x1s).reshape({nb, p.M, p.K}), x2e = xb.expand(x2s).reshape({nb, p.K, p.N});
+    for (int64_t i = 0; i < nb; i++) product(x1e[i], x2e[i], i * p.M);
     return out;
 }
 
 // ---------------------------------------------------------------- npu_weight_quant_batchmatmul
 
 struct WqPlan {
-    std::vector<int64_t> out_shape;
+    at::DimVector out_shape;
     int64_t M, N, K, groups;
     int bits;
     bool packed_k;       // int4 words along K: weight [K/8, N], the transposed view of [N, K/8]
@@ -608,7 +616,7 @@ WqPlan weight_quant_plan(const Tensor &x, const Tensor &weight, const Tensor &an
             check_requant(*o, "quant_offset", false);
         }
     }
-    p.out_shape = x.sizes().vec();
+    p.out_shape = x.sizes();
     p.out_shape.back() = p.N;
     return p;
 }
@@ -633,9 +641,9 @@ Tensor weight_quant_hip(const Tensor &x, const Tensor &weight, const Tensor &ant
     check_same_device("npu_weight_quant_batchmatmul",
                       {&x, &weight, &antiquant_scale, opt(antiquant_offset), opt(quant_scale), opt(quant_offset), opt(bias)});
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    Tensor out = at::empty(p.out_shape, x.options());
+    Tensor out = new_empty(kLaunch, x, p.out_shape, x.scalar_type());
     if (out.numel() == 0) return out;
-    Tensor x2 = x.reshape({p.M, p.K});
+    Tensor x2 = x.dim() == 2 ? x : x.reshape({p.M, p.K});
     if (x2.stride(1) != 1 || x2.stride(0) < p.K) x2 = x2.contiguous();
     Tensor w;
     int64_t ldw_k, ldw_n;
@@ -656,21 +664,20 @@ Tensor weight_quant_hip(const Tensor &x, const Tensor &weight, const Tensor &ant
     Tensor s = antiquant_scale, o;
     if (const Tensor *t = opt(antiquant_offset)) o = *t;
     if (!p.packed_k || (o.defined() && o.strides() != s.strides())) {
-        s = s.contiguous();
-        if (o.defined()) o = o.contiguous();
+        s = packed(s);
+        if (o.defined()) o = packed(o);
     }
     const int64_t ld_param_g = s.dim() == 2 ? s.stride(0) : 0, ld_param_n = s.dim() == 2 ? s.stride(1) : s.stride(0);
     Tensor bias_c;
-    if (const Tensor *t = opt(bias)) bias_c = t->reshape({p.N}).contiguous();
-    Tensor out2d = out.view({p.M, p.N});
+    if (const Tensor *t = opt(bias)) bias_c = packed(*t);
     const size_t ws_bytes = mi355_weight_quant_matmul_workspace(p.M, p.N, p.K, p.bits, group_size);
     Tensor ws;
     if (ws_bytes) ws = zeroed_workspace(x, ws_bytes);
     check_status(mi355_weight_quant_matmul(x2.data_ptr(), x.scalar_type() == at::kHalf ? MI355_DTYPE_FP16 : MI355_DTYPE_BF16,
                                            w.data_ptr(), p.bits, s.data_ptr(), o.defined() ? o.data_ptr() : nullptr,
                                            bias_c.defined() ? bias_c.data_ptr() : nullptr,
-                                           out2d.data_ptr(), p.M, p.N, p.K, group_size, ld_param_g, ld_param_n, x2.stride(0),
-                                           ldw_k, ldw_n, out2d.stride(0),
+                                           out.data_ptr(), p.M, p.N, p.K, group_size, ld_param_g, ld_param_n, x2.stride(0),
+                                           ldw_k, ldw_n, p.N,
                                            ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? (size_t)ws.numel() : 0,
                                            stream_of(x)),
                  "npu_weight_quant_batchmatmul");
@@ -691,8 +698,8 @@ Tensor weight_quant_hip(const Tensor &x, const Tensor &weight, const Tensor &ant
         scale_f = qs->reshape({-1}).contiguous();
         if (const Tensor *qo = opt(quant_offset)) offset_f = at::clamp(at::round(qo->reshape({-1})), -256.0, 255.0).contiguous();
     }
-    Tensor out8 = at::empty(p.out_shape, x.options().dtype(at::kChar));
-    check_status(mi355_quantize(out2d.data_ptr(), x.scalar_type() == at::kHalf ? MI355_DTYPE_FP16 : MI355_DTYPE_BF16,
+    Tensor out8 = new_empty(kLaunch, x, p.out_shape, at::kChar);
+    check_status(mi355_quantize(out.data_ptr(), x.scalar_type() == at::kHalf ? MI355_DTYPE_FP16 : MI355_DTYPE_BF16,
                                 scale_f.data_ptr<float>(), scale_f.numel(), offset_f.defined() ? offset_f.data_ptr() : nullptr,
                                 MI355_DTYPE_FP32, offset_f.defined() ? offset_f.numel() : 0, out8.data_ptr(), MI355_Q_INT8, p.M, p.N, 1,
                                 0, stream_of(x)),
@@ -710,20 +717,22 @@ void swiglu_check(const Tensor &input, int64_t dim)
     TORCH_CHECK(input.size(-1) % 2 == 0, "npu_swiglu: the split dimension must be even");
 }
 
-Tensor swiglu_meta(const Tensor &input, int64_t dim)
+Tensor swiglu_alloc(Alloc how, const Tensor &input, int64_t dim)
 {
     swiglu_check(input, dim);
-    auto shape = input.sizes().vec();
+    at::DimVector shape(input.sizes());
     shape.back() /= 2;
-    return at::empty(shape, input.options());
+    return new_empty(how, input, shape, input.scalar_type());
 }
+
+Tensor swiglu_meta(const Tensor &input, int64_t dim) { return swiglu_alloc(kMeta, input, dim); }
 
 Tensor swiglu_hip(const Tensor &input, int64_t dim)
 {
-    Tensor out = swiglu_meta(input, dim);
+    Tensor out = swiglu_alloc(kLaunch, input, dim);
     if (out.numel() == 0) return out;
     c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    Tensor x = input.contiguous();
+    Tensor x = packed(input);
     const int64_t half = out.size(-1);
     check_status(mi355_swiglu(x.data_ptr(), out.data_ptr(), out.numel() / half, half, 2 * half, stream_of(input)), "npu_swiglu");
     return out;
@@ -765,13 +774,11 @@ void swiglu_quant_check(const Tensor &x, const optional<Tensor> &smooth_scales, 
     TORCH_CHECK(!dst_type.has_value() || *dst_type == at::kChar, "npu_swiglu_quant: only dst_type=torch.int8 is supported");
 }
 
-std::tuple<Tensor, Tensor> swiglu_quant_alloc(const Tensor &x)
+std::tuple<Tensor, Tensor> swiglu_quant_alloc(Alloc how, const Tensor &x)
 {
-    auto shape = x.sizes().vec();
+    at::DimVector shape(x.sizes());
     shape.back() /= 2;
-    auto scale_shape = shape;
-    scale_shape.pop_back();
-    return {at::empty(shape, x.options().dtype(at::kChar)), at::empty(scale_shape, x.options().dtype(at::kFloat))};
+    return {new_empty(how, x, shape, at::kChar), new_empty(how, x, x.sizes().slice(0, x.dim() - 1), at::kFloat)};
 }
 
 std::tuple<Tensor, Tensor> swiglu_quant_meta(const Tensor &x, const optional<Tensor> &smooth_scales,
@@ -781,7 +788,7 @@ std::tuple<Tensor, Tensor> swiglu_quant_meta(const Tensor &x, const optional<Ten
 {
     (void)activate_left;
     swiglu_quant_check(x, smooth_scales, offsets, group_index, quant_mode, group_list_type, dst_type);
-    return swiglu_quant_alloc(x);
+    return swiglu_quant_alloc(kMeta, x);
 }
 
 std::tuple<Tensor, Tensor> swiglu_quant_hip(const Tensor &x, const optional<Tensor> &smooth_scales,
@@ -792,7 +799,7 @@ std::tuple<Tensor, Tensor> swiglu_quant_hip(const Tensor &x, const optional<Tens
     swiglu_quant_check(x, smooth_scales, offsets, group_index, quant_mode, group_list_type, dst_type);
     check_same_device("npu_swiglu_quant", {&x, opt(smooth_scales), opt(group_index)});
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    auto [y, scale] = swiglu_quant_alloc(x);
+    auto [y, scale] = swiglu_quant_alloc(kLaunch, x);
     const int64_t half = x.size(-1) / 2;
     const int64_t rows = half ? y.numel() / half : 0;
     if (rows == 0 || half == 0) {
@@ -807,7 +814,7 @@ std::tuple<Tensor, Tensor> swiglu_quant_hip(const Tensor &x, const optional<Tens
         xin = xin.contiguous();
     }
     if (const Tensor *g = opt(group_index)) {
-        Tensor sm = opt(smooth_scales)->contiguous();
+        Tensor sm = packed(*opt(smooth_scales));
         Tensor gi = (group_list_type == 1 ? g->cumsum(0) : *g).to(at::kInt).contiguous();     // counts -> running totals
         check_status(mi355_swiglu_quant_grouped(xin.data_ptr(), activate_left ? 1 : 0, sm.data_ptr(), gi.data_ptr<int32_t>(),
                                                 gi.numel(), y.data_ptr<int8_t>(), scale.data_ptr<float>(), rows, half, row_stride,
@@ -816,7 +823,7 @@ std::tuple<Tensor, Tensor> swiglu_quant_hip(const Tensor &x, const optional<Tens
         return {y, scale};
     }
     if (const Tensor *smp = opt(smooth_scales)) {
-        Tensor sm = smp->contiguous();
+        Tensor sm = packed(*smp);
         check_status(mi355_swiglu_quant_smooth(xin.data_ptr(), activate_left ? 1 : 0, sm.data_ptr(), y.data_ptr<int8_t>(),
                                                scale.data_ptr<float>(), rows, half, row_stride, stream_of(x)),
                      "npu_swiglu_quant");
@@ -853,24 +860,30 @@ at::ScalarType anti_quant_check(const Tensor &x, const Tensor &scale, const opti
     return dst;
 }
 
+Tensor anti_quant_alloc(Alloc how, const Tensor &x, const Tensor &scale, const optional<Tensor> &offset,
+                        optional<at::ScalarType> dst_dtype, optional<at::ScalarType> src_dtype)
+{
+    const at::ScalarType dst = anti_quant_check(x, scale, offset, dst_dtype, src_dtype);
+    at::DimVector shape(x.sizes());
+    if (x.scalar_type() == at::kInt) shape.back() *= 8;
+    return new_empty(how, x, shape, dst);
+}
+
 Tensor anti_quant_meta(const Tensor &x, const Tensor &scale, const optional<Tensor> &offset,
                        optional<at::ScalarType> dst_dtype, optional<at::ScalarType> src_dtype)
 {
-    const at::ScalarType dst = anti_quant_check(x, scale, offset, dst_dtype, src_dtype);
-    auto shape = x.sizes().vec();
-    if (x.scalar_type() == at::kInt) shape.back() *= 8;
-    return at::empty(shape, x.options().dtype(dst));
+    return anti_quant_alloc(kMeta, x, scale, offset, dst_dtype, src_dtype);
 }
 
 Tensor anti_quant_hip(const Tensor &x, const Tensor &scale, const optional<Tensor> &offset,
                       optional<at::ScalarType> dst_dtype, optional<at::ScalarType> src_dtype)
 {
     check_same_device("npu_anti_quant", {&x, &scale, opt(offset)});
-    Tensor out = anti_quant_meta(x, scale, offset, dst_dtype, src_dtype);
+    Tensor out = anti_quant_alloc(kLaunch, x, scale, offset, dst_dtype, src_dtype);
     if (out.numel() == 0) return out;
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    Tensor xin = x.contiguous(), sc = scale.contiguous();
-    Tensor of = opt(offset) ? opt(offset)->contiguous() : Tensor();
+    Tensor xin = packed(x), sc = packed(scale);
+    Tensor of = opt(offset) ? packed(*opt(offset)) : Tensor();
     const int64_t cols = out.size(-1), rows = out.numel() / cols;
     const bool int4 = x.scalar_type() == at::kInt;
     check_status(mi355_anti_quant(xin.data_ptr(), int4 ? 4 : 8, sc.data_ptr<float>(), sc.numel(),
@@ -938,11 +951,11 @@ Tensor quantize_hip(const Tensor &x, const Tensor &scales, const optional<Tensor
 {
     check_same_device("npu_quantize", {&x, &scales, opt(zero_points)});
     const QuantizePlan pl = quantize_check(x, scales, zero_points, dtype, axis);
-    Tensor out = at::empty(x.sizes(), x.options().dtype(pl.out));
+    Tensor out = new_empty(kLaunch, x, x.sizes(), pl.out);
     if (out.numel() == 0) return out;
     c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    Tensor xin = x.contiguous();
-    Tensor sc = scales.to(at::kFloat).contiguous();            // a few hundred to a few thousand elements
+    Tensor xin = packed(x);
+    Tensor sc = packed(scales.scalar_type() == at::kFloat ? scales : scales.to(at::kFloat));            // a few hundred to a few thousand elements
     Tensor zp;                                                 // int32 and float32 zero points go to the kernel as they are
     if (const Tensor *z = opt(zero_points))
         zp = (z->scalar_type() == at::kInt || z->scalar_type() == at::kFloat ? *z : z->to(at::kFloat)).contiguous();

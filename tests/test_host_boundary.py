@@ -429,3 +429,51 @@ def test_weight_quant_workspace_query_follows_the_preferred_kernel():
         assert q(rows, 14336, 4096, 4, 128) == repack
         assert q(rows, 14336, 4096, 8, 0) == 0                # int8 tiled GEMM with enough tiles: no split, no workspace
     assert q(0, 14336, 4096, 4, 128) == 0 and q(16, 14336, 4096, 5, 128) == 0
+
+
+def test_direct_calls_keep_the_packets_behaviour(pa):
+    """Calls of torch.ops.npu.* take a native call slot (csrc/op_call.cpp); whatever it does not convert goes to the packet's own
+    call: __torch_function__ overrides and modes, dispatch modes, wrong arguments (same error), compilation, positional and
+    keyword forms, parameters, and results equal to the overload's."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    op = torch.ops.npu.npu_dynamic_quant
+    assert op is pa.npu_dynamic_quant and isinstance(op, torch._ops.OpOverloadPacket)
+    x = _m(3, 64, dtype=torch.bfloat16)
+    sm = _m(64, dtype=torch.bfloat16)
+    for args, kw in (((x,), {}), ((), {"input": x}), ((x,), {"smooth_scales": sm, "dst_type": torch.int8}),
+                     ((torch.nn.Parameter(x, requires_grad=False),), {"smooth_scales": None})):
+        got, want = op(*args, **kw), op.default(*args, **kw)
+        assert [(t.shape, t.dtype, t.device) for t in got] == [(t.shape, t.dtype, t.device) for t in want]
+    for args, kw in (((), {}), ((x, 5), {}), ((x,), {"foo": 1}), ((x,), {"dst_type": "a"}), ((torch.zeros(2, 4),), {}), ((None,), {}),
+                     ((_m(2, 4, dtype=torch.float32),), {})):
+        with pytest.raises(Exception) as direct:
+            op(*args, **kw)
+        with pytest.raises(type(direct.value)):
+            op.default(*args, **kw)
+    seen = []
+
+    class Fn(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(("function mode", func))
+            return func(*args, **(kwargs or {}))
+
+    class Disp(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(("dispatch mode", func))
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(("subclass", func))
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    with Fn():
+        op(x)
+    with Disp():
+        op(x)
+    op(x.as_subclass(Sub))
+    op(x, smooth_scales=sm.as_subclass(Sub))
+    assert [s[0] for s in seen] == ["function mode", "dispatch mode", "subclass", "subclass"]
+    assert seen[0][1] is op and seen[1][1] is op.default
