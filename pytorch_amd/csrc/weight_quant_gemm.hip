@@ -90,11 +90,13 @@ __global__ __launch_bounds__(512, 1) void wq_gemm_kernel(const WqGemmArgs p)
     const __amdgpu_buffer_rsrc_t rsrc_a =
         make_rsrc(p.x + (int64_t)m0 * p.ldx, (uint32_t)(((int64_t)(rows_a - 1) * p.ldx + p.K) * 2));
     const int rr = lane >> 3;
-    const uint32_t voff_a = (uint32_t)(rr * (int)p.ldx * 2 + (((lane & 7) ^ (((wave & 1) << 2) | (rr >> 1))) * 16));
+    const int k_lane = ((lane & 7) ^ (((wave & 1) << 2) | (rr >> 1))) * 8;      // first k of this lane's piece
+    const uint32_t voff_a = (uint32_t)((rr * (int)p.ldx + k_lane) * 2);
     const uint32_t unit_stride_a = 16u * (uint32_t)p.ldx;
     auto issue_a = [&](int s) {
         char *slot = lds + (s % 3) * A_BYTES;
-        const uint32_t vo = s < NSTG ? voff_a : kOutOfRange;
+        // (a K that is not a multiple of 128 ends in a partial or empty stage: the activations past K are zeros)
+        const uint32_t vo = s < NSTG && (s0 + s) * 64 + k_lane < p.K ? voff_a : kOutOfRange;
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             const int u = i * NW + wave;
@@ -500,7 +502,7 @@ WqGemmPlan make_wq_gemm_plan(int64_t M, int64_t N, int64_t K, int w_bits, int64_
     pl.grouped = group_size > 0 && group != K;
     const bool layout_ok = layout == 1 ? ldw_bytes >= row_bytes && (uint64_t)K * (uint64_t)ldw_bytes < (1ull << 32)
                                        : layout == 2 && w_bits == 8 && ldw >= K && (uint64_t)N * (uint64_t)ldw < (1ull << 32);
-    pl.ok = M > 32 && layout_ok && K >= 128 && K % 128 == 0 && group % 128 == 0 && N % 8 == 0 && ldw_bytes % 4 == 0 &&
+    pl.ok = M > 32 && layout_ok && K >= 128 && (K % 128 == 0 ? group % 128 == 0 : K % 8 == 0 && !pl.grouped && w_bits == 8) && N % 8 == 0 && ldw_bytes % 4 == 0 &&
             ldx % 8 == 0 && (x == nullptr || aligned(x, 16)) && (w == nullptr || aligned(w, 4)) &&
             (scale == nullptr || aligned(scale, 4)) && (offset == nullptr || aligned(offset, 4)) &&
             (uint64_t)128 * (uint64_t)ldx * 2 < (1ull << 31) &&
@@ -513,7 +515,7 @@ WqGemmPlan make_wq_gemm_plan(int64_t M, int64_t N, int64_t K, int w_bits, int64_
     pl.tiles_m = (int)((M + pl.bm - 1) / pl.bm);
     pl.tiles_n = pl.k_major ? (int)((N + 127) / 128) : (int)((row_bytes + 127) / 128);
     pl.unit_stages = pl.grouped ? (int)(group / 64) : 2;
-    pl.n_units = (int)(K / (64 * pl.unit_stages));
+    pl.n_units = (int)((K + 64 * pl.unit_stages - 1) / (64 * pl.unit_stages));
     const int64_t tiles = (int64_t)pl.tiles_m * pl.tiles_n;
     int64_t S = tiles < kNumCU ? kNumCU / tiles : 1;
     if (S > pl.n_units) S = pl.n_units;

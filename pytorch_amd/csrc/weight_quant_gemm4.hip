@@ -89,7 +89,7 @@ __global__ __launch_bounds__(512, 1) void wq_gemm4_kernel(const WqGemm4Args p)
     const int tile = strip * p.tiles_m + mb;
     const int m0 = mb * BM;
     const int n0 = strip * 256;
-    const int total_stages = p.K / BK;
+    const int total_stages = (p.K + BK - 1) / BK;              // int8: the last stage may be partial (zeros from x past K)
     const int units = total_stages / p.gstages;                // K is split in whole scale groups
     const int u0 = (int)((int64_t)units * chunk / p.S), u1 = (int)((int64_t)units * (chunk + 1) / p.S);
     const int s0 = u0 * p.gstages, NSTG = (u1 - u0) * p.gstages;
@@ -122,8 +122,9 @@ __global__ __launch_bounds__(512, 1) void wq_gemm4_kernel(const WqGemm4Args p)
             const int u = i * NW + wave;
             if (WBITS == 4 || i == 0) {                        // int8: eight units of activations, one per wavefront
                 const int row = WBITS == 4 ? 4 * u + (lane >> 4) : 8 * u + (lane >> 3);
-                const uint32_t vo = WBITS == 4 ? (uint32_t)(row * (int)p.ldx * 2 + (((lane & 15) ^ (row & 15)) * 16))
-                                               : (uint32_t)(row * (int)p.ldx * 2 + (((lane & 7) ^ (row & 7)) * 16));
+                uint32_t vo = WBITS == 4 ? (uint32_t)(row * (int)p.ldx * 2 + (((lane & 15) ^ (row & 15)) * 16))
+                                         : (uint32_t)(row * (int)p.ldx * 2 + (((lane & 7) ^ (row & 7)) * 16));
+                if (WBITS == 8 && (s0 + s) * BK + ((lane & 7) ^ (row & 7)) * 8 >= p.K) vo = kOutOfRange;
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_void *)(sa + u * 1024), 16, vo, (uint32_t)(s0 + s) * (uint32_t)(BK * 2), 0, 0);
             }
             if constexpr (WBITS == 4) {
@@ -519,7 +520,7 @@ WqGemm4Plan make_wq_gemm4_plan(int64_t M, int64_t N, int64_t K, int w_bits, int6
     const int64_t bk = w_bits == 4 ? 128 : 64, strip_bytes = w_bits == 4 ? 128 : 256;
     const int64_t group = group_size > 0 ? group_size : K;
     const bool grouped = group_size > 0 && group != K;
-    pl.ok = knob(kKnobWqGemm4Off) != 1 && (w_bits == 4 || w_bits == 8) && M > 32 && K >= 128 && K % 128 == 0 &&
+    pl.ok = knob(kKnobWqGemm4Off) != 1 && (w_bits == 4 || w_bits == 8) && M > 32 && K >= 128 && (K % 128 == 0 || (w_bits == 8 && !grouped && K % 8 == 0)) &&
             N % (w_bits == 4 ? 8 : 4) == 0 && (!grouped || group % bk == 0) &&
             ldw_bytes >= row_bytes && ldw_bytes % 16 == 0 && ldx % 8 == 0 && (x == nullptr || aligned(x, 16)) &&
             (w == nullptr || aligned(w, 16)) && (scale == nullptr || aligned(scale, 4)) && (offset == nullptr || aligned(offset, 4)) &&
@@ -527,7 +528,7 @@ WqGemm4Plan make_wq_gemm4_plan(int64_t M, int64_t N, int64_t K, int w_bits, int6
             (uint64_t)(K / group) * (uint64_t)N * 2 < (1ull << 31) && M <= 0x7fffffff;
     if (!pl.ok) return pl;
     pl.strips = (int)((row_bytes + strip_bytes - 1) / strip_bytes);
-    const int64_t stages = K / bk;
+    const int64_t stages = (K + bk - 1) / bk;
     const int64_t units = grouped ? K / group : stages;
     // few tiles: split K in whole scale groups (per channel: in equal numbers of stages)
     pl.bm = 64;

@@ -31,7 +31,7 @@ __global__ __launch_bounds__(512) void wq_kmajor_decode_kernel(const WqKmDecodeA
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    const int KT = p.K / kStep;
+    const int KT = (p.K + kStep - 1) / kStep;                             // the last step may be partial: zeros from x past K
     const int s0 = KT * wave / 8, ns = KT * (wave + 1) / 8 - s0;          // this wavefront's steps (at most NS)
     const int strips = (p.N + 15) / 16;
     const int my_strips = (strips - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(512) void wq_kmajor_decode_kernel(const WqKmDecodeA
             for (int i = 0; i < 4; i++) {
                 const int row = mt * 16 + 4 * i + (lane >> 4);
                 xf[j][mt][i] = __builtin_amdgcn_raw_buffer_load_b128(
-                    rsrc_x, j < ns && row < p.M ? (uint32_t)((row * (int)p.ldx) * 2 + (lane & 15) * 16) : kOutOfRange,
+                    rsrc_x, j < ns && row < p.M && (s0 + j) * kStep + (lane & 15) * 8 < p.K ? (uint32_t)((row * (int)p.ldx) * 2 + (lane & 15) * 16) : kOutOfRange,
                     (uint32_t)(s0 + j) * (kStep * 2), 0);
             }
 
@@ -202,7 +202,7 @@ int launch(const WqKmDecodeArgs &p, hipStream_t s)
 template <int ACT>
 int launch_act(const WqKmDecodeArgs &p, hipStream_t s)
 {
-    const int ns = (p.K / kStep + 7) / 8;
+    const int ns = ((p.K + kStep - 1) / kStep + 7) / 8;
     if (p.M <= 16) return ns <= 4 ? launch<1, 4, ACT>(p, s) : launch<1, 8, ACT>(p, s);
     return launch<2, 4, ACT>(p, s);
 }
@@ -213,9 +213,9 @@ bool wq_kmajor_decode_shape(int64_t M, int64_t N, int64_t K, int64_t group_size)
 {
     if (knob(kKnobWqDecodeOff) == 1 || knob(kKnobWqSplit) != 0) return false;
     if (group_size > 0 && group_size != K) return false;                  // one scale per column
-    if (M < 1 || M > 32 || K % kStep != 0 || K < 8 * kStep || N < 2048 || N % 4 != 0) return false;
+    if (M < 1 || M > 32 || K % 16 != 0 || K < 8 * kStep || N < 2048 || N % 4 != 0) return false;
     // the activations of a wavefront's eighth of K stay in registers: 8 steps with one tile of 16 rows, 4 with two
-    const int64_t steps = (K / kStep + 7) / 8;
+    const int64_t steps = ((K + kStep - 1) / kStep + 7) / 8;
     return M <= 16 ? steps <= 8 : steps <= 4;
 }
 

@@ -209,7 +209,8 @@ __global__ __launch_bounds__(W * KS * 64) void wq_stream_kernel(const WqArgs p)
             char *dst = xs + (((r >> 4) * 64 + (r & 15)) << 4);
 #pragma unroll 4
             for (int q = lane; q < pieces; q += 64) {
-                const u32x4 v = *reinterpret_cast<const u32x4 *>(xrow + q * 8);
+                // (past K: zeros)
+                const u32x4 v = cstep0 * 32 + q * 8 < p.K ? *reinterpret_cast<const u32x4 *>(xrow + q * 8) : u32x4{0u, 0u, 0u, 0u};
                 *reinterpret_cast<u32x4 *>(dst + ((((q >> 2) * MT) * 64 + (q & 3) * 16) << 4)) = v;
             }
         }
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(512) void wq_kmajor_kernel(const WqArgs p)
             for (int h = 0; h < XH; h++) {
                 const int q = lane + 64 * h;
                 const int st = ch * CH + (q >> 4);
-                const bool ok = r < rows_valid && st < nsteps;
+                const bool ok = r < rows_valid && st < nsteps && (step0 + ch * CH) * 128 + q * 8 < p.K;
                 // lane-dependent part in the vector offset, the chunk's position in the scalar offset
                 xst[i][h] = __builtin_amdgcn_raw_buffer_load_b128(
                     rsrc_x, ok ? (uint32_t)((r * (int)p.ldx + q * 8) * 2) : kOutOfRange, (uint32_t)(step0 + ch * CH) * 256u, 0);
@@ -560,7 +561,9 @@ WqPlan make_plan(int64_t M, int64_t N, int64_t K, int w_bits, int64_t group_size
     const int64_t row_bytes = w_bits == 4 ? N / 2 : N;
     const int64_t ldw_bytes = w_bits == 4 ? ldw_k * 4 : ldw_k;
     const int64_t group = group_size > 0 ? group_size : K;
-    pl.fast = K > 0 && K % 32 == 0 && group % 32 == 0 && n_major && row_bytes % 16 == 0 && ldw_bytes % 16 == 0 &&
+    // (int8 with one scale per column: any multiple of 8, the activations past K count as zeros)
+    const bool ragged = w_bits == 8 && group == K && K % 128 != 0 && K % 8 == 0;
+    pl.fast = K > 0 && (ragged || (K % 32 == 0 && group % 32 == 0)) && n_major && row_bytes % 16 == 0 && ldw_bytes % 16 == 0 &&
               ldx % 8 == 0 && (x == nullptr || aligned(x, 16)) && (w == nullptr || aligned(w, 16)) &&
               (scale == nullptr || aligned(scale, 16)) && (offset == nullptr || aligned(offset, 16)) &&
               (uint64_t)K * (uint64_t)ldw_bytes < (1ull << 32) && (uint64_t)M * (uint64_t)ldx * 2 < (1ull << 32) &&
@@ -571,10 +574,10 @@ WqPlan make_plan(int64_t M, int64_t N, int64_t K, int w_bits, int64_t group_size
     pl.mchunks = (int)((M + pl.mt * 16 - 1) / (pl.mt * 16));
     const bool grouped = group_size > 0 && group != K;
     // loop body of 4 steps when a scale group (per channel: the whole of K) is a whole number of them, else 1 step
-    const int64_t span = (grouped ? group : K) / 32;
+    const int64_t span = ragged ? 4 : (grouped ? group : K) / 32;
     pl.bs = span % 4 == 0 ? 4 : 1;
     pl.unit_steps = grouped ? (int)(group / 32) : pl.bs;
-    pl.n_units = (int)(K / (32 * pl.unit_steps));
+    pl.n_units = (int)((K + 32 * pl.unit_steps - 1) / (32 * pl.unit_steps));
     // W adjacent strips per workgroup; the remaining wavefronts slice K.  Pairs of strips read DRAM markedly
     // better, but halve the number of tiles: with few strips that means a deeper split of K and a longer exchange.
     pl.w = pl.strips >= 112 ? 2 : 1;
@@ -675,7 +678,8 @@ WqKmPlan make_kmajor_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, i
     WqKmPlan pl{};
     const int64_t group = group_size > 0 ? group_size : K;
     // N % 4: the output side stores quads of four columns (other N take the generic kernel)
-    pl.fast = K > 0 && K % 128 == 0 && group % 128 == 0 && N % 4 == 0 && ldw_n >= K && ldw_n % 16 == 0 && ldx % 8 == 0 &&
+    // (one scale per column: any K of whole 16-byte pieces, the activations past K count as zeros)
+    pl.fast = K > 0 && (K % 128 == 0 ? group % 128 == 0 : group == K && K % 16 == 0) && N % 4 == 0 && ldw_n >= K && ldw_n % 16 == 0 && ldx % 8 == 0 &&
               (x == nullptr || aligned(x, 16)) && (w == nullptr || aligned(w, 16)) &&
               (uint64_t)N * (uint64_t)ldw_n < (1ull << 32) && (uint64_t)M * (uint64_t)ldx * 2 < (1ull << 32);
     if (!pl.fast) return pl;
@@ -684,7 +688,7 @@ WqKmPlan make_kmajor_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, i
     pl.tiles = (int)((N + 127) / 128);
     pl.grouped = group_size > 0 && group != K;
     pl.unit_steps = pl.grouped ? (int)(group / 128) : 1;
-    pl.n_units = (int)(K / (128 * pl.unit_steps));
+    pl.n_units = (int)((K + 128 * pl.unit_steps - 1) / (128 * pl.unit_steps));
     int S = kNumCU / (pl.tiles * pl.mchunks);
     if (S > pl.n_units) S = pl.n_units;
     if (S > 16) S = 16;

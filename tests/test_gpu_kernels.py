@@ -658,6 +658,23 @@ def test_w8a16(capi, golden, M, K, N):
     print("w8a16", M, K, N, stats)
 
 
+@pytest.mark.parametrize("nk", [True, False])
+@pytest.mark.parametrize("M,K,N,f16", [(3, 1040, 2048, False), (20, 1168, 2052, True), (16, 9120, 1024, True), (30, 4464, 264, False),
+                                       (40, 2496, 1024, False), (65, 144, 320, True), (130, 1944, 600, False), (7, 1136, 520, True)])
+def test_w8a16_partial_last_step(capi, golden, M, K, N, f16, nk):
+    """int8 weights, one scale per column, K not a multiple of 128: every kernel of both layouts (decode, streaming, tiled, with
+    and without a split of K) ends in a partial step whose activations past K count as zeros.  The activations are a view of a
+    wider matrix whose columns past K hold NaN."""
+    d = workloads.w8a16_inputs(seed=M + K, M=M, K=K, N=N, weight_nk=nk)
+    dt = torch.float16 if f16 else torch.bfloat16
+    d = {k: (v.to(dt) if v.is_floating_point() else v) for k, v in d.items()}
+    xw = torch.full((M, K + 64), float("nan"), dtype=dt, device="cuda")
+    xw[:, :K] = d["x"].cuda()
+    out = capi.weight_quant_matmul(xw[:, :K], d["weight"].cuda(), d["antiquant_scale"].cuda(), d["antiquant_offset"].cuda())
+    _, want = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]), _bits(d["antiquant_offset"]), dtype="fp16" if f16 else "bf16")
+    bf16_gate(out, torch.from_numpy(want))
+
+
 def test_w8a16_kmajor_and_no_offset(capi, golden):
     d = workloads.w8a16_inputs(seed=3, M=8, K=1024, N=192, weight_nk=True)
     out = capi.weight_quant_matmul(d["x"].cuda(), d["weight"].cuda(), d["antiquant_scale"].cuda(),
