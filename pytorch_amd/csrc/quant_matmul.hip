@@ -312,19 +312,23 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
         // contiguous KiB of LDS (piece g of row r at g * 256 + r * 16), which is what a direct load writes (lane l at
         // l * 16 behind the instruction's base).
         const int st_row = lane & 15, st_g = lane >> 4;
-        auto stage = [&](int ch) {
+        auto stage_pieces = [&](int ch, auto last_c) {
             char *buf = lds + (ch & 1) * XBUF;
-            const bool last = (ch + 1) * CH * BK > kbytes;                   // reaches past the end of K: a scalar test per chunk
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int combo = wave * 4 + j;                              // (group of 16 rows, group of 4 pieces)
                 const int mt = combo % WTM, qg = combo / WTM;                // pieces 4 qg .. 4 qg + 3: step qg / 2, half qg % 2
                 const int row = mt * 16 + st_row, q = qg * 4 + st_g;
-                uint32_t vo = (uint32_t)(row * (int)p.lda + q * 16);
-                if (last && ch * CH * BK + q * 16 >= kbytes) vo = kOutOfRange;
+                const bool past = decltype(last_c)::value && ch * CH * BK + q * 16 >= kbytes;
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_void *)(buf + (((qg >> 1) * WTM + mt) * 2 + (qg & 1)) * 1024), 16,
-                                                         vo, (uint32_t)(kt0 + ch * CH) * BK, 0, 0);
+                                                         past ? kOutOfRange : (uint32_t)(row * (int)p.lda + q * 16),
+                                                         (uint32_t)(kt0 + ch * CH) * BK, 0, 0);
             }
+        };
+        // only the chunk that reaches past the end of K (a scalar test) compares its pieces with it
+        auto stage = [&](int ch) {
+            if ((ch + 1) * CH * BK > kbytes) stage_pieces(ch, std::true_type{});
+            else stage_pieces(ch, std::false_type{});
         };
         // a chunk has landed: at most the `younger` loads issued behind its four are outstanding; and every wavefront is
         // done with the other buffer

@@ -503,7 +503,11 @@ def test_quant_matmul_long_k_plans(capi, M, K, N):
 
 QMM_DECODE_CASES = [(1, 4096, 4096), (7, 1024, 2048), (16, 1152, 2056), (5, 14336, 4096), (3, 11008, 2048), (16, 16384, 2048),
                     (1, 1024, 8200), (17, 4096, 6144), (32, 8192, 2048), (30, 2176, 4100), (33, 4096, 4104), (64, 2048, 5120),
-                    (48, 1024, 16384)]
+                    (48, 1024, 16384),
+                    # several passes over K, narrow outputs
+                    (16, 18432, 520), (20, 10240, 1288), (32, 14336, 4100), (64, 5120, 300), (40, 9344, 3072), (2, 1280, 16),
+                    # several chunks of rows
+                    (45, 1024, 1284), (129, 2048, 900), (100, 4096, 1540), (250, 1152, 516)]
 
 
 @pytest.mark.parametrize("M,K,N", QMM_DECODE_CASES)
