@@ -73,7 +73,7 @@ struct QmmArgs {
     const uint64_t *qparam;    // packed quantisation parameters [scale_len] (replace `scale`), or null
     int out_i8;                // re-quantised int8 output (needs qparam)
     int stream_out;            // 16-bit and int8 outputs with aligned rows: non-temporal row stores (chosen by the launcher)
-    int tiles_m, tiles_n, tiles_per_xcd;
+    int tiles_m, tiles_n, items_per_xcd;
     int S;                     // workgroups that share the K range of a tile
     int32_t *partial;          // workspace [tile][chunk][wavefront][accumulator quad][lane] int32x4 (S > 1)
     uint32_t *counter;         // workspace [tile], zero on entry, left zero (S > 1)
@@ -129,13 +129,14 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     extern __shared__ __attribute__((aligned(1024))) char lds[];
 
     // XCD-aware rasterisation: workgroups are dealt round-robin to the 8 XCDs, each of which has
-    // a private L2; give every XCD a contiguous run of tiles, M fastest, so its workgroups
-    // share weight columns.
-    const int xcd = blockIdx.x & 7;
-    const int slot = blockIdx.x >> 3;
-    const int tile = xcd * p.tiles_per_xcd + slot % p.tiles_per_xcd;
-    const int chunk = slot / p.tiles_per_xcd;                // K chunk of this workgroup (split K)
-    if (tile >= p.tiles_m * p.tiles_n) return;
+    // a private L2; give every XCD a contiguous run of (tile, K chunk) items, chunks fastest, then M, so its workgroups
+    // share weight columns and the chunks of a tile meet in one L2.  The items, not the tiles, are dealt out evenly: 84 tiles
+    // split three ways are 32 workgroups on an XCD's 32 CUs, where eleven tiles times three chunks were 33, i.e. a second
+    // round (256x11392x2688: 33 us instead of 21).
+    const int item = (blockIdx.x & 7) * p.items_per_xcd + (blockIdx.x >> 3);
+    if (item >= p.tiles_m * p.tiles_n * p.S) return;
+    const int tile = p.S == 1 ? item : item / p.S;
+    const int chunk = item - tile * p.S;                     // K chunk of this workgroup (split K)
     const int m0 = (tile % p.tiles_m) * BM;
     const int n0 = (tile / p.tiles_m) * BN;
 
@@ -289,6 +290,10 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
         constexpr int TBUF = 2048;
         constexpr int R = 4;                                    // weight steps in flight per wavefront
         constexpr int RING = R + 1;                             // ... and the one being read
+        // One row tile: every weight byte is read once, so it need not displace anything (non-temporal).  With several row tiles
+        // (EPI 1) their workgroups sit side by side on an XCD and the first one's lines must stay in its L2 for the others
+        // (256x11392x2688, four row tiles: 40 us when each of them went to memory, 24 with ordinary loads).
+        constexpr int POLICY = EPI == 1 ? 0 : 2;
         char *const tbuf = lds + 2 * XBUF + wave * (RING * TBUF);
         const int c16 = lane & 15, g4 = lane >> 4;
         uint32_t voff_w[2];
@@ -304,8 +309,8 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             const bool ok = st < KT;
             const uint32_t kb = (uint32_t)(kt0 + st) * BK;
             char *dst = tbuf + slot * TBUF;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_void *)dst, 16, ok ? voff_w[0] : kOutOfRange, kb, 0, 2);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_void *)(dst + 1024), 16, ok ? voff_w[1] : kOutOfRange, kb, 0, 2);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_void *)dst, 16, ok ? voff_w[0] : kOutOfRange, kb, 0, POLICY);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_void *)(dst + 1024), 16, ok ? voff_w[1] : kOutOfRange, kb, 0, POLICY);
         };
         // staging: the chunk is 64 rows x 512 bytes = 2048 pieces of 16 bytes, four per thread, by direct-to-LDS loads.  A
         // wavefront's instruction takes 16 rows x 4 consecutive pieces (64 bytes of a row): in fragment order those are one
@@ -958,13 +963,13 @@ int launch_qmm(QmmArgs p, hipStream_t s)
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + BN - 1) / BN;
     const int tiles = p.tiles_m * p.tiles_n;
-    p.tiles_per_xcd = (tiles + 7) / 8;
+    p.items_per_xcd = (tiles * p.S + 7) / 8;
     if (p.S > 1 && (uint64_t)p.S * BM * BN * 4 >= (1ull << 32)) return MI355_ERR_UNSUPPORTED;
     auto kern = qmm_kernel<WGM, WGN, WTM, WTN, NS, LOOP, EPI>;
     static int attr_status = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     if (attr_status != hipSuccess) return MI355_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3(8 * p.tiles_per_xcd * p.S), dim3(WGM * WGN * 64), lds_bytes, s, p);
+    hipLaunchKernelGGL(kern, dim3(8 * p.items_per_xcd), dim3(WGM * WGN * 64), lds_bytes, s, p);
     return check_launch();
 }
 
@@ -979,10 +984,10 @@ struct TileChoice {
     double single_us, round_us;
     int whole;
 };
-constexpr TileChoice kTiles[] = {{256, 256, 256, 58.0, 59.0, 0}, {256, 224, 256, 52.5, 52.0, 0}, {256, 192, 256, 44.5, 45.5, 0},
-                                 {128, 320, 256, 48.0, 43.0, 0}, {128, 256, 256, 40.0, 45.6, 0}, {128, 192, 512, 55.8, 58.8, 0},
-                                 {128, 128, 512, 40.0, 43.3, 0}, {64, 256, 512, 40.0, 52.6, 0},  {64, 128, 512, 24.0, 30.0, 0},
-                                 {128, 192, 256, 32.0, 32.0, 1}, {128, 128, 256, 24.0, 24.8, 1}};
+constexpr TileChoice kTiles[] = {{256, 256, 256, 48.6, 50.0, 0}, {256, 224, 256, 40.1, 42.9, 0}, {256, 192, 256, 39.0, 37.1, 0},
+                                 {128, 320, 256, 41.8, 38.3, 0}, {128, 256, 256, 38.3, 36.2, 0}, {128, 192, 512, 38.1, 53.9, 0},
+                                 {128, 128, 512, 31.4, 35.7, 0}, {64, 256, 512, 36.8, 47.9, 0},  {64, 128, 512, 25.1, 20.6, 0},
+                                 {128, 192, 256, 30.5, 26.2, 1}, {128, 128, 256, 22.7, 19.2, 1}};
 
 // Workspace layout: [arrival counters | split-K partial sums | transposed weight | padded operands].
 struct QmmPlan {
@@ -998,16 +1003,13 @@ struct QmmPlan {
 // bounds small tiles on a long K (64x128 tiles on 1024x14336x4096: 1.4 GB, 107 us), and a split of K moves
 // wgs x bm x bn x 4 bytes of partial sums out and in again, the S - 1 foreign chunks of a tile through the one workgroup
 // that collects them (128x256 tiles split twelve ways: 39 us where a four-way split of 64x128 tiles takes 25).
-// Constants fitted to sweeps over tile x split on M = 128 .. 2048, K = 8192 .. 28672 and on M = 80 .. 512 over the
-// projections of transformer layers with K = 4096 .. 14336 (46 shapes: the estimate's choice is 0.7 % slower than the
-// measured best on average and 8 % at worst; at K = 4096 without a split the estimate is the table itself).
+// Table and constants are fitted to sweeps over every tile and split of 290 shapes, M = 33 .. 2048, K = 1024 .. 14336, N = 1024
+// .. 28672 drawn evenly over their logarithms: the estimate's choice is 0.7 % slower than the measured best on average and
+// 17 % at worst (4 % and 25 % with constants fitted to layer projections of K = 4096 .. 14336 only).
 constexpr size_t kMaxPartialBytes = (size_t)128 << 20;
 constexpr uint64_t kStreamOutMaxBytes = (uint64_t)32 << 20;     // the L2s of the eight XCDs together
-constexpr double kBaseUs = 6.0, kL2BytesPerUs = 12e6, kExchangeUs = 1.0, kExchangeBytesPerUs = 10e6, kCollectorBytesPerUs = 100e3;
-constexpr double kAloneOnCu = 0.85;
-// a split of a whole-stage tile measured 2-4 us above what the terms below give (its partial sums are 64-96 KiB per
-// workgroup); and of two plans with the same estimate the one that leaves fewer CUs idle is the faster one
-constexpr double kWholeSplitUs = 3.0, kIdleCuUs = 2.0;
+constexpr double kBaseUs = 4.0, kL2BytesPerUs = 13.1e6, kExchangeUs = 2.9, kExchangeBytesPerUs = 6.0e6, kCollectorBytesPerUs = 163e3;
+constexpr double kAloneOnCu = 0.78, kStreamAloneOnCu = 0.70;    // 64-row tiles alone on their CU run the streaming loop or deep rings
 
 void choose_tile_and_split(int64_t M, int64_t N, int64_t K, bool may_split, size_t partial_cap, TileChoice *tile, int *split)
 {
@@ -1045,14 +1047,13 @@ void choose_tile_and_split(int64_t M, int64_t N, int64_t K, bool may_split, size
             // time, as if all did (128x128 split six ways, 384 workgroups: 42 us where eight ways, 512, take 38)
             if (c.slots == 512 && rounds == 1 && wgs > 256) loop_us *= 512.0 / (double)wgs;
             // ... and with at most 256 every workgroup has a CU to itself
-            if (c.slots == 512 && wgs <= 256) loop_us *= kAloneOnCu;
+            if (c.slots == 512 && wgs <= 256) loop_us *= c.bm == 64 ? kStreamAloneOnCu : kAloneOnCu;
             double cost = kBaseUs + loop_us;
             const double l2 = kBaseUs + (double)tiles * (c.bm + c.bn) * (double)K / kL2BytesPerUs;
             if (l2 > cost) cost = l2;
             if (s_eff > 1)
                 cost += kExchangeUs + (double)wgs * c.bm * c.bn * 8.0 / kExchangeBytesPerUs +
-                        (double)(s_eff - 1) * c.bm * c.bn * 4.0 / kCollectorBytesPerUs + (c.whole ? kWholeSplitUs : 0.0);
-            if (wgs < 256) cost += kIdleCuUs * (1.0 - (double)wgs / 256.0);
+                        (double)(s_eff - 1) * c.bm * c.bn * 4.0 / kCollectorBytesPerUs;
             if (cost < best_cost) {
                 best_cost = cost;
                 *tile = c;
@@ -1298,7 +1299,10 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
         const int dk = knob(kKnobQmmDeepOff);              // 1: neither; 2: the ring instead of the streaming loop
         const bool deep = wgs <= 256 && dk != 1;
         if (deep && c.bm == 64 && c.bn == 256) return launch_qmm<1, 8, 4, 2, 3>(p, s);
-        if (deep && c.bm == 64 && c.bn == 128) return dk == 2 ? launch_qmm<1, 8, 4, 1, 4>(p, s) : launch_qmm<1, 8, 4, 1, -1>(p, s);
+        if (deep && c.bm == 64 && c.bn == 128) {
+            if (dk == 2) return launch_qmm<1, 8, 4, 1, 4>(p, s);
+            return p.M <= 64 ? launch_qmm<1, 8, 4, 1, -1>(p, s) : launch_qmm<1, 8, 4, 1, -1, 0, 1>(p, s);
+        }
     }
     MI355_QMM_CASE(64, 256, 1, 8)
     MI355_QMM_CASE(64, 128, 1, 8)

@@ -95,8 +95,13 @@ __global__ __launch_bounds__(512, 1) void wq_gemm_kernel(const WqGemmArgs p)
     const uint32_t unit_stride_a = 16u * (uint32_t)p.ldx;
     auto issue_a = [&](int s) {
         char *slot = lds + (s % 3) * A_BYTES;
-        // (a K that is not a multiple of 128 ends in a partial or empty stage: the activations past K are zeros)
-        const uint32_t vo = s < NSTG && (s0 + s) * 64 + k_lane < p.K ? voff_a : kOutOfRange;
+        uint32_t vo = s < NSTG ? voff_a : kOutOfRange;
+        // a K that is not a multiple of 128 ends in a partial or empty stage: the activations past K are zeros (a scalar test,
+        // the lanes compare in that stage only)
+        if ((s0 + s) * 64 + 64 > p.K) {
+            asm volatile("" : "+v"(vo));
+            vo = (s0 + s) * 64 + k_lane < p.K ? vo : kOutOfRange;
+        }
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             const int u = i * NW + wave;
