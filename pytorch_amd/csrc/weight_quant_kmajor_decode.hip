@@ -1,6 +1,6 @@
 // npu_weight_quant_batchmatmul for decode-sized batches of int8 weights stored [N, K] (the transposed view that
 // torch_npu's LinearWeightQuant passes, torch_npu/contrib/module/linear_weight_quant.py:106), one scale / offset per
-// output column, at most 32 activation rows.
+// output column, decode-sized batches.
 //
 // The structure is that of the decode kernel of npu_quant_matmul (quant_matmul_decode.hip): a workgroup of eight
 // wavefronts owns strips of 16 weight rows (= 16 output columns) over the whole of K, wavefront w the w-th eighth of K; at
@@ -9,7 +9,8 @@
 // step) and are turned into MFMA operand order through a private swizzled LDS tile; the wavefront's slice of the
 // activations is loaded once, turned around the same way and kept in registers for all strips; the eight partial sums of
 // a strip meet in LDS (two areas in turn, one barrier per strip) and the first wavefronts write it out while the others go
-// on.  No split of K over workgroups, no workspace, no barrier in front of the data.
+// on.  No split of K over workgroups, no workspace, no barrier in front of the data.  A K whose activations do not fit the
+// registers is walked in passes (the strips' sums wait in LDS), and the rows of a narrow output are cut into chunks, as there.
 //
 // Arithmetic as in the other weight-only kernels: the MFMA multiplies the activations by the integer weight, which is an
 // exact bf16 / fp16 number, and  out = scale * (P + offset * X) + bias  in float32 with P the sum of products and X the
@@ -22,22 +23,27 @@ namespace {
 
 constexpr int kStep = 128;                      // weight bytes (= k) per step: four MFMAs of 32
 constexpr int kMaxWorkgroups = 256;
+constexpr int kMaxLds = 160 * 1024;
+constexpr int64_t kMaxChunkBytes = 128 << 20;   // what a launch may read through the L2 (about 10 us)
 
-// MT tiles of 16 activation rows; NS (even) steps per wavefront and strip, PF of them in flight; ACT 0 bf16, 1 fp16.
-template <int MT, int NS, int PF, int ACT>
+// MT tiles of 16 activation rows; NS (even) steps per wavefront, pass and strip, PF of them in flight; ACT 0 bf16, 1 fp16;
+// PASSES: K may take several passes.
+template <int MT, int NS, int PF, int ACT, bool PASSES>
 __global__ __launch_bounds__(512) void wq_kmajor_decode_kernel(const WqKmDecodeArgs p)
 {
-    static_assert(NS % 2 == 0 && NS % PF == 0 && PF % 2 == 0, "static ring slots and LDS buffer parities");
+    static_assert(NS % 2 == 0 && NS % PF == 0 && PF % 2 == 0 && PF <= NS, "static ring slots and LDS buffer parities");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
     const int KT = (p.K + kStep - 1) / kStep;                             // the last step may be partial: zeros from x past K
-    const int s0 = KT * wave / 8, ns = KT * (wave + 1) / 8 - s0;          // this wavefront's steps (at most NS)
+    const int s0 = KT * wave / 8, ns = KT * (wave + 1) / 8 - s0;          // this wavefront's steps (at most NS per pass)
+    const int passes = PASSES ? ((KT + 7) / 8 + NS - 1) / NS : 1;
+    const int m_base = (int)blockIdx.y * 16 * MT, rows = min(16 * MT, p.M - m_base);          // this workgroup's activation rows
     const int strips = (p.N + 15) / 16;
     const int my_strips = (strips - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
 
     const __amdgpu_buffer_rsrc_t rsrc_w = make_rsrc(p.w, (uint32_t)((int64_t)(p.N - 1) * p.ldw + p.K));
-    const __amdgpu_buffer_rsrc_t rsrc_x = make_rsrc(p.x, (uint32_t)(((int64_t)(p.M - 1) * p.ldx + p.K) * 2));
+    const __amdgpu_buffer_rsrc_t rsrc_x = make_rsrc(p.x + (int64_t)m_base * p.ldx, (uint32_t)(((int64_t)(rows - 1) * p.ldx + p.K) * 2));
     const __amdgpu_buffer_rsrc_t rsrc_sc = make_rsrc(p.scale, (uint32_t)p.N * 2u);
     const __amdgpu_buffer_rsrc_t rsrc_of = make_rsrc(p.offset, p.offset ? (uint32_t)p.N * 2u : 0u);
     const __amdgpu_buffer_rsrc_t rsrc_bias = make_rsrc(p.bias, p.bias ? (uint32_t)p.N * 2u : 0u);
@@ -53,27 +59,37 @@ __global__ __launch_bounds__(512) void wq_kmajor_decode_kernel(const WqKmDecodeA
     char *const tb = lds + wave * kWaveBytes;
     float *const red = reinterpret_cast<float *>(lds + 8 * kWaveBytes);   // [parity][wavefront][tile][lane][4]
     float *const xsum = red + 2 * 8 * MT * 256;                           // [wavefront][tile][lane][4]
+    f32x4 *const kept = reinterpret_cast<f32x4 *>(xsum + 8 * MT * 256) + wave * MT * 64 + lane;   // sums between passes: [strip][wavefront][tile][lane]
 
-    // The wavefront's slice of the activations, once: a step is 16 rows x 256 bytes; an instruction loads four whole
-    // rows (lane l: 16 bytes of row 4 i + l / 16), the step goes through LDS, and lane (c, g) reads for MFMA t the
-    // 8 k at 64 (t / 2) + 16 g + 8 (t % 2) of row c.
+    // The wavefront's slice of the activations of a pass: a step is 16 rows x 256 bytes; an instruction loads four whole rows
+    // (lane l: 16 bytes of row r = 4 i + l / 16), the step goes through LDS, and lane (c, g) reads for MFMA t the 8 k at
+    // 64 (t / 2) + 16 g + 8 (t % 2) of row c.  Lane l fetches piece (l % 16) ^ r, so that the reads of a piece of all 16 rows,
+    // which are 256 bytes apart, meet 16 different quads of banks.  Rows past the last one are not written to LDS: what their
+    // lanes read only reaches accumulator rows that are never stored.  (8192x1024 at one row: 11.2 us without the swizzle, 16
+    // rows: 9.1 with it; loads straight in operand order, 16 rows x 64 bytes each, 7.5 at one row but 12.6 at 16.)
     u32x4 xf[NS][MT][4];
+    auto load_x = [&](int pass) {
 #pragma unroll
-    for (int j = 0; j < NS; j++)
+        for (int j = 0; j < NS; j++) {
+            const int st = pass * NS + j;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++)
+            for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int row = mt * 16 + 4 * i + (lane >> 4);
-                xf[j][mt][i] = __builtin_amdgcn_raw_buffer_load_b128(
-                    rsrc_x, j < ns && row < p.M && (s0 + j) * kStep + (lane & 15) * 8 < p.K ? (uint32_t)((row * (int)p.ldx) * 2 + (lane & 15) * 16) : kOutOfRange,
-                    (uint32_t)(s0 + j) * (kStep * 2), 0);
-            }
+                for (int i = 0; i < 4; i++) {
+                    const int r16 = 4 * i + (lane >> 4), row = mt * 16 + r16, piece = (lane & 15) ^ r16;
+                    xf[j][mt][i] = __builtin_amdgcn_raw_buffer_load_b128(
+                        rsrc_x, st < ns && row < rows && (s0 + st) * kStep + piece * 8 < p.K ? (uint32_t)((row * (int)p.ldx) * 2 + piece * 16) : kOutOfRange,
+                        (uint32_t)(s0 + st) * (kStep * 2), 0);
+                }
+        }
+    };
+    load_x(0);
 
-    // weights: flat step f = strip index * NS + step; ring slot f % PF, LDS buffer f % 2
+    // weights: flat step f = (pass * strips + strip index) * NS + step; ring slot f % PF, LDS buffer f % 2
     u32x4 wr[PF][2];
-    auto load_w = [&](int slot, int t, int st) {
-        const bool ok = t < my_strips && st < ns;
+    auto load_w = [&](int slot, int pass, int t, int j) {
+        const int st = pass * NS + j;
+        const bool ok = (!PASSES || pass < passes) && t < my_strips && st < ns;
         const uint32_t so = (uint32_t)(((int)blockIdx.x + t * (int)gridDim.x) * 16) * (uint32_t)p.ldw + (uint32_t)(s0 + st) * kStep;
 #pragma unroll
         for (int h = 0; h < 2; h++) wr[slot][h] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, ok ? voff_w[h] : kOutOfRange, so, kNonTemporal);
@@ -84,41 +100,64 @@ __global__ __launch_bounds__(512) void wq_kmajor_decode_kernel(const WqKmDecodeA
         for (int h = 0; h < 2; h++) *reinterpret_cast<u32x4 *>(dst + h * 1024) = wr[slot][h];
     };
 #pragma unroll
-    for (int r = 0; r < PF; r++) load_w(r, r / NS, r % NS);
+    for (int r = 0; r < PF; r++) load_w(r, 0, 0, r);
 
-    // turn the activation steps around (a wavefront's LDS operations complete in order) and add up the rows
+    // turn the activation steps around (a wavefront's LDS operations complete in order) and add up the rows, in four
+    // independent chains of MFMAs
     const u32x4 ones = u32x4{kOnes2<ACT>, kOnes2<ACT>, kOnes2<ACT>, kOnes2<ACT>};
     f32x4 X[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) X[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < NS; j++)
+    auto turn_x = [&](int pass) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
-            char *xb = tb + 4096;
+            f32x4 part[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) *reinterpret_cast<u32x4 *>(xb + i * 1024 + lane * 16) = xf[j][mt][i];
+            for (int t = 0; t < 4; t++) part[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                xf[j][mt][t] = *reinterpret_cast<const u32x4 *>(xb + c * 256 + ((t >> 1) * 8 + 2 * g + (t & 1)) * 16);
-                X[mt] = mfma_act<ACT>(xf[j][mt][t], ones, X[mt]);
+            for (int j = 0; j < NS; j++) {
+                if (PASSES && pass * NS + j >= ns) continue;              // zeros; a short last pass is common
+                char *xb = tb + 4096;
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (mt * 16 + 4 * i < rows) *reinterpret_cast<u32x4 *>(xb + i * 1024 + lane * 16) = xf[j][mt][i];
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    xf[j][mt][t] = *reinterpret_cast<const u32x4 *>(xb + c * 256 + (((t >> 1) * 8 + 2 * g + (t & 1)) ^ c) * 16);
+                    part[t] = mfma_act<ACT>(xf[j][mt][t], ones, part[t]);
+                }
             }
+            X[mt] += (part[0] + part[1]) + (part[2] + part[3]);
         }
+    };
     // every wavefront's row sums meet once: lane (c, g) of the accumulator holds rows 4 g + q (the same for every column)
+    auto publish_x = [&]() {
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) *reinterpret_cast<f32x4 *>(xsum + ((wave * MT + mt) * 64 + lane) * 4) = X[mt];
+        for (int mt = 0; mt < MT; mt++) *reinterpret_cast<f32x4 *>(xsum + ((wave * MT + mt) * 64 + lane) * 4) = X[mt];
+    };
+    turn_x(0);
+    if (passes == 1) publish_x();
 
     // wavefront t < MT finishes tile t of every strip: lane l writes row l / 4, columns 4 (l % 4) .. + 3
     const bool finisher = wave < MT;
     const int er = lane >> 2, ec = (lane & 3) * 4;
-    const int em = wave * 16 + er;
+    const int em = m_base + wave * 16 + er;
     // accumulator element (row 4 g + q, column c) lies at float index (c + 16 g) * 4 + q of a wavefront's tile
     const int e_idx = (16 * (er >> 2)) * 4 + (er & 3);                    // + 4 * column
     float xtot = 0.0f;
     bool xtot_ready = false;
 
     to_lds_w(0, 0);
+    for (int pass = 0; pass < passes; pass++) {
+    if (PASSES && pass > 0) {
+        load_x(pass);
+        turn_x(pass);
+        if (pass + 1 == passes) publish_x();
+    }
     for (int t = 0; t < my_strips; t++) {
+        // the item behind this one: the next strip, or the first strip of the next pass
+        const bool wrap = PASSES && t + 1 == my_strips;
+        const int next_pass = wrap ? pass + 1 : pass, next_t = wrap ? 0 : t + 1;
         const int n0 = ((int)blockIdx.x + t * (int)gridDim.x) * 16;
         const int en = n0 + ec;
         // antiquantisation parameters of this strip (wavefronts that finish no tile get an out-of-range offset: no branch
@@ -130,7 +169,7 @@ __global__ __launch_bounds__(512) void wq_kmajor_decode_kernel(const WqKmDecodeA
 
         f32x4 P[MT];
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) P[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int mt = 0; mt < MT; mt++) P[mt] = PASSES && pass > 0 ? kept[(t * 8 * MT + mt) * 64] : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < NS; j++) {
             const char *src = tb + (j & 1) * 2048;
@@ -138,7 +177,8 @@ __global__ __launch_bounds__(512) void wq_kmajor_decode_kernel(const WqKmDecodeA
             const u32x4 w1 = *reinterpret_cast<const u32x4 *>(src + (t_rd ^ 64));
             to_lds_w((j + 1) % PF, (j + 1) & 1);                          // the next step's registers take the other buffer
             __builtin_amdgcn_sched_barrier(0);
-            load_w(j % PF, t + (j + PF) / NS, (j + PF) % NS);             // this step's registers are free again
+            // this step's registers are free again
+            load_w(j % PF, j + PF < NS ? pass : next_pass, j + PF < NS ? t : next_t, (j + PF) % NS);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int q = 0; q < 4; q++) {
@@ -153,6 +193,11 @@ __global__ __launch_bounds__(512) void wq_kmajor_decode_kernel(const WqKmDecodeA
             }
         }
 
+        if (PASSES && pass + 1 < passes) {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) kept[(t * 8 * MT + mt) * 64] = P[mt];
+            continue;
+        }
         float *const rd = red + (t & 1) * (8 * MT * 256);
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) *reinterpret_cast<f32x4 *>(rd + ((wave * MT + mt) * 64 + lane) * 4) = P[mt];
@@ -185,26 +230,55 @@ __global__ __launch_bounds__(512) void wq_kmajor_decode_kernel(const WqKmDecodeA
             }
         }
     }
+    }
 }
 
-template <int MT, int NS, int ACT>
+int lds_need(int mt, int64_t N, bool passes)
+{
+    const int64_t strips = (N + 15) / 16;
+    return 8 * 8192 + 3 * 8 * mt * 1024 + (passes ? (int)((strips + kMaxWorkgroups - 1) / kMaxWorkgroups) * 8 * mt * 1024 : 0);
+}
+
+template <int MT, int NS, int PF, int ACT, bool PASSES>
 int launch(const WqKmDecodeArgs &p, hipStream_t s)
 {
-    constexpr int lds_bytes = 8 * 8192 + 2 * 8 * MT * 1024 + 8 * MT * 1024;
-    auto kern = wq_kmajor_decode_kernel<MT, NS, 4, ACT>;
-    static int attr_status = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    const int lds_bytes = lds_need(MT, p.N, PASSES);
+    auto kern = wq_kmajor_decode_kernel<MT, NS, PF, ACT, PASSES>;
+    static int attr_status = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
     if (attr_status != hipSuccess) return MI355_ERR_LAUNCH;
     const int strips = (p.N + 15) / 16;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(strips < kMaxWorkgroups ? strips : kMaxWorkgroups)), dim3(512), lds_bytes, s, p);
+    const unsigned chunks = (unsigned)((p.M + 16 * MT - 1) / (16 * MT));
+    hipLaunchKernelGGL(kern, dim3((unsigned)(strips < kMaxWorkgroups ? strips : kMaxWorkgroups), chunks), dim3(512), lds_bytes, s, p);
     return check_launch();
+}
+
+// Tiles of 16 rows per workgroup (1, 2 or 4), 0: another kernel is the faster one.
+int row_tiles(int64_t M, int64_t N, int64_t K)
+{
+    if (M < 1 || M > 128 || K % 16 != 0 || K < 8 * kStep || N % 4 != 0) return 0;
+    const int64_t strips = (N + 15) / 16;
+    const int64_t steps = ((K + kStep - 1) / kStep + 7) / 8;              // of the busiest wavefront
+    for (int mt = 1; mt <= 4; mt *= 2) {
+        const int64_t chunks = (M + 16 * mt - 1) / (16 * mt);
+        // what the workgroups read through the L2 in all: their strip of the weight and the 16-bit activations
+        const int64_t bytes = strips * chunks * (16 + 32 * mt) * K;
+        if (chunks > 1 && (strips * chunks > kMaxWorkgroups || bytes > kMaxChunkBytes)) continue;
+        if (mt == 4 && bytes > kMaxChunkBytes) continue;
+        // the activations of a wavefront's eighth of K stay in registers: 8 steps with one tile, 4 with two, 2 with four
+        if (steps > 8 / mt && lds_need(mt, N, true) > kMaxLds) continue;
+        return mt;
+    }
+    return 0;
 }
 
 template <int ACT>
 int launch_act(const WqKmDecodeArgs &p, hipStream_t s)
 {
     const int ns = ((p.K + kStep - 1) / kStep + 7) / 8;
-    if (p.M <= 16) return ns <= 4 ? launch<1, 4, ACT>(p, s) : launch<1, 8, ACT>(p, s);
-    return launch<2, 4, ACT>(p, s);
+    const int mt = row_tiles(p.M, p.N, p.K);
+    if (mt == 1) return ns <= 4 ? launch<1, 4, 4, ACT, false>(p, s) : ns <= 8 ? launch<1, 8, 4, ACT, false>(p, s) : launch<1, 8, 4, ACT, true>(p, s);
+    if (mt == 2) return ns <= 4 ? launch<2, 4, 4, ACT, false>(p, s) : launch<2, 4, 4, ACT, true>(p, s);
+    return ns <= 2 ? launch<4, 2, 2, ACT, false>(p, s) : launch<4, 2, 2, ACT, true>(p, s);
 }
 
 } // namespace
@@ -213,10 +287,7 @@ bool wq_kmajor_decode_shape(int64_t M, int64_t N, int64_t K, int64_t group_size)
 {
     if (knob(kKnobWqDecodeOff) == 1 || knob(kKnobWqSplit) != 0) return false;
     if (group_size > 0 && group_size != K) return false;                  // one scale per column
-    if (M < 1 || M > 32 || K % 16 != 0 || K < 8 * kStep || N < 2048 || N % 4 != 0) return false;
-    // the activations of a wavefront's eighth of K stay in registers: 8 steps with one tile of 16 rows, 4 with two
-    const int64_t steps = ((K + kStep - 1) / kStep + 7) / 8;
-    return M <= 16 ? steps <= 8 : steps <= 4;
+    return row_tiles(M, N, K) > 0;
 }
 
 int launch_wq_kmajor_decode(const WqKmDecodeArgs &p, int act_f16, hipStream_t s)

@@ -917,6 +917,24 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
     if (!params_rowmajor) return generic();
     if (w_bits == 8 && ldw_k == 1 && ldw_n != 1) {
         // K-major: the transposed view of an [N, K] weight
+        if (wq_kmajor_decode_shape(M, N, K, group_size)) {
+            // few rows, one scale per column: the barrier-free kernel that splits K inside the workgroup
+            WqKmDecodeArgs d;
+            d.x = static_cast<const uint16_t *>(x_bf16);
+            d.w = static_cast<const int8_t *>(w);
+            d.scale = static_cast<const uint16_t *>(scale_bf16);
+            d.offset = static_cast<const uint16_t *>(offset_bf16);
+            d.bias = static_cast<const uint16_t *>(bias);
+            d.out = static_cast<uint16_t *>(out_bf16);
+            d.ldx = ldx;
+            d.ldw = ldw_n;
+            d.ldo = ldo;
+            d.M = (int)M;
+            d.N = (int)N;
+            d.K = (int)K;
+            const int st = launch_wq_kmajor_decode(d, f16 ? 1 : 0, s);
+            if (st != MI355_ERR_UNSUPPORTED) return st;
+        }
         const WqGemmPlan gk = make_wq_gemm_plan(M, N, K, 8, group_size, 2, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
         if (gk.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2))) {
             if (gk.S > 1) {
@@ -929,24 +947,6 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
         const WqKmPlan km = make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
         const bool params_ok = aligned(scale_bf16, 2) && (!offset_bf16 || aligned(offset_bf16, 2));
         if (km.fast && params_ok) {
-            if (wq_kmajor_decode_shape(M, N, K, group_size)) {
-                // at most 32 rows, one scale per column: the barrier-free kernel that splits K inside the workgroup
-                WqKmDecodeArgs d;
-                d.x = static_cast<const uint16_t *>(x_bf16);
-                d.w = static_cast<const int8_t *>(w);
-                d.scale = static_cast<const uint16_t *>(scale_bf16);
-                d.offset = static_cast<const uint16_t *>(offset_bf16);
-                d.bias = static_cast<const uint16_t *>(bias);
-                d.out = static_cast<uint16_t *>(out_bf16);
-                d.ldx = ldx;
-                d.ldw = ldw_n;
-                d.ldo = ldo;
-                d.M = (int)M;
-                d.N = (int)N;
-                d.K = (int)K;
-                const int st = launch_wq_kmajor_decode(d, f16 ? 1 : 0, s);
-                if (st != MI355_ERR_UNSUPPORTED) return st;
-            }
             if (km.S > 1) {
                 if (!workspace || workspace_bytes < km.partial_bytes + km.counter_bytes) return MI355_ERR_WORKSPACE;
                 if (!aligned(workspace, 16)) return MI355_ERR_ALIGNMENT;

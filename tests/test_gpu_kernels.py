@@ -691,7 +691,10 @@ def test_w8a16_kmajor_and_no_offset(capi, golden):
 
 
 @pytest.mark.parametrize("M,K,N,f16", [(1, 4096, 4096, False), (16, 8192, 2048, False), (7, 1152, 2052, True), (16, 2176, 4104, False),
-                                       (17, 4096, 2048, False), (32, 3072, 6144, True), (3, 1024, 8200, False)])
+                                       (17, 4096, 2048, False), (32, 3072, 6144, True), (3, 1024, 8200, False),
+                                       # passes over K, narrow outputs, chunks of rows, four row tiles
+                                       (5, 9232, 1028, False), (32, 5120, 4100, True), (50, 2064, 2052, False), (128, 1152, 260, True),
+                                       (64, 2048, 3076, False)])
 def test_w8a16_kmajor_decode_kernel(capi, golden, M, K, N, f16):
     """int8 weight stored [N, K], one scale per column, at most 32 rows: the kernel that splits K over the wavefronts of a
     workgroup and walks over strips of 16 columns (one and two tiles of 16 rows, 1 to 8 steps per wavefront, even and
@@ -998,6 +1001,11 @@ KPACKED_CASES = [
     (16, 3072, 8224, 128, True, True, True),        # more strips than workgroups, uneven steps, fp16
     (17, 4096, 2048, 128, False, True, True),       # two tiles of rows (at most two steps per wavefront)
     (32, 3072, 4104, 128, True, False, False),      # the same, uneven steps, a strip that ends past N, fp16
+    (2, 1280, 1048, 128, False, True, True),        # fewer steps than wavefronts, narrow
+    (6, 10496, 1032, 128, True, True, False),       # several passes over K
+    (30, 6144, 520, 128, False, True, True),        # chunks of one row tile, passes
+    (50, 2304, 4104, 128, False, True, False),      # chunks of two row tiles, two rounds of workgroups
+    (121, 4096, 264, 128, True, False, True),       # eight chunks
     # from 256 rows up the weight is rewritten per call with its words along N (weight_quant_repack.hip)
     (256, 512, 1000, 128, False, True, True),       # ragged columns: 125 words per row, the last tile partly valid
     (300, 1024, 520, 256, True, True, False),       # ragged rows, groups of two stages, fp16
