@@ -1071,8 +1071,10 @@ QmmPlan make_qmm_plan(int64_t M, int64_t N, int64_t K, int64_t ldb_k, int64_t ld
     QmmPlan pl{};
     const bool tiled_shape = K >= BK;
     const int64_t Kp = (K + 15) / 16 * 16;
-    // the decode kernel splits K inside its workgroups (it is not used while a tile or a split is forced)
-    const bool decode = qmm_decode_shape(M, N, Kp) && knob(kKnobQmmSplit) == 0 && knob(kKnobQmmTile) == 0;
+    // The decode kernel splits K inside its workgroups and needs no scratch (it is not used while a tile or a split is forced).
+    // Operands that it refuses for their alignment run on the tiled kernel: unsplit where the output is wide, but a narrow one, or
+    // one of several row chunks, is a handful of tiles (64x4096x256: two) and keeps its split and the scratch for that.
+    const bool decode = qmm_decode_shape(M, N, Kp) && M <= 64 && N >= 2048 && knob(kKnobQmmSplit) == 0 && knob(kKnobQmmTile) == 0;
     // a contiguous [K,N] weight is transposed into the workspace
     pl.transpose_bytes = tiled_shape && ldb_k != 1 && ldb_n == 1 ? (size_t)N * (size_t)Kp : 0;
     // rows that are not a multiple of 16 bytes are copied into padded ones
@@ -1197,7 +1199,7 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
     const int64_t K_in = K;
     if (tiled) K = Kp;
     if (tiled && knob(kKnobQmmSplit) == 0 && knob(kKnobQmmTile) == 0) {
-        // at most 64 rows: the barrier-free kernel that splits K inside the workgroup (quant_matmul_decode.hip)
+        // few rows: the barrier-free kernel that splits K inside the workgroup (quant_matmul_decode.hip)
         QmmDecodeArgs d;
         d.a = a;
         d.bt = bt;

@@ -1,4 +1,4 @@
-// Internal interface of the decode-shaped int8 x int8 kernel (at most 64 activation rows, weight stored [N, K]); not part of
+// Internal interface of the decode-shaped int8 x int8 kernel (at most 256 activation rows, weight stored [N, K]); not part of
 // the C ABI.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -24,7 +24,7 @@ struct QmmDecodeArgs {
     int scale_len;             // 1 or N
 };
 
-// The part of the decision that depends on the shape alone (the workspace query uses it: the kernel needs no workspace).
+// The part of the decision that depends on the shape alone (the planner uses it: the kernel needs no workspace).
 __attribute__((visibility("hidden"))) bool qmm_decode_shape(int64_t M, int64_t N, int64_t K);
 
 // MI355_ERR_UNSUPPORTED when pointers or pitches do not fit the kernel: the caller then takes the tiled kernel.

@@ -269,7 +269,8 @@ int launch(const QmmDecodeArgs &p, hipStream_t s)
 // Tiles of 16 rows per workgroup (1, 2 or 4), 0: the tiled kernel is the faster one.
 int row_tiles(int64_t M, int64_t N, int64_t K)
 {
-    if (M < 1 || M > 256 || K % 16 != 0 || K < 8 * kStep) return 0;
+    // (parameters and results go in pieces of four columns; any other width takes the tiled kernel and its split of K)
+    if (M < 1 || M > 256 || N % 4 != 0 || K % 16 != 0 || K < 8 * kStep) return 0;
     const int64_t strips = (N + 15) / 16;
     const int64_t steps = ((K + kStep - 1) / kStep + 7) / 8;              // of the busiest wavefront
     for (int mt = 1; mt <= 4; mt *= 2) {
@@ -300,7 +301,7 @@ int launch_qmm_decode(const QmmDecodeArgs &p, hipStream_t s)
     if ((p.lda & 15) != 0 || (p.ldbt & 15) != 0 || !aligned(p.a, 16) || !aligned(p.bt, 16) || p.ldbt < p.K)
         return MI355_ERR_UNSUPPORTED;
     // dequantisation parameters and results in pieces of four columns
-    if ((p.N & 3) != 0 || (p.ldc & 3) != 0 || !aligned(p.out, p.out_i32 ? 16 : 8) || !aligned(p.qparam ? static_cast<const void *>(p.qparam) : static_cast<const void *>(p.scale), 16) ||
+    if ((p.ldc & 3) != 0 || !aligned(p.out, p.out_i32 ? 16 : 8) || !aligned(p.qparam ? static_cast<const void *>(p.qparam) : static_cast<const void *>(p.scale), 16) ||
         (p.bias && !aligned(p.bias, p.bias_kind == MI355_BIAS_BF16 ? 8 : 16)))
         return MI355_ERR_UNSUPPORTED;
     // 32-bit buffer offsets over the whole weight and all activation rows

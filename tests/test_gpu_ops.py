@@ -618,6 +618,43 @@ def test_workspace_outlives_growth_after_capture(pa):
     torch.cuda.synchronize()
 
 
+def test_split_k_graph_survives_workspace_growth(pa):
+    """The same with a first product whose graph uses the workspace: 258 columns are not whole pieces of four, so the tiled kernel
+    runs with K split over workgroups that meet at counters there."""
+    from pytorch_amd import _capi
+    g = torch.Generator().manual_seed(21)
+    M, K, N = 64, 4096, 258
+    q = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8).cuda()
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).cuda().t()
+    sc, ps = (torch.rand(N, generator=g) * 1e-2).cuda(), (torch.rand(M, generator=g) * 1e-2).cuda()
+    Kb, Nb = 14336, 4096
+    qb = torch.randint(-127, 128, (M, Kb), generator=g, dtype=torch.int8).cuda()
+    wb = torch.randint(-127, 128, (Nb, Kb), generator=g, dtype=torch.int8).cuda().t()
+    scb = (torch.rand(Nb, generator=g) * 1e-2).cuda()
+    small_ws = _capi.lib().mi355_quant_matmul_workspace(M, N, K, 1, K)
+    big_ws = _capi.lib().mi355_quant_matmul_workspace(M, Nb, Kb, 1, Kb)
+    floor = _capi.ZERO_AREA_BYTES + (1 << 20)          # the smallest buffer the operator layer allocates
+    assert 0 < small_ws <= floor < big_ws, (small_ws, big_ws)          # the second call must outgrow the first buffer
+    small = lambda: pa.npu_quant_matmul(q, w, sc, pertoken_scale=ps, output_dtype=torch.bfloat16)
+    big = lambda: pa.npu_quant_matmul(qb, wb, scb, pertoken_scale=ps, output_dtype=torch.bfloat16)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        want = small().clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = small()
+        want_big = big().clone()                       # eager, same stream: allocates the larger workspace
+        stream.synchronize()
+        for it in range(3):
+            out.zero_()
+            graph.replay()
+            stream.synchronize()
+            assert torch.equal(out, want), f"replay {it} after the workspace grew differs"
+            assert torch.equal(big(), want_big)
+            assert torch.equal(small(), want)
+    torch.cuda.synchronize()
+
+
 def test_captures_without_warmup_on_their_stream(pa):
     """The usual capture idiom warms up on one stream and captures on another (torch.cuda.graph picks its own): a
     split-K operator then meets a stream without a workspace while capturing.  Every capture gets a workspace of its
