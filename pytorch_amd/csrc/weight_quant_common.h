@@ -80,6 +80,21 @@ constexpr float kImageMul = (WBITS == 4 && ACT == 0) ? 2.0f : 1.0f;    // weight
 template <int WBITS>
 constexpr float kImageBias = WBITS == 4 ? 24.0f : 0.0f;
 __device__ __forceinline__ float sbyte_f32(uint32_t w, int i) { return (float)(int8_t)((w >> (8 * i)) & 0xffu); }
+// The images of the four signed bytes of a word, in order.  fp16: byte + 128 as the low mantissa bits of 1024 (a byte permute per
+// pair), minus 1152, exactly (2.5 instructions per pair; a conversion per byte and a pack take 5.5).
+template <int ACT>
+__device__ __forceinline__ u32x2 sbytes_act4(uint32_t w)
+{
+    if constexpr (ACT == 0) {
+        return u32x2{pack_act2<ACT>(sbyte_f32(w, 0), sbyte_f32(w, 1)), pack_act2<ACT>(sbyte_f32(w, 2), sbyte_f32(w, 3))};
+    } else {
+        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+        const f16x2 bias = {(_Float16)1152.0f, (_Float16)1152.0f};
+        const uint32_t u = w ^ 0x80808080u;
+        const auto pair = [&](uint32_t sel) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, u, sel)) - bias); };
+        return u32x2{pair(0x04010400u), pair(0x04030402u)};
+    }
+}
 
 template <int WBITS, int ACT>
 __device__ __forceinline__ void expand_pair(const uint32_t (&w)[8], int jb, uint32_t magic, u32x4 &b0, u32x4 &b1)

@@ -1,0 +1,27 @@
+// Internal interface of the tiled weight-only GEMM for int8 weights stored [N, K] with one scale per column (more than 32
+// activation rows); not part of the C ABI.
+#pragma once
+#include <stddef.h>
+#include <stdint.h>
+
+namespace mi355 {
+
+struct WqKmGemmPlan {
+    bool ok;                               // the kernel accepts this problem
+    int wtm;                               // 64 * wtm activation rows per workgroup tile
+    int S;                                 // workgroups that share the K range of a tile
+    size_t counter_bytes, partial_bytes;   // workspace when S > 1: [arrival counters | partial sums]
+};
+
+// `ldw`: bytes between columns.  Null pointers (the workspace query) count as aligned.
+__attribute__((visibility("hidden"))) WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw,
+                                                                            int64_t ldx, const void *x, const void *w,
+                                                                            const void *scale, const void *offset);
+
+// Launches the kernel; `workspace` holds counter_bytes + partial_bytes when plan.S > 1.
+__attribute__((visibility("hidden"))) int launch_wq_kmajor_gemm(const WqKmGemmPlan &plan, const void *x, int act_f16, const void *w,
+                                                                const void *scale, const void *offset, const void *bias, void *out, int64_t M,
+                                                                int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldo, void *workspace,
+                                                                void *stream);
+
+} // namespace mi355

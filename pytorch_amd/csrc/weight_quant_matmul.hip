@@ -39,6 +39,7 @@
 #include "weight_quant_kmajor_decode.h"
 #include "weight_quant_common.h"
 #include "weight_quant_gemm.h"
+#include "weight_quant_kmajor_gemm.h"
 #include "weight_quant_kpacked.h"
 #include "weight_quant_kpacked_decode.h"
 #include "weight_quant_decode.h"
@@ -798,8 +799,10 @@ extern "C" size_t mi355_weight_quant_matmul_workspace(int64_t M, int64_t N, int6
             const WqPlan pl = make_plan(M, N, K, w_bits, group_size, true, ldw_n_major, ldx, nullptr, nullptr, nullptr, nullptr);
             if (pl.fast && pl.partial_bytes + pl.counter_bytes > need) need = pl.partial_bytes + pl.counter_bytes;
         }
+        const WqKmGemmPlan kmg = w_bits == 8 ? make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_k_major, ldx, nullptr, nullptr, nullptr, nullptr) : WqKmGemmPlan{};
+        if (kmg.ok && kmg.counter_bytes + kmg.partial_bytes > need) need = kmg.counter_bytes + kmg.partial_bytes;
         for (int layout = 1; layout <= (w_bits == 8 ? 2 : 1); layout++) {
-            if (layout == 1 && preferred != kPreferGemm) continue;
+            if (layout == 1 ? preferred != kPreferGemm : kmg.ok) continue;
             const WqGemmPlan gp = make_wq_gemm_plan(M, N, K, w_bits, group_size, layout, layout == 2 ? ldw_k_major : ldw_n_major, ldx,
                                                     nullptr, nullptr, nullptr, nullptr);
             const size_t gneed = gp.counter_bytes + gp.partial_bytes;
@@ -934,6 +937,15 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             d.K = (int)K;
             const int st = launch_wq_kmajor_decode(d, f16 ? 1 : 0, s);
             if (st != MI355_ERR_UNSUPPORTED) return st;
+        }
+        const WqKmGemmPlan kg = make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
+        if (kg.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2))) {
+            if (kg.S > 1) {
+                if (!workspace || workspace_bytes < kg.counter_bytes + kg.partial_bytes) return MI355_ERR_WORKSPACE;
+                if (!aligned(workspace, 16)) return MI355_ERR_ALIGNMENT;
+            }
+            return launch_wq_kmajor_gemm(kg, x_bf16, f16 ? 1 : 0, w, scale_bf16, offset_bf16, bias, out_bf16, M, N, K, ldx, ldw_n, ldo,
+                                         workspace, stream);
         }
         const WqGemmPlan gk = make_wq_gemm_plan(M, N, K, 8, group_size, 2, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
         if (gk.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2))) {

@@ -680,6 +680,43 @@ def test_w8a16_partial_last_step(capi, golden, M, K, N, f16, nk):
     bf16_gate(out, torch.from_numpy(want))
 
 
+@pytest.mark.parametrize("M,K,N,f16,offset", [(33, 128, 8, True, True), (64, 136, 120, False, True), (65, 448, 136, True, False),
+                                             (129, 1040, 264, False, True), (193, 2112, 128, True, True), (256, 1000, 392, False, False),
+                                             (257, 640, 1000, True, True), (321, 3080, 72, False, True)])
+def test_w8a16_kmajor_tiled_kernel(capi, golden, M, K, N, f16, offset):
+    """int8 weight stored [N, K], one scale per column, more than 32 rows: every height of the tile (64 to 256 rows) unsplit and with
+    K split, at ragged rows and columns, one stage of K up to many and a partial last one, with and without an offset and a bias.
+    The activations are a view of a wider matrix whose columns past K hold NaN; the weight rows are pitched."""
+    d = workloads.w8a16_inputs(seed=M + K, M=M, K=K, N=N, weight_nk=True)
+    dt = torch.float16 if f16 else torch.bfloat16
+    d = {k: (v.to(dt) if v.is_floating_point() else v) for k, v in d.items()}
+    xw = torch.full((M, K + 64), float("nan"), dtype=dt, device="cuda")
+    xw[:, :K] = d["x"].cuda()
+    ww = torch.full((N, K + 24), 77, dtype=torch.int8, device="cuda")
+    ww[:, :K] = d["weight"].t().cuda()
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(N)).to(dt) if offset else None
+    of = d["antiquant_offset"] if offset else None
+    _, want = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]), None if of is None else _bits(of),
+                                         dtype="fp16" if f16 else "bf16")
+    want = torch.from_numpy(want) if bias is None else torch.from_numpy(want) + bias.float()
+    stages = (K + 63) // 64
+    try:
+        capi.set_tuning("MI355_WQ_DECODE_OFF", 1)
+        for bm in (64, 128, 192, 256):
+            capi.set_tuning("MI355_WQG_BM", bm)
+            for split in (1, 2, 3, 7):
+                if split > stages:
+                    continue
+                capi.set_tuning("MI355_WQG_SPLIT", split)
+                for _ in range(2):                             # the second launch meets the counters the first one left
+                    out = capi.weight_quant_matmul(xw[:, :K], ww[:, :K].t(), d["antiquant_scale"].cuda(), None if of is None else of.cuda(),
+                                                   bias=None if bias is None else bias.cuda())
+                    bf16_gate(out, want)
+    finally:
+        for k in ("MI355_WQ_DECODE_OFF", "MI355_WQG_BM", "MI355_WQG_SPLIT"):
+            capi.set_tuning(k, 0)
+
+
 def test_w8a16_kmajor_and_no_offset(capi, golden):
     d = workloads.w8a16_inputs(seed=3, M=8, K=1024, N=192, weight_nk=True)
     out = capi.weight_quant_matmul(d["x"].cuda(), d["weight"].cuda(), d["antiquant_scale"].cuda(),
