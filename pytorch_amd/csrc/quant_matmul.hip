@@ -107,7 +107,8 @@ __device__ __forceinline__ int32_t requant1(int32_t a, int32_t bi, float sc, flo
 // WGM x WGN wavefronts per workgroup, each owning (16*WTM) x (16*WTN) of the output tile.
 // LOOP 0: the generic K loop below; 3: the same with as many activation slots as weight slots (whole stages requested
 // NS steps ahead); 1, 2: the loop of quant_matmul_wide.h (4 x 2 wavefronts of 64 rows) with its
-// instruction order 0 (refills in a block) or 1 (refills spread over the step)
+// instruction order 0 (refills in a block) or 1 (refills spread over the step); 4: 2 and a partial last step of K (in one kernel
+// with the loop, the step that few launches take costs 2048x4096x28672 0.5 %)
 // EPI (the widest wavefront tile only, see LEAN below): which variants of the LDS-parameter epilogue this instantiation holds
 template <int WGM, int WGN, int WTM, int WTN, int NS, int LOOP = 0, int EPI = 0>
 __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
@@ -118,7 +119,9 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     constexpr int UNITS_BP = (UNITS_B + NW - 1) / NW * NW;
     constexpr int LA = UNITS_A / NW, LB = UNITS_BP / NW;     // loads of a wavefront per activation / weight stage
     constexpr int A_BYTES = UNITS_A * 1024, B_BYTES = UNITS_BP * 1024;
-    constexpr bool WIDE = LOOP == 1 || LOOP == 2;
+    constexpr bool WIDE = LOOP == 1 || LOOP == 2 || LOOP == 4;
+    constexpr bool TAIL = LOOP != 2;                         // a partial K step may follow the wide loop
+    constexpr int ORDER = LOOP == 1 ? 0 : 1;                 // instruction order of the wide loop
     constexpr bool WHOLE = NS >= 4 || LOOP == 3;             // whole stages: activations get NS slots as well
     // the epilogues that take their parameters from LDS (quant_matmul_wide.h: wavefronts of 64 rows): the wide loop's tiles
     // and the whole-stage 128-row tiles, which keep the vectors behind their ring
@@ -145,8 +148,8 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     MI355_TS(0)
     // Wavefronts w and w + 4 of a workgroup share a SIMD.  In the wide loop the two wavefronts of a SIMD take different
     // roles (one refills activations, one weights): wn = 0, 1, 0, 1, 1, 0, 1, 0 for wavefronts 0 .. 7.
-    const int wm = LOOP == 1 || LOOP == 2 ? ((wave & 3) >> 1) + 2 * (wave >> 2) : wave / WGN;
-    const int wn = LOOP == 1 || LOOP == 2 ? ((wave >> 2) ^ wave) & 1 : wave % WGN;
+    const int wm = WIDE ? ((wave & 3) >> 1) + 2 * (wave >> 2) : wave / WGN;
+    const int wn = WIDE ? ((wave >> 2) ^ wave) & 1 : wave % WGN;
     // K steps of this workgroup.  A K that is not a multiple of 128 ends in a partial step: the activations of the missing
     // bytes are loaded as zeros (kbytes below), so what the weight rows hold there (the next row, or padding) does not
     // matter.  The wide loop, whose loads take scalar offsets only, runs the whole steps and leaves the partial one to tail_step.
@@ -259,8 +262,9 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             st.unit_stride = unit_stride_a;
             st.sbase = (uint32_t)u0 * unit_stride_a + (uint32_t)kt0 * BK;
             st.dst0 = (uint32_t)u0 * 1024u;
-            wide::k_loop<WTN, 0, LOOP - 1>(acc, lds, st);
-            if (p.K % BK != 0 && chunk == p.S - 1) wide::tail_step<WTN, 0>(acc, lds, st, p.K % BK, lane);
+            wide::k_loop<WTN, 0, ORDER>(acc, lds, st);
+            if constexpr (TAIL)
+                if (p.K % BK != 0 && chunk == p.S - 1) wide::tail_step<WTN, 0>(acc, lds, st, p.K % BK, lane);
         } else {
             const int u0 = wm * G::LBW;                                   // a quarter of the weight rows
             st.rsrc = rsrc_b;
@@ -269,8 +273,9 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             st.unit_stride = unit_stride_b;
             st.sbase = (uint32_t)u0 * unit_stride_b + (uint32_t)kt0 * BK;
             st.dst0 = (uint32_t)u0 * 1024u;
-            wide::k_loop<WTN, 1, LOOP - 1>(acc, lds, st);
-            if (p.K % BK != 0 && chunk == p.S - 1) wide::tail_step<WTN, 1>(acc, lds, st, p.K % BK, lane);
+            wide::k_loop<WTN, 1, ORDER>(acc, lds, st);
+            if constexpr (TAIL)
+                if (p.K % BK != 0 && chunk == p.S - 1) wide::tail_step<WTN, 1>(acc, lds, st, p.K % BK, lane);
         }
         MI355_TS(2)
         __syncthreads();
@@ -957,7 +962,7 @@ int launch_qmm(QmmArgs p, hipStream_t s)
     constexpr int NS = DEEP < 0 ? 0 : DEEP ? DEEP : 2 * a_bytes + 2 * b_bytes <= 80 * 1024 && staging_bytes <= 80 * 1024 ? 2 : 3;
     // DEEP < 0: the streaming K loop (two activation chunks of 32 KiB and a ring of five 2 KiB weight steps per wavefront)
     constexpr size_t stage_bytes = DEEP < 0 ? (size_t)2 * 32768 + 8 * 5 * 2048 : (DEEP ? DEEP : 2) * a_bytes + NS * b_bytes;
-    constexpr size_t ring_bytes = LOOP == 1 || LOOP == 2 ? (size_t)wide::Geometry<WTN>::LDS_BYTES : stage_bytes + (LOOP == 3 ? 3072 : 0);
+    constexpr size_t ring_bytes = LOOP == 1 || LOOP == 2 || LOOP == 4 ? (size_t)wide::Geometry<WTN>::LDS_BYTES : stage_bytes + (LOOP == 3 ? 3072 : 0);
     constexpr size_t lds_bytes = ring_bytes > staging_bytes ? ring_bytes : staging_bytes;
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
     p.tiles_m = (p.M + BM - 1) / BM;
@@ -1276,11 +1281,14 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
                 if (lk == 2) return launch_qmm<4, 2, 4, 7, 0, 1>(p, s);
                 // the instantiation whose LDS-parameter epilogue serves this call's kind of bias and scale
                 const bool to16 = !p.out_i32 && !p.out_i8;
-                if (to16 && !p.qparam && (p.bias_kind == MI355_BIAS_INT32 || p.bias_kind == MI355_BIAS_FP32)) return launch_qmm<4, 2, 4, 7, 0, 2, 1>(p, s);
-                if (to16 && p.qparam && !p.pertoken && (p.bias_kind == MI355_BIAS_NONE || p.bias_kind == MI355_BIAS_INT32)) return launch_qmm<4, 2, 4, 7, 0, 2, 2>(p, s);
-                return launch_qmm<4, 2, 4, 7, 0, 2>(p, s);
+                const int epi = to16 && !p.qparam && (p.bias_kind == MI355_BIAS_INT32 || p.bias_kind == MI355_BIAS_FP32) ? 1
+                              : to16 && p.qparam && !p.pertoken && (p.bias_kind == MI355_BIAS_NONE || p.bias_kind == MI355_BIAS_INT32) ? 2 : 0;
+                if (p.K % BK != 0)
+                    return epi == 1 ? launch_qmm<4, 2, 4, 7, 0, 4, 1>(p, s) : epi == 2 ? launch_qmm<4, 2, 4, 7, 0, 4, 2>(p, s) : launch_qmm<4, 2, 4, 7, 0, 4>(p, s);
+                return epi == 1 ? launch_qmm<4, 2, 4, 7, 0, 2, 1>(p, s) : epi == 2 ? launch_qmm<4, 2, 4, 7, 0, 2, 2>(p, s) : launch_qmm<4, 2, 4, 7, 0, 2>(p, s);
             }
-            if (c.bm == 256 && c.bn == 192) return lk == 2 ? launch_qmm<4, 2, 4, 6, 0, 1>(p, s) : launch_qmm<4, 2, 4, 6, 0, 2>(p, s);
+            if (c.bm == 256 && c.bn == 192)
+                return lk == 2 ? launch_qmm<4, 2, 4, 6, 0, 1>(p, s) : p.K % BK != 0 ? launch_qmm<4, 2, 4, 6, 0, 4>(p, s) : launch_qmm<4, 2, 4, 6, 0, 2>(p, s);
         }
     }
     MI355_QMM_CASE(256, 224, 4, 2)

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(512, 1) void wq_gemm4_kernel(const WqGemm4Args p)
     const int tile = strip * p.tiles_m + mb;
     const int m0 = mb * BM;
     const int n0 = strip * 256;
-    const int total_stages = (p.K + BK - 1) / BK;              // int8: the last stage may be partial (zeros from x past K)
+    const int total_stages = WBITS == 4 ? p.K / BK : (p.K + BK - 1) / BK;   // int8: the last stage may be partial (zeros from x past K)
     const int units = total_stages / p.gstages;                // K is split in whole scale groups
     const int u0 = (int)((int64_t)units * chunk / p.S), u1 = (int)((int64_t)units * (chunk + 1) / p.S);
     const int s0 = u0 * p.gstages, NSTG = (u1 - u0) * p.gstages;
