@@ -876,10 +876,8 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             void *scale_gn = ws + kWorkspaceZeroBytes + repack_weight_bytes(N, K);
             void *offset_gn = offset_bf16 ? static_cast<char *>(scale_gn) + repack_param_bytes(N, K, group_size) : nullptr;
             const int64_t pitch = repack_pitch_words(N);
-            int st = launch_repack_int4_k_to_n(w, ldw_n, w_kn, pitch, N, K, stream);
-            if (st == MI355_OK) st = launch_gather_params_u16(scale_bf16, ld_param_g, ld_param_n, scale_gn, n_groups, N, stream);
-            if (st == MI355_OK && offset_bf16)
-                st = launch_gather_params_u16(offset_bf16, ld_param_g, ld_param_n, offset_gn, n_groups, N, stream);
+            const int st = launch_repack_int4_k_to_n(w, ldw_n, w_kn, pitch, scale_bf16, offset_bf16, ld_param_g, ld_param_n, scale_gn, offset_gn,
+                                                     n_groups, N, K, stream);
             if (st != MI355_OK) return st;
             const WqGemm4Plan g4 = make_wq_gemm4_plan(M, N, K, 4, group_size, pitch, ldx, x_bf16, w_kn, scale_gn, offset_gn);
             if (!g4.ok) return MI355_ERR_LAUNCH;       // planned with these strides a few lines up

@@ -2,18 +2,48 @@
 // torch_npu/contrib/module/linear_weight_quant.py:71,106) and many activation rows: the register-expanding GEMM for
 // words along N is 30-45 % faster than the kernel for this layout from 64 rows up, so from 256 rows up the weight is
 // rewritten per call into the workspace with its words along N (a nibble transpose, bound by the 2 x K x N / 2 bytes it
-// moves) and the parameters are gathered into row-major [G, N]; the repack costs less than the difference.
+// moves) and the parameters are gathered into row-major [G, N]; the repack costs less than the difference.  All of it is one
+// launch: weight and parameters are independent, and a launch of its own for each of
+// the three costs 3 - 4 us more (400x4096x4096 41.3 -> 38.4 us, 1024x1280x1280 33.3 -> 29.0).
 #include "common.h"
 #include "weight_quant_repack.h"
 
 namespace mi355 {
 namespace {
 
+struct RepackArgs {
+    const uint32_t *w_nk;
+    uint32_t *w_kn;
+    int64_t ldw_n, ldw_out;
+    const uint16_t *scale, *offset;            // offset may be null
+    uint16_t *scale_gn, *offset_gn;
+    int64_t ld_g, ld_n;
+    int N, K, G;
+    int k_blocks;                              // blocks of 32 words along K; the grid rows behind them gather parameters
+};
+
+constexpr int kGatherGroups = 16;              // groups per workgroup: their parameters of a column are few cache lines where they adjoin
+
 // A workgroup turns 256 weight rows (n) x 32 words (256 k) into 256 rows (k) x 32 words (256 n).  Both sides move
 // whole 128-byte row segments; in between a thread transposes 8 x 8 nibble blocks in registers.
-__global__ __launch_bounds__(256) void repack_int4_k_to_n_kernel(const uint32_t *__restrict__ w_nk, int64_t ldw_n,
-                                                                 uint32_t *__restrict__ w_kn, int64_t ldw_out, int N, int K)
+__global__ __launch_bounds__(256) void repack_int4_k_to_n_kernel(const RepackArgs p)
 {
+    if ((int)blockIdx.y >= p.k_blocks) {
+        // scales, then offsets: element (g, n) at src[g * ld_g + n * ld_n] -> dst[g * N + n]
+        const int parts = (p.G + kGatherGroups - 1) / kGatherGroups, row = (int)blockIdx.y - p.k_blocks;
+        const bool second = row >= parts;
+        const uint16_t *src = second ? p.offset : p.scale;
+        uint16_t *dst = second ? p.offset_gn : p.scale_gn;
+        const int n = blockIdx.x * 256 + threadIdx.x, g0 = (second ? row - parts : row) * kGatherGroups;
+        if (n >= p.N) return;
+#pragma unroll 4
+        for (int g = g0; g < min(g0 + kGatherGroups, p.G); g++) dst[(int64_t)g * p.N + n] = src[(int64_t)g * p.ld_g + (int64_t)n * p.ld_n];
+        return;
+    }
+    const uint32_t *__restrict__ const w_nk = p.w_nk;
+    uint32_t *__restrict__ const w_kn = p.w_kn;
+    const int64_t ldw_n = p.ldw_n, ldw_out = p.ldw_out;
+    const int N = p.N, K = p.K;
     // one buffer, used twice: [n][word] with the 16-byte chunk c of row r at chunk c ^ (r & 7), then, after every thread
     // has its blocks in registers, [k][word (n block), rotated by the k word] with a pitch of 33
     __shared__ __attribute__((aligned(16))) uint32_t buf[256 * 33];
@@ -81,28 +111,29 @@ __global__ __launch_bounds__(256) void repack_int4_k_to_n_kernel(const uint32_t 
     }
 }
 
-__global__ __launch_bounds__(256) void gather_params_u16_kernel(const uint16_t *__restrict__ src, int64_t ld_g, int64_t ld_n,
-                                                                uint16_t *__restrict__ dst, int G, int N)
-{
-    const int n = blockIdx.x * 256 + threadIdx.x, g = blockIdx.y;
-    if (n < N) dst[(int64_t)g * N + n] = src[(int64_t)g * ld_g + (int64_t)n * ld_n];
-}
-
 } // namespace
 
-int launch_repack_int4_k_to_n(const void *w_nk, int64_t ldw_n, void *w_kn, int64_t ldw_out, int64_t N, int64_t K, void *stream)
+int launch_repack_int4_k_to_n(const void *w_nk, int64_t ldw_n, void *w_kn, int64_t ldw_out, const void *scale, const void *offset, int64_t ld_g,
+                              int64_t ld_n, void *scale_gn, void *offset_gn, int64_t G, int64_t N, int64_t K, void *stream)
 {
-    const dim3 grid((unsigned)((N + 255) / 256), (unsigned)((K / 8 + 31) / 32));
-    hipLaunchKernelGGL(repack_int4_k_to_n_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const uint32_t *>(w_nk), ldw_n, static_cast<uint32_t *>(w_kn), ldw_out, (int)N, (int)K);
-    return check_launch();
-}
-
-int launch_gather_params_u16(const void *src, int64_t ld_g, int64_t ld_n, void *dst, int64_t G, int64_t N, void *stream)
-{
-    hipLaunchKernelGGL(gather_params_u16_kernel, dim3((unsigned)((N + 255) / 256), (unsigned)G), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(src), ld_g, ld_n, static_cast<uint16_t *>(dst),
-                       (int)G, (int)N);
+    RepackArgs p;
+    p.w_nk = static_cast<const uint32_t *>(w_nk);
+    p.w_kn = static_cast<uint32_t *>(w_kn);
+    p.ldw_n = ldw_n;
+    p.ldw_out = ldw_out;
+    p.scale = static_cast<const uint16_t *>(scale);
+    p.offset = static_cast<const uint16_t *>(offset);
+    p.scale_gn = static_cast<uint16_t *>(scale_gn);
+    p.offset_gn = static_cast<uint16_t *>(offset_gn);
+    p.ld_g = ld_g;
+    p.ld_n = ld_n;
+    p.N = (int)N;
+    p.K = (int)K;
+    p.G = (int)G;
+    p.k_blocks = (int)((K / 8 + 31) / 32);
+    const unsigned parts = (unsigned)((G + kGatherGroups - 1) / kGatherGroups);
+    const dim3 grid((unsigned)((N + 255) / 256), (unsigned)p.k_blocks + parts * (offset ? 2u : 1u));
+    hipLaunchKernelGGL(repack_int4_k_to_n_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), p);
     return check_launch();
 }
 
