@@ -58,7 +58,9 @@ constexpr int kMaxPolls4 = 1 << 20;
 // 64 rows (two steps), and a wavefront owns one 128-byte half of the rows x one span of 16 dwords with all four bytes
 // of its dwords: again four column tiles per lane (columns 128 s2 + 64 h + 4 c .. + 3), expanded with a byte-to-float
 // conversion and a packing conversion per pair of weights (the weight is its own image, converted with its sign).
-template <int ACT, bool STAGE_GROUPS, int WBITS = 4>
+// RAGGED (int8): K is not a multiple of 64, the last stage is partial: activations past K are loaded as zeros.  An instantiation of its
+// own: the comparison in the loop costs every other launch 3 % (1432x9088x3072: 177 -> 183 us).
+template <int ACT, bool STAGE_GROUPS, int WBITS = 4, bool RAGGED = false>
 __global__ __launch_bounds__(512, 1) void wq_gemm4_kernel(const WqGemm4Args p)
 {
     constexpr int SETS = 2, NW = 4 * SETS, BM = 64, BK = WBITS == 4 ? 128 : 64, SLOTS = 4;
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(512, 1) void wq_gemm4_kernel(const WqGemm4Args p)
     const int tile = strip * p.tiles_m + mb;
     const int m0 = mb * BM;
     const int n0 = strip * 256;
-    const int total_stages = WBITS == 4 ? p.K / BK : (p.K + BK - 1) / BK;   // int8: the last stage may be partial (zeros from x past K)
+    const int total_stages = RAGGED ? (p.K + BK - 1) / BK : p.K / BK;
     const int units = total_stages / p.gstages;                // K is split in whole scale groups
     const int u0 = (int)((int64_t)units * chunk / p.S), u1 = (int)((int64_t)units * (chunk + 1) / p.S);
     const int s0 = u0 * p.gstages, NSTG = (u1 - u0) * p.gstages;
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(512, 1) void wq_gemm4_kernel(const WqGemm4Args p)
                 const int row = WBITS == 4 ? 4 * u + (lane >> 4) : 8 * u + (lane >> 3);
                 uint32_t vo = WBITS == 4 ? (uint32_t)(row * (int)p.ldx * 2 + (((lane & 15) ^ (row & 15)) * 16))
                                          : (uint32_t)(row * (int)p.ldx * 2 + (((lane & 7) ^ (row & 7)) * 16));
-                if (WBITS == 8 && (s0 + s) * BK + ((lane & 7) ^ (row & 7)) * 8 >= p.K) vo = kOutOfRange;
+                if (RAGGED && (s0 + s) * BK + ((lane & 7) ^ (row & 7)) * 8 >= p.K) vo = kOutOfRange;
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_void *)(sa + u * 1024), 16, vo, (uint32_t)(s0 + s) * (uint32_t)(BK * 2), 0, 0);
             }
             if constexpr (WBITS == 4) {
@@ -496,13 +498,13 @@ __global__ __launch_bounds__(512, 1) void wq_gemm4_kernel(const WqGemm4Args p)
         }
 }
 
-template <int ACT, bool STAGE_GROUPS, int WBITS>
+template <int ACT, bool STAGE_GROUPS, int WBITS, bool RAGGED = false>
 int launch4(const WqGemm4Args &p, unsigned grid, hipStream_t s)
 {
     // four slots of activations (64 rows x 128 / 64 k) and raw weights (16 KiB either way), parameters, row sums
     constexpr size_t lds_bytes = (size_t)4 * 64 * (WBITS == 4 ? 256 : 128) + 4 * 16384 + 8 * 1024 + 2 * 2 * 64 * 4;
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
-    auto kern = wq_gemm4_kernel<ACT, STAGE_GROUPS, WBITS>;
+    auto kern = wq_gemm4_kernel<ACT, STAGE_GROUPS, WBITS, RAGGED>;
     static int attr_status = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (attr_status != hipSuccess) return MI355_ERR_LAUNCH;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds_bytes, s, p);
@@ -582,6 +584,7 @@ int launch_wq_gemm4(const WqGemm4Plan &plan, const void *x, int act_f16, const v
     const int64_t tiles = (int64_t)plan.tiles_m * plan.strips;
     (void)tiles;
     const unsigned grid = (unsigned)((plan.strips + 7) / 8 * 8 * plan.tiles_m * plan.S);
+    if (w_bits == 8 && K % 64 != 0) return act_f16 ? launch4<1, false, 8, true>(p, grid, s) : launch4<0, false, 8, true>(p, grid, s);
     if (w_bits == 8) return act_f16 ? launch4<1, false, 8>(p, grid, s) : launch4<0, false, 8>(p, grid, s);
     // int4: a variant of its own where a scale group is one stage
     if (p.grouped && plan.gstages == 1) return act_f16 ? launch4<1, true, 4>(p, grid, s) : launch4<0, true, 4>(p, grid, s);
