@@ -19,10 +19,11 @@ struct WqGemmPlan {
 
 // layout 1: weight rows contiguous along N, `ldw` elements (int8 bytes / int32 words) between k rows;
 // layout 2: int8 stored [N, K], `ldw` bytes between columns; anything else: not eligible.
+// `room`: the workspace that a split of K may use.
 __attribute__((visibility("hidden"))) WqGemmPlan make_wq_gemm_plan(int64_t M, int64_t N, int64_t K, int w_bits,
                                                                    int64_t group_size, int layout, int64_t ldw,
                                                                    int64_t ldx, const void *x, const void *w,
-                                                                   const void *scale, const void *offset);
+                                                                   const void *scale, const void *offset, size_t room = ~(size_t)0);
 
 // Launches the tiled kernel; `workspace` holds counter_bytes + partial_bytes when plan.S > 1.
 __attribute__((visibility("hidden"))) int launch_wq_gemm(const WqGemmPlan &plan, const void *x, int act_f16, const void *w,

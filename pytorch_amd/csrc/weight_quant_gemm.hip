@@ -497,7 +497,7 @@ int launch_any(WqGemmArgs &p, const WqGemmPlan &pl, hipStream_t s)
 } // namespace
 
 WqGemmPlan make_wq_gemm_plan(int64_t M, int64_t N, int64_t K, int w_bits, int64_t group_size, int layout, int64_t ldw,
-                             int64_t ldx, const void *x, const void *w, const void *scale, const void *offset)
+                             int64_t ldx, const void *x, const void *w, const void *scale, const void *offset, size_t room)
 {
     WqGemmPlan pl{};
     pl.k_major = layout == 2;
@@ -528,11 +528,12 @@ WqGemmPlan make_wq_gemm_plan(int64_t M, int64_t N, int64_t K, int w_bits, int64_
     if (const int f = knob(kKnobWqgSplit))              // tuning aid
         if (f >= 1 && f <= pl.n_units) S = f;
     if (S > 1 && ((uint64_t)S * pl.bm * bn * 4 >= (1ull << 32) || (size_t)tiles * 4 > kWorkspaceCounterBytes)) S = 1;
+    const uint64_t chunk_bytes = (uint64_t)tiles * pl.bm * bn * 4;
+    while (S > 1 && kWorkspaceZeroBytes + (uint64_t)S * chunk_bytes > room) S--;
     pl.S = (int)S;
     pl.accum = pl.grouped && (pl.n_units + pl.S - 1) / pl.S > 1;
-    pl.partial_bytes = pl.S > 1 ? (size_t)tiles * pl.S * pl.bm * bn * 4 : 0;
+    pl.partial_bytes = pl.S > 1 ? (size_t)(pl.S * chunk_bytes) : 0;
     pl.counter_bytes = pl.S > 1 ? kWorkspaceZeroBytes : 0;
-    (void)bn;
     return pl;
 }
 

@@ -788,6 +788,9 @@ extern "C" size_t mi355_weight_quant_matmul_workspace(int64_t M, int64_t N, int6
     // Per layout it asks for the kernel the launch prefers (preferred_n_major_kernel); a kernel further down the order, which
     // only runs when a pointer is misaligned, falls through to the generic kernel if its own request is not met (the
     // streaming kernel would ask for S x M x N x 4 bytes at large M: hundreds of MiB that no launch of a sane caller uses).
+    // int8 [K, N] rows whose pitch is no multiple of 16 (a column slice of a wider weight) prefer the tiled kernel, which is
+    // asked for as well (17 MiB at most; 228x4160x1808 unsplit is 30 workgroups on 256 CUs).  Whatever else the real strides
+    // make a launch prefer is planned within the workspace that this query asks for.
     auto pad = [](int64_t v, int64_t to) { return (v + to - 1) / to * to; };
     size_t need = 0;
     for (int padded = 0; padded < 2; padded++) {
@@ -802,7 +805,7 @@ extern "C" size_t mi355_weight_quant_matmul_workspace(int64_t M, int64_t N, int6
         const WqKmGemmPlan kmg = w_bits == 8 ? make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_k_major, ldx, nullptr, nullptr, nullptr, nullptr) : WqKmGemmPlan{};
         if (kmg.ok && kmg.counter_bytes + kmg.partial_bytes > need) need = kmg.counter_bytes + kmg.partial_bytes;
         for (int layout = 1; layout <= (w_bits == 8 ? 2 : 1); layout++) {
-            if (layout == 1 ? preferred != kPreferGemm : kmg.ok) continue;
+            if (layout == 1 ? w_bits == 4 && preferred != kPreferGemm : kmg.ok) continue;
             const WqGemmPlan gp = make_wq_gemm_plan(M, N, K, w_bits, group_size, layout, layout == 2 ? ldw_k_major : ldw_n_major, ldx,
                                                     nullptr, nullptr, nullptr, nullptr);
             const size_t gneed = gp.counter_bytes + gp.partial_bytes;
@@ -866,6 +869,16 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
                            static_cast<uint16_t *>(out_bf16), (int)M, (int)N, (int)K, group, ldx, ldw_k, ldw_n, ldo, ld_param_g,
                            ld_param_n, kpacked ? 1 : 0, f16 ? 1 : 0);
         return check_launch();
+    };
+    // The workspace of a plan that splits K.  The query knows no strides, and a launch may split where the query did not: given a
+    // workspace of the size the query asks for, the launch plans within it; only a smaller one is refused.
+    const auto fit_workspace = [&](auto &plan, auto plan_within) -> int {
+        const size_t have = workspace ? workspace_bytes : 0;
+        if (plan.S > 1 && have < plan.counter_bytes + plan.partial_bytes) {
+            if (have < mi355_weight_quant_matmul_workspace(M, N, K, w_bits, group_size)) return MI355_ERR_WORKSPACE;
+            plan = plan_within(have);
+        }
+        return plan.S == 1 || aligned(workspace, 16) ? MI355_OK : MI355_ERR_ALIGNMENT;
     };
     if (kpacked) {
         if (repack_applies(M, N, K, group_size, ldx, x_bf16) && ldw_n % 4 == 0 && aligned(w, 16) && aligned(scale_bf16, 2) &&
@@ -1026,22 +1039,26 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
     // on to the next one when its own request is not met; the preferred one reports the missing workspace.
     const int preferred = n_major ? preferred_n_major_kernel(M, N, K, w_bits, group_size, ldw_k, ldx) : kPreferStream;
     const auto workspace_holds = [&](size_t bytes) { return workspace && workspace_bytes >= bytes && aligned(workspace, 16); };
-    const WqGemmPlan gp = make_wq_gemm_plan(M, N, K, w_bits, group_size, n_major ? 1 : 0, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16);
-    if (gp.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2)) &&
-        (gp.S == 1 || preferred >= kPreferGemm || workspace_holds(gp.counter_bytes + gp.partial_bytes))) {
-        if (gp.S > 1) {
-            if (!workspace || workspace_bytes < gp.counter_bytes + gp.partial_bytes) return MI355_ERR_WORKSPACE;
-            if (!aligned(workspace, 16)) return MI355_ERR_ALIGNMENT;
-        }
+    WqGemmPlan gp = make_wq_gemm_plan(M, N, K, w_bits, group_size, n_major ? 1 : 0, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16);
+    const bool gemm_runs = gp.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2));
+    if (gemm_runs && preferred >= kPreferGemm) {
+        const int st = fit_workspace(gp, [&](size_t room) {
+            return make_wq_gemm_plan(M, N, K, w_bits, group_size, 1, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
+        });
+        if (st != MI355_OK) return st;
+    }
+    if (gemm_runs && (gp.S == 1 || workspace_holds(gp.counter_bytes + gp.partial_bytes))) {
         return launch_wq_gemm(gp, x_bf16, f16 ? 1 : 0, w, w_bits, scale_bf16, offset_bf16, bias, out_bf16, M, N, K, ldx, ldw_k,
                               ldo, workspace, stream);
     }
     const WqPlan pl = make_plan(M, N, K, w_bits, group_size, n_major, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16);
     if (!pl.fast) return generic();
-    if (pl.S > 1) {
-        if (preferred != kPreferStream && !workspace_holds(pl.partial_bytes + pl.counter_bytes)) return generic();
-        if (!workspace || workspace_bytes < pl.partial_bytes + pl.counter_bytes) return MI355_ERR_WORKSPACE;
-        if (!aligned(workspace, 16)) return MI355_ERR_ALIGNMENT;
+    if (pl.S > 1 && !workspace_holds(pl.partial_bytes + pl.counter_bytes)) {
+        // (it may need its split for its activations to fit the LDS, so there is no plan within a smaller workspace)
+        if (preferred != kPreferStream) return generic();
+        const size_t have = workspace ? workspace_bytes : 0;
+        if (have >= pl.partial_bytes + pl.counter_bytes) return MI355_ERR_ALIGNMENT;
+        return have < mi355_weight_quant_matmul_workspace(M, N, K, w_bits, group_size) ? MI355_ERR_WORKSPACE : generic();
     }
 
     WqArgs p;

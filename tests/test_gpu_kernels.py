@@ -1518,6 +1518,26 @@ def test_weight_quant_padded_rows_get_their_workspace(capi, golden, bits, N):
     bf16_gate(out, torch.from_numpy(gold), floor=True)
 
 
+@pytest.mark.parametrize("bits,M,K,N,pitch", [(8, 82, 664, 1368, 1372), (8, 228, 1088, 904, 908), (8, 40, 512, 256, 264),
+                                              (4, 110, 1536, 544, 69), (4, 64, 768, 256, 35)])
+def test_weight_quant_column_slice_of_a_wider_weight(capi, golden, bits, M, K, N, pitch):
+    """More than 32 rows and words along N in rows whose pitch is no multiple of 16 bytes (columns cut out of a wider weight): the
+    tiled kernel through LDS images, with K split and with a workspace of exactly the size the query asks for (int4: unsplit)."""
+    if bits == 8:
+        d = workloads.w8a16_inputs(seed=N, M=M, K=K, N=N)
+        gs, cols = 0, N
+    else:
+        d = workloads.w4a16_inputs(seed=N, M=M, K=K, N=N, group_size=128)
+        gs, cols = 128, N // 8
+    wide = torch.full((K, pitch), 77, dtype=d["weight"].dtype)
+    wide[:, :cols] = d["weight"]
+    capi._wq_workspaces.clear()
+    out = capi.weight_quant_matmul(d["x"].cuda(), wide.cuda()[:, :cols], d["antiquant_scale"].cuda(), d["antiquant_offset"].cuda(), group_size=gs)
+    _, gold = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]),
+                                         _bits(d["antiquant_offset"]), group_size=gs)
+    bf16_gate(out, torch.from_numpy(gold))
+
+
 def test_w4a16_repeated_launches_reuse_workspace(capi, golden):
     """The split-K exchange reuses one workspace and its arrival counters across launches: alternate two
     problems many times and check every result (a stale partial sum or counter would show up here)."""

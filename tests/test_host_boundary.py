@@ -477,3 +477,31 @@ def test_direct_calls_keep_the_packets_behaviour(pa):
     op(x, smooth_scales=sm.as_subclass(Sub))
     assert [s[0] for s in seen] == ["function mode", "dispatch mode", "subclass", "subclass"]
     assert seen[0][1] is op and seen[1][1] is op.default
+
+
+def _weight_quant_status(M, N, K, bits, group, ldx, ldw_k, ldw_n, workspace_bytes=None):
+    """Status of mi355_weight_quant_matmul on addresses that nothing is mapped at, with the workspace its own query asks for (or
+    `workspace_bytes`): host logic only.  Without a GPU every call that the planners accept ends in the launch error."""
+    import ctypes
+    from pytorch_amd import _capi
+    if torch.cuda.is_available():
+        pytest.skip("the addresses are not real")
+    L, p = _capi.lib(), [ctypes.c_void_p(i << 32) for i in range(1, 8)]
+    need = L.mi355_weight_quant_matmul_workspace(M, N, K, bits, group) if workspace_bytes is None else workspace_bytes
+    ld_param = N if group and group != K else 0
+    return L.mi355_weight_quant_matmul(p[0], 0, p[1], bits, p[2], p[3], p[4], p[5], M, N, K, group, ld_param, 1, ldx, ldw_k, ldw_n, N,
+                                       p[6] if need else None, need, None)
+
+
+_LAUNCH_ERROR, _WORKSPACE_ERROR = -5, -4
+
+
+@pytest.mark.parametrize("bits,M,K,N,group", [(8, 82, 664, 13696, 0), (8, 1253, 1152, 704, 0), (8, 228, 4160, 1808, 0), (8, 40, 1000, 1024, 0),
+                                              (8, 33, 4096, 4096, 0), (8, 300, 4096, 1024, 128), (4, 64, 4096, 2048, 128),
+                                              (4, 110, 1536, 544, 128), (4, 1940, 10624, 1952, 0)])
+@pytest.mark.parametrize("pitch", [0, 1, 2, 3, 4, 8, 16])
+def test_weight_quant_runs_with_the_workspace_it_asks_for(bits, M, K, N, group, pitch):
+    """Weights with words along N whose rows are cut out of a wider matrix, at every pitch: the query knows no strides, and what it
+    asks for has to do for the kernel that the launch picks by the real ones.  (pitch in words of four bytes.)"""
+    ldw = N // 8 + pitch if bits == 4 else N + 4 * pitch
+    assert _weight_quant_status(M, N, K, bits, group, K, ldw, 1) == _LAUNCH_ERROR
