@@ -506,7 +506,8 @@ WqGemmPlan make_wq_gemm_plan(int64_t M, int64_t N, int64_t K, int w_bits, int64_
     const int64_t group = group_size > 0 ? group_size : K;
     pl.grouped = group_size > 0 && group != K;
     const bool layout_ok = layout == 1 ? ldw_bytes >= row_bytes && (uint64_t)K * (uint64_t)ldw_bytes < (1ull << 32)
-                                       : layout == 2 && w_bits == 8 && ldw >= K && (uint64_t)N * (uint64_t)ldw < (1ull << 32);
+                                       // (one scale per column: weight_quant_kmajor_gemm.hip takes everything that this kernel would)
+                                       : layout == 2 && w_bits == 8 && pl.grouped && ldw >= K && (uint64_t)N * (uint64_t)ldw < (1ull << 32);
     pl.ok = M > 32 && layout_ok && K >= 128 && (K % 128 == 0 ? group % 128 == 0 : K % 8 == 0 && !pl.grouped && w_bits == 8) && N % 8 == 0 && ldw_bytes % 4 == 0 &&
             ldx % 8 == 0 && (x == nullptr || aligned(x, 16)) && (w == nullptr || aligned(w, 4)) &&
             (scale == nullptr || aligned(scale, 4)) && (offset == nullptr || aligned(offset, 4)) &&

@@ -13,10 +13,12 @@ struct WqKmGemmPlan {
     size_t counter_bytes, partial_bytes;   // workspace when S > 1: [arrival counters | partial sums]
 };
 
-// `ldw`: bytes between columns.  Null pointers (the workspace query) count as aligned.
+// `ldw`: bytes between columns.  Null pointers (the workspace query) count as aligned.  `room`: the workspace that a split of K
+// may use.
 __attribute__((visibility("hidden"))) WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw,
                                                                             int64_t ldx, const void *x, const void *w,
-                                                                            const void *scale, const void *offset);
+                                                                            const void *scale, const void *offset,
+                                                                            size_t room = ~(size_t)0);
 
 // Launches the kernel; `workspace` holds counter_bytes + partial_bytes when plan.S > 1.
 __attribute__((visibility("hidden"))) int launch_wq_kmajor_gemm(const WqKmGemmPlan &plan, const void *x, int act_f16, const void *w,

@@ -349,11 +349,14 @@ int launch_act(const WqKmGemmArgs &p, int wtm, hipStream_t s)
 } // namespace
 
 WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw, int64_t ldx, const void *x,
-                                      const void *w, const void *scale, const void *offset)
+                                      const void *w, const void *scale, const void *offset, size_t room)
 {
     WqKmGemmPlan pl{};
+    // the rows of a tile are addressed with 32-bit buffer offsets: rows far apart (one token of every sequence of a [128, 1024, 4096]
+    // batch: a pitch of 4194304) rule out the tall tiles
+    const auto offsets_fit = [&](int wtm) { return (uint64_t)(64 * wtm) * (uint64_t)ldx * 2 < (1ull << 31); };
     pl.ok = M > 32 && M <= 0x7fffffff && (group_size == 0 || group_size == K) && K >= 128 && K % 8 == 0 && N % 8 == 0 && ldw >= K &&
-            ldw % 4 == 0 && (uint64_t)N * (uint64_t)ldw < (1ull << 32) && ldx % 8 == 0 && (uint64_t)256 * (uint64_t)ldx * 2 < (1ull << 31) &&
+            ldw % 4 == 0 && (uint64_t)N * (uint64_t)ldw < (1ull << 32) && ldx % 8 == 0 && offsets_fit(2) &&
             (x == nullptr || aligned(x, 16)) && (w == nullptr || aligned(w, 4)) && (scale == nullptr || aligned(scale, 4)) &&
             (offset == nullptr || aligned(offset, 4)) && !knob(kKnobWqGemmOff);
     if (!pl.ok) return pl;
@@ -369,13 +372,15 @@ WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t g
     double best = 1e300;
     for (int wtm = 1; wtm <= 4; wtm++) {
         if (forced_bm > 0 && forced_bm % 64 == 0 && forced_bm <= 256 && forced_bm != 64 * wtm) continue;
+        if (!offsets_fit(wtm)) continue;
         const int64_t tiles = ((M + 64 * wtm - 1) / (64 * wtm)) * ((N + kBN - 1) / kBN);
         if (tiles > 0x7fffffff / 16) continue;
         for (int S = 1; S <= 16; S++) {
             const int64_t slots = wtm == 1 ? 2 * kNumCU : kNumCU, wgs = tiles * S;
             if (forced ? S != forced_split : S > 1 && (wgs > slots || stages / S < 4)) continue;
             const int64_t chunk_bytes = 64 * wtm * kBN * 4;
-            if (S > 1 && ((uint64_t)tiles * 4 > kWorkspaceCounterBytes || (uint64_t)(wgs * chunk_bytes) > ((uint64_t)128 << 20))) continue;
+            if (S > 1 && ((uint64_t)tiles * 4 > kWorkspaceCounterBytes || (uint64_t)(wgs * chunk_bytes) > ((uint64_t)128 << 20) ||
+                          kWorkspaceZeroBytes + (uint64_t)(wgs * chunk_bytes) > room)) continue;
             double us = (double)((wgs + slots - 1) / slots * ((stages + S - 1) / S)) * kStageUs[wtm == 1 && wgs <= kNumCU ? 0 : wtm];
             const double mem = (double)K * (double)N / kWeightBytesPerUs, l2 = (double)tiles * (128 * wtm + kBN) * (double)K / kL2BytesPerUs;
             us = kBaseUs + (us > mem ? us > l2 ? us : l2 : mem > l2 ? mem : l2);

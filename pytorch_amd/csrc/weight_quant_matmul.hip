@@ -674,7 +674,7 @@ struct WqKmPlan {
 };
 
 WqKmPlan make_kmajor_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw_n, int64_t ldx, const void *x,
-                          const void *w)
+                          const void *w, size_t room = ~(size_t)0)
 {
     WqKmPlan pl{};
     const int64_t group = group_size > 0 ? group_size : K;
@@ -698,6 +698,7 @@ WqKmPlan make_kmajor_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, i
         if (f >= 1 && f <= pl.n_units) S = f;
     if ((uint64_t)S * (uint64_t)M * (uint64_t)N * 4 >= (1ull << 32)) S = 1;
     if (S > 1 && (size_t)pl.tiles * pl.mchunks * sizeof(uint32_t) > kWorkspaceCounterBytes) S = 1;
+    while (S > 1 && kWorkspaceZeroBytes + (uint64_t)S * (uint64_t)M * (uint64_t)N * 4 > room) S--;
     if (wq_kmajor_decode_shape(M, N, K, group_size)) S = 1;   // the decode kernel splits K inside its workgroups
     pl.S = S;
     pl.partial_bytes = S > 1 ? (size_t)S * M * N * sizeof(float) : 0;
@@ -949,31 +950,31 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             const int st = launch_wq_kmajor_decode(d, f16 ? 1 : 0, s);
             if (st != MI355_ERR_UNSUPPORTED) return st;
         }
-        const WqKmGemmPlan kg = make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
-        if (kg.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2))) {
-            if (kg.S > 1) {
-                if (!workspace || workspace_bytes < kg.counter_bytes + kg.partial_bytes) return MI355_ERR_WORKSPACE;
-                if (!aligned(workspace, 16)) return MI355_ERR_ALIGNMENT;
-            }
+        const bool out_ok = aligned(out_bf16, 2) && (!bias || aligned(bias, 2));
+        WqKmGemmPlan kg = make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
+        if (kg.ok && out_ok) {
+            const int st = fit_workspace(kg, [&](size_t room) {
+                return make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
+            });
+            if (st != MI355_OK) return st;
+        }
+        if (kg.ok && out_ok)
             return launch_wq_kmajor_gemm(kg, x_bf16, f16 ? 1 : 0, w, scale_bf16, offset_bf16, bias, out_bf16, M, N, K, ldx, ldw_n, ldo,
                                          workspace, stream);
-        }
-        const WqGemmPlan gk = make_wq_gemm_plan(M, N, K, 8, group_size, 2, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
-        if (gk.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2))) {
-            if (gk.S > 1) {
-                if (!workspace || workspace_bytes < gk.counter_bytes + gk.partial_bytes) return MI355_ERR_WORKSPACE;
-                if (!aligned(workspace, 16)) return MI355_ERR_ALIGNMENT;
-            }
+        WqGemmPlan gk = make_wq_gemm_plan(M, N, K, 8, group_size, 2, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
+        if (gk.ok && out_ok) {
+            const int st = fit_workspace(gk, [&](size_t room) {
+                return make_wq_gemm_plan(M, N, K, 8, group_size, 2, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
+            });
+            if (st != MI355_OK) return st;
             return launch_wq_gemm(gk, x_bf16, f16 ? 1 : 0, w, 8, scale_bf16, offset_bf16, bias, out_bf16, M, N, K, ldx, ldw_n, ldo,
                                   workspace, stream);
         }
-        const WqKmPlan km = make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
+        WqKmPlan km = make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
         const bool params_ok = aligned(scale_bf16, 2) && (!offset_bf16 || aligned(offset_bf16, 2));
         if (km.fast && params_ok) {
-            if (km.S > 1) {
-                if (!workspace || workspace_bytes < km.partial_bytes + km.counter_bytes) return MI355_ERR_WORKSPACE;
-                if (!aligned(workspace, 16)) return MI355_ERR_ALIGNMENT;
-            }
+            const int st = fit_workspace(km, [&](size_t room) { return make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, room); });
+            if (st != MI355_OK) return st;
             WqArgs p{};
             p.x = static_cast<const uint16_t *>(x_bf16);
             p.w = w;

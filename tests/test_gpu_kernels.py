@@ -1538,6 +1538,19 @@ def test_weight_quant_column_slice_of_a_wider_weight(capi, golden, bits, M, K, N
     bf16_gate(out, torch.from_numpy(gold))
 
 
+@pytest.mark.parametrize("M,K,N,ldx", [(33, 512, 264, 4194304), (33, 200, 136, 4194304), (33, 256, 128, 8388600)])
+def test_w8a16_activation_rows_far_apart(capi, golden, M, K, N, ldx):
+    """int8 weight stored [N, K] and rows of activations so far apart that 32-bit offsets reach 128 rows but not 256, with a workspace
+    of the size the query (which plans dense rows) asks for."""
+    d = workloads.w8a16_inputs(seed=M + K, M=M, K=K, N=N, weight_nk=True)
+    x = torch.empty((M - 1) * ldx + K, dtype=d["x"].dtype, device="cuda").as_strided((M, K), (ldx, 1))
+    x.copy_(d["x"])
+    capi._wq_workspaces.clear()
+    out = capi.weight_quant_matmul(x, d["weight"].cuda(), d["antiquant_scale"].cuda(), d["antiquant_offset"].cuda())
+    _, want = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]), _bits(d["antiquant_offset"]))
+    bf16_gate(out, torch.from_numpy(want))
+
+
 def test_w4a16_repeated_launches_reuse_workspace(capi, golden):
     """The split-K exchange reuses one workspace and its arrival counters across launches: alternate two
     problems many times and check every result (a stale partial sum or counter would show up here)."""

@@ -505,3 +505,12 @@ def test_weight_quant_runs_with_the_workspace_it_asks_for(bits, M, K, N, group, 
     asks for has to do for the kernel that the launch picks by the real ones.  (pitch in words of four bytes.)"""
     ldw = N // 8 + pitch if bits == 4 else N + 4 * pitch
     assert _weight_quant_status(M, N, K, bits, group, K, ldw, 1) == _LAUNCH_ERROR
+
+
+@pytest.mark.parametrize("M,K,N", [(128, 4096, 4096), (64, 1024, 1024), (192, 11264, 1664), (33, 512, 264), (300, 1000, 2048)])
+@pytest.mark.parametrize("ldx", [4194296, 4194304, 8388600, 8388608])
+def test_weight_quant_activation_rows_far_apart(M, K, N, ldx):
+    """One token of every sequence of a long batch: rows of activations up to 2^23 elements apart, which only part of a kernel's tiles
+    can address, against an int8 weight of either layout, with the workspace that the query (which plans dense rows) asks for."""
+    assert _weight_quant_status(M, N, K, 8, 0, ldx, 1, K) == _LAUNCH_ERROR
+    assert _weight_quant_status(M, N, K, 8, 0, ldx, N, 1) == _LAUNCH_ERROR
