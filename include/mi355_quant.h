@@ -274,6 +274,8 @@ int mi355_quant_matmul_noalloc(const int8_t *a, const int8_t *b, const float *pe
  *   out[m*ldo+n] = round( sum_k float(x[m,k]) * ((float(w[k,n]) + float(offset[g,n])) * float(scale[g,n])) + float(bias[n]) )
  *   group_size: 0 (per channel) or a multiple of 32 that divides K
  *   workspace: at least mi355_weight_quant_matmul_workspace(...) bytes (may be NULL when that is 0), 16-byte aligned.
+ *              (int8 with a K that is not a multiple of 32, or stored [N, K] and not a multiple of 128, also runs without
+ *              one: K is then not split.)
  *              It holds the arrival counters and partial sums of a split over K; its first
  *              MI355_WORKSPACE_ZERO_BYTES must be zero before the first launch that uses the buffer and are left
  *              zero by every launch (see mi355_quant_matmul), so one zero-initialised buffer can serve all later

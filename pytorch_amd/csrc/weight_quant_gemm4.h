@@ -15,10 +15,11 @@ struct WqGemm4Plan {
     size_t zone_bytes;       // bytes of the workspace's zero area used for the exchange (S > 1)
 };
 
+// `room`: the workspace that a split of K may use (its zero area).
 __attribute__((visibility("hidden"))) WqGemm4Plan make_wq_gemm4_plan(int64_t M, int64_t N, int64_t K, int w_bits,
                                                                      int64_t group_size, int64_t ldw_k, int64_t ldx,
                                                                      const void *x, const void *w, const void *scale,
-                                                                     const void *offset);
+                                                                     const void *offset, size_t room = ~(size_t)0);
 
 __attribute__((visibility("hidden"))) int launch_wq_gemm4(const WqGemm4Plan &plan, const void *x, int act_f16, const void *w,
                                                           int w_bits, const void *scale, const void *offset, const void *bias, void *out,

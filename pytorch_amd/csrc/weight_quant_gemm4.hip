@@ -514,7 +514,7 @@ int launch4(const WqGemm4Args &p, unsigned grid, hipStream_t s)
 } // namespace
 
 WqGemm4Plan make_wq_gemm4_plan(int64_t M, int64_t N, int64_t K, int w_bits, int64_t group_size, int64_t ldw_k, int64_t ldx,
-                               const void *x, const void *w, const void *scale, const void *offset)
+                               const void *x, const void *w, const void *scale, const void *offset, size_t room)
 {
     WqGemm4Plan pl{};
     // int4: rows of N / 8 words, 128-row stages, 128-byte strips; int8: rows of N bytes, 64-row stages, 256-byte strips
@@ -541,6 +541,7 @@ WqGemm4Plan make_wq_gemm4_plan(int64_t M, int64_t N, int64_t K, int w_bits, int6
     if (S > 8) S = 8;
     if (const int f = knob(kKnobWqgSplit))
         if (f >= 1 && f <= units) S = f;
+    if (room < kWorkspaceZeroBytes) S = 1;
     // the sums of S - 1 chunks per tile and one word per tile (the XCD of its collector)
     auto zone = [&](int64_t s) { return (uint64_t)(s - 1) * (uint64_t)tiles * (uint64_t)pl.bm * 256u * 4u + (uint64_t)tiles * 4u; };
     while (S > 1 && (zone(S) > kWorkspaceZoneBytes || (!grouped && stages % S != 0))) S--;

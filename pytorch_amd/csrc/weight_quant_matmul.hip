@@ -872,12 +872,19 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
         return check_launch();
     };
     // The workspace of a plan that splits K.  The query knows no strides, and a launch may split where the query did not: given a
-    // workspace of the size the query asks for, the launch plans within it; only a smaller one is refused.
-    const auto fit_workspace = [&](auto &plan, auto plan_within) -> int {
-        const size_t have = workspace ? workspace_bytes : 0;
-        if (plan.S > 1 && have < plan.counter_bytes + plan.partial_bytes) {
-            if (have < mi355_weight_quant_matmul_workspace(M, N, K, w_bits, group_size)) return MI355_ERR_WORKSPACE;
-            plan = plan_within(have);
+    // workspace of the size the query asks for, the launch plans within it; only a smaller one is refused.  An int8 K that is not a
+    // multiple of 128 also runs without one (a step of 32 is enough where the streaming kernel reads the weight).
+    const bool n_major = w_bits == 4 || (ldw_n == 1 && ldw_k >= N);
+    const size_t room = workspace ? workspace_bytes : 0;
+    const auto must_have = [&]() {
+        if (room >= mi355_weight_quant_matmul_workspace(M, N, K, w_bits, group_size)) return false;
+        if (w_bits != 8 || group != K || K % 128 == 0) return true;
+        return K % 32 == 0 && make_plan(M, N, K, 8, group_size, n_major, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16).S > 1;
+    };
+    const auto fit_workspace = [&](auto &plan, size_t bytes, auto plan_within_room) -> int {
+        if (plan.S > 1 && room < bytes) {
+            if (must_have()) return MI355_ERR_WORKSPACE;
+            plan = plan_within_room();
         }
         return plan.S == 1 || aligned(workspace, 16) ? MI355_OK : MI355_ERR_ALIGNMENT;
     };
@@ -953,7 +960,7 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
         const bool out_ok = aligned(out_bf16, 2) && (!bias || aligned(bias, 2));
         WqKmGemmPlan kg = make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
         if (kg.ok && out_ok) {
-            const int st = fit_workspace(kg, [&](size_t room) {
+            const int st = fit_workspace(kg, kg.counter_bytes + kg.partial_bytes, [&]() {
                 return make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
             });
             if (st != MI355_OK) return st;
@@ -963,7 +970,7 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
                                          workspace, stream);
         WqGemmPlan gk = make_wq_gemm_plan(M, N, K, 8, group_size, 2, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
         if (gk.ok && out_ok) {
-            const int st = fit_workspace(gk, [&](size_t room) {
+            const int st = fit_workspace(gk, gk.counter_bytes + gk.partial_bytes, [&]() {
                 return make_wq_gemm_plan(M, N, K, 8, group_size, 2, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
             });
             if (st != MI355_OK) return st;
@@ -973,7 +980,7 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
         WqKmPlan km = make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
         const bool params_ok = aligned(scale_bf16, 2) && (!offset_bf16 || aligned(offset_bf16, 2));
         if (km.fast && params_ok) {
-            const int st = fit_workspace(km, [&](size_t room) { return make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, room); });
+            const int st = fit_workspace(km, km.counter_bytes + km.partial_bytes, [&]() { return make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, room); });
             if (st != MI355_OK) return st;
             WqArgs p{};
             p.x = static_cast<const uint16_t *>(x_bf16);
@@ -1000,7 +1007,6 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             return f16 ? launch_kmajor_any<1>(p, km, s) : launch_kmajor_any<0>(p, km, s);
         }
     }
-    const bool n_major = w_bits == 4 || (ldw_n == 1 && ldw_k >= N);
     if (w_bits == 4) {
         // at most 32 rows, words along N: the barrier-free decode kernel
         const WqDecodePlan dp = make_wq_decode_plan(M, N, K, 4, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16);
@@ -1025,12 +1031,12 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
     }
     if (w_bits == 8 && n_major) {
         // int8 [K, N], more than 32 rows: the same register-expanding kernel
-        const WqGemm4Plan g8 = make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16);
+        WqGemm4Plan g8 = make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16);
         if (g8.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2))) {
-            if (g8.S > 1) {
-                if (!workspace || workspace_bytes < kWorkspaceZeroBytes) return MI355_ERR_WORKSPACE;
-                if (!aligned(workspace, 16)) return MI355_ERR_ALIGNMENT;
-            }
+            const int st = fit_workspace(g8, kWorkspaceZeroBytes, [&]() {
+                return make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
+            });
+            if (st != MI355_OK) return st;
             return launch_wq_gemm4(g8, x_bf16, f16 ? 1 : 0, w, 8, scale_bf16, offset_bf16, bias, out_bf16, M, N, K, group_size, ldx, ldw_k,
                                    ldo, workspace, stream);
         }
@@ -1043,7 +1049,7 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
     WqGemmPlan gp = make_wq_gemm_plan(M, N, K, w_bits, group_size, n_major ? 1 : 0, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16);
     const bool gemm_runs = gp.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2));
     if (gemm_runs && preferred >= kPreferGemm) {
-        const int st = fit_workspace(gp, [&](size_t room) {
+        const int st = fit_workspace(gp, gp.counter_bytes + gp.partial_bytes, [&]() {
             return make_wq_gemm_plan(M, N, K, w_bits, group_size, 1, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
         });
         if (st != MI355_OK) return st;
@@ -1057,9 +1063,8 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
     if (pl.S > 1 && !workspace_holds(pl.partial_bytes + pl.counter_bytes)) {
         // (it may need its split for its activations to fit the LDS, so there is no plan within a smaller workspace)
         if (preferred != kPreferStream) return generic();
-        const size_t have = workspace ? workspace_bytes : 0;
-        if (have >= pl.partial_bytes + pl.counter_bytes) return MI355_ERR_ALIGNMENT;
-        return have < mi355_weight_quant_matmul_workspace(M, N, K, w_bits, group_size) ? MI355_ERR_WORKSPACE : generic();
+        if (room >= pl.partial_bytes + pl.counter_bytes) return MI355_ERR_ALIGNMENT;
+        return must_have() ? MI355_ERR_WORKSPACE : generic();
     }
 
     WqArgs p;

@@ -1551,6 +1551,17 @@ def test_w8a16_activation_rows_far_apart(capi, golden, M, K, N, ldx):
     bf16_gate(out, torch.from_numpy(want))
 
 
+@pytest.mark.parametrize("nk", [True, False])
+@pytest.mark.parametrize("M,K,N", [(40, 1000, 1024), (118, 456, 112), (20, 2168, 1024), (300, 2184, 264)])
+def test_w8a16_ragged_k_without_a_workspace(capi, golden, monkeypatch, M, K, N, nk):
+    """A K that is not a multiple of 128 (nor of 32) runs without a workspace: plans that would split K run unsplit."""
+    d = workloads.w8a16_inputs(seed=M + K, M=M, K=K, N=N, weight_nk=nk)
+    monkeypatch.setattr(capi, "_wq_workspace", lambda device, nbytes: None)
+    out = capi.weight_quant_matmul(d["x"].cuda(), d["weight"].cuda(), d["antiquant_scale"].cuda(), d["antiquant_offset"].cuda())
+    _, want = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]), _bits(d["antiquant_offset"]))
+    bf16_gate(out, torch.from_numpy(want))
+
+
 def test_w4a16_repeated_launches_reuse_workspace(capi, golden):
     """The split-K exchange reuses one workspace and its arrival counters across launches: alternate two
     problems many times and check every result (a stale partial sum or counter would show up here)."""

@@ -514,3 +514,14 @@ def test_weight_quant_activation_rows_far_apart(M, K, N, ldx):
     can address, against an int8 weight of either layout, with the workspace that the query (which plans dense rows) asks for."""
     assert _weight_quant_status(M, N, K, 8, 0, ldx, 1, K) == _LAUNCH_ERROR
     assert _weight_quant_status(M, N, K, 8, 0, ldx, N, 1) == _LAUNCH_ERROR
+
+
+@pytest.mark.parametrize("M,K,N,pad", [(40, 1000, 1024, 0), (118, 352, 112, 4), (85, 1112, 2048, 8), (20, 2160, 1024, 16), (8, 264, 8192, 0), (300, 8200, 512, 4)])
+def test_weight_quant_int8_ragged_k_needs_no_workspace(M, K, N, pad):
+    """An int8 K that is not a multiple of 128 runs without a workspace, in either layout; any other K asks for the one it needs."""
+    assert _weight_quant_status(M, N, K, 8, 0, K, 1, K + pad, 0) == _LAUNCH_ERROR
+    if K % 32:
+        assert _weight_quant_status(M, N, K, 8, 0, K, N + pad, 1, 0) == _LAUNCH_ERROR
+    assert _weight_quant_status(200, 1024, 4096, 8, 0, 4096, 1, 4096, 0) == _WORKSPACE_ERROR
+    assert _weight_quant_status(48, 1024, 4096, 8, 0, 4096, 1024, 1, 0) == _WORKSPACE_ERROR
+    assert _weight_quant_status(48, 1024, 4000, 8, 0, 4000, 1024, 1, 0) == _WORKSPACE_ERROR
