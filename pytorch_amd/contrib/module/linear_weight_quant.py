@@ -74,27 +74,42 @@ class LinearWeightQuant(PreparedCopiesMixin, nn.Module):
     def _as_group_major(param):
         return param.transpose(-1, -2) if param is not None and param.dim() == 2 else param
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def _runs_unprepared(self, x: torch.Tensor) -> bool:
+        # 2 to 32 rows: the decode kernel for the module's own storage (words along K) is the faster one
+        # (int4 [14336, 4096/8], 8 / 32 rows: 9.8 / 15.4 us against 10.3 / 17.2 on the repacked copy)
+        rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
+        return self.antiquant_group_size == 128 and 2 <= rows <= 32
+
+    def _eager(self, x):
+        """The forward pass with parameters read from their table and, where the copy made by ``prepare_()`` is not used, one native
+        call; ``NotImplemented`` for what ``forward`` has to handle."""
         prepared = self.__dict__.get("_prepared")
         weight = parameter(self, "weight")
         quant_scale, quant_offset, bias = parameter(self, "quant_scale"), parameter(self, "quant_offset"), parameter(self, "bias")
-        if prepared is not None and weight.dtype == torch.int32 and self.antiquant_group_size == 128:
-            # 2 to 32 rows: the decode kernel for the module's own storage (words along K) is the faster one
-            # (int4 [14336, 4096/8], 8 / 32 rows: 9.8 / 15.4 us against 10.3 / 17.2 on the repacked copy)
-            rows = x.numel() // x.shape[-1] if x.shape[-1] else 0
-            if 2 <= rows <= 32:
-                prepared = None
-        if prepared is not None:
+        if prepared is not None and not (weight.dtype == torch.int32 and self._runs_unprepared(x)):
             weight, scale, offset = prepared
             return torch.ops.npu.npu_weight_quant_batchmatmul(x, weight, scale, offset, quant_scale, quant_offset, bias,
                                                               self.antiquant_group_size, self.inner_precise,
                                                               weight_dtype=self.weight_dtype)
-        scale, offset = parameter(self, "antiquant_scale"), parameter(self, "antiquant_offset")
-        if self.weight_dtype is None and not torch.compiler.is_compiling():
-            out = _op_call.linear_weight_quant(x, weight, scale, offset, quant_scale, quant_offset, bias, self.antiquant_group_size,
-                                               self.inner_precise)
+        if self.weight_dtype is not None or torch.compiler.is_compiling():
+            return NotImplemented
+        return _op_call.linear_weight_quant(x, weight, parameter(self, "antiquant_scale"), parameter(self, "antiquant_offset"), quant_scale,
+                                            quant_offset, bias, self.antiquant_group_size, self.inner_precise)
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if not torch.jit.is_scripting():
+            out = self._eager(x)
             if out is not NotImplemented:
                 return out
+        prepared = getattr(self, "_prepared", None)
+        if prepared is not None and self.weight.dtype == torch.int32 and self._runs_unprepared(x):
+            prepared = None
+        if prepared is not None:
+            weight, scale, offset = prepared
+            return torch.ops.npu.npu_weight_quant_batchmatmul(x, weight, scale, offset, self.quant_scale, self.quant_offset,
+                                                              self.bias, self.antiquant_group_size, self.inner_precise,
+                                                              weight_dtype=self.weight_dtype)
         return torch.ops.npu.npu_weight_quant_batchmatmul(
-            x, weight.transpose(-1, -2), self._as_group_major(scale), self._as_group_major(offset), quant_scale, quant_offset, bias,
+            x, self.weight.transpose(-1, -2), self._as_group_major(self.antiquant_scale),
+            self._as_group_major(self.antiquant_offset), self.quant_scale, self.quant_offset, self.bias,
             self.antiquant_group_size, self.inner_precise, weight_dtype=self.weight_dtype)

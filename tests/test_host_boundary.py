@@ -368,6 +368,17 @@ def test_linear_weight_quant_marshalling(pa, monkeypatch):
     assert args[7] == 128 and args[8] == 0 and kwargs == {"weight_dtype": None}
 
 
+def test_linear_weight_quant_can_be_scripted(pa):
+    from pytorch_amd.contrib.module import LinearWeightQuant
+    m = LinearWeightQuant(256, 64, bias=False, antiquant_offset=True, antiquant_group_size=128).to("meta")
+    m.weight.data = _m(64, 256, dtype=torch.int8)
+    m.antiquant_scale.data = _m(64, 2, dtype=torch.bfloat16)
+    m.antiquant_offset.data = _m(64, 2, dtype=torch.bfloat16)
+    s = torch.jit.script(m)
+    assert "npu::npu_weight_quant_batchmatmul" in str(s.inlined_graph)
+    assert s(_m(3, 256, dtype=torch.bfloat16)).shape == (3, 64) and dict(s.state_dict()).keys() == dict(m.state_dict()).keys()
+
+
 def test_prepared_copies_are_dropped_when_the_module_moves_or_reloads(pa):
     """prepare_() keeps derived weight copies in plain attributes; .to()/.half()/load_state_dict must drop them so that a
     stale or wrong-device copy can never be used (no kernel runs here: the copies are set by hand)."""
