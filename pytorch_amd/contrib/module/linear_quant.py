@@ -86,7 +86,8 @@ class _QuantLinearBase(PreparedCopiesMixin, nn.Module):
 
     def forward(self, linear_quant_input: torch.Tensor) -> torch.Tensor:
         x = linear_quant_input
-        weight, scale, offset = parameter(self, "weight"), parameter(self, "scale"), parameter(self, "offset")
+        weight = self.weight                                        # (not from the table: a tracer's proxy in its place must be seen)
+        scale, offset = parameter(self, "scale"), parameter(self, "offset")
         pertoken_scale, bias = parameter(self, "pertoken_scale"), parameter(self, "bias")
         if self._validate_dtypes or x.dtype != torch.int8 or weight.dtype != torch.int8:
             self._check_dtypes(x)

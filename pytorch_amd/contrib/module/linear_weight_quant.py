@@ -84,7 +84,9 @@ class LinearWeightQuant(PreparedCopiesMixin, nn.Module):
         """The forward pass with parameters read from their table and, where the copy made by ``prepare_()`` is not used, one native
         call; ``NotImplemented`` for what ``forward`` has to handle."""
         prepared = self.__dict__.get("_prepared")
-        weight = parameter(self, "weight")
+        weight = self.weight                                        # (not from the table: a tracer's proxy in its place must be seen)
+        if not isinstance(weight, torch.Tensor):
+            return NotImplemented
         quant_scale, quant_offset, bias = parameter(self, "quant_scale"), parameter(self, "quant_offset"), parameter(self, "bias")
         if prepared is not None and not (weight.dtype == torch.int32 and self._runs_unprepared(x)):
             weight, scale, offset = prepared

@@ -379,6 +379,35 @@ def test_linear_weight_quant_can_be_scripted(pa):
     assert s(_m(3, 256, dtype=torch.bfloat16)).shape == (3, 64) and dict(s.state_dict()).keys() == dict(m.state_dict()).keys()
 
 
+@pytest.mark.parametrize("prepared", [False, True])
+@pytest.mark.parametrize("own_input", [False, True])
+@pytest.mark.parametrize("weight_only", [True, False])
+def test_quant_linears_refuse_symbolic_tracing(pa, monkeypatch, weight_only, own_input, prepared):
+    """torch.fx.symbolic_trace stops at the modules' decisions on types and shapes; it must not get past them and leave the weight (or
+    the product with a tensor that the traced module owns) in the graph as a constant."""
+    from pytorch_amd import _op_call
+    from pytorch_amd.contrib.module import LinearQuant, LinearWeightQuant
+    for name in ("linear_quant", "linear_weight_quant"):           # (the native call is for the GPU: here it takes what it is given)
+        monkeypatch.setattr(_op_call, name, lambda x, w, *a: x.new_empty(x.shape[0], w.shape[0]) if type(x) is torch.Tensor else NotImplemented)
+
+    class Root(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.lin = LinearWeightQuant(256, 64, bias=False) if weight_only else LinearQuant(256, 64, bias=False)
+            self.lin.to("meta").weight.data = _m(64, 256, dtype=torch.int8)
+            if prepared and weight_only:
+                self.lin._prepared = (_m(256, 64, dtype=torch.int8), _m(64, dtype=torch.float32), None)
+            elif prepared:
+                self.lin._prepared_i8 = _m(64, 256, dtype=torch.int8)
+            self.register_buffer("x", _m(3, 256, dtype=torch.bfloat16 if weight_only else torch.int8))
+
+        def forward(self, y):
+            return self.lin(self.x if own_input else y)
+
+    with pytest.raises(torch.fx.proxy.TraceError):
+        torch.fx.symbolic_trace(Root())
+
+
 def test_prepared_copies_are_dropped_when_the_module_moves_or_reloads(pa):
     """prepare_() keeps derived weight copies in plain attributes; .to()/.half()/load_state_dict must drop them so that a
     stale or wrong-device copy can never be used (no kernel runs here: the copies are set by hand)."""
