@@ -12,6 +12,7 @@ struct WqGemm4Plan {
     int tiles_m, strips;     // workgroup tiles: row blocks x strips of 256 columns (128 bytes of an int4 row, 256 of an int8 row)
     int S;                   // workgroups that share a tile's K range
     int gstages;             // stages (128 rows of int4, 64 of int8) per scale group (per channel: all stages of a workgroup)
+    bool uneven;             // no split of K into equal chunks exists
     size_t zone_bytes;       // bytes of the workspace's zero area used for the exchange (S > 1)
 };
 

@@ -43,6 +43,7 @@ struct WqGemm4Args {
     uint32_t ldw_bytes, row_bytes;
     int M, N, K;
     int gstages;                    // stages per scale group
+    int units, unit_stages;         // what K is split in: scale groups, per channel stages
     int grouped;
     int tiles_m, strips, S;
     int l2_exchange;                // producers on the collector's XCD leave their sums in the L2
@@ -91,10 +92,9 @@ __global__ __launch_bounds__(512, 1) void wq_gemm4_kernel(const WqGemm4Args p)
     const int tile = strip * p.tiles_m + mb;
     const int m0 = mb * BM;
     const int n0 = strip * 256;
-    const int total_stages = RAGGED ? (p.K + BK - 1) / BK : p.K / BK;
-    const int units = total_stages / p.gstages;                // K is split in whole scale groups
-    const int u0 = (int)((int64_t)units * chunk / p.S), u1 = (int)((int64_t)units * (chunk + 1) / p.S);
-    const int s0 = u0 * p.gstages, NSTG = (u1 - u0) * p.gstages;
+    // K is split in whole scale groups, per channel in stages (the group is then longer than any chunk and ends with it)
+    const int u0 = p.units * chunk / p.S, u1 = p.units * (chunk + 1) / p.S;
+    const int s0 = u0 * p.unit_stages, NSTG = (u1 - u0) * p.unit_stages;
 
     // ---- global -> LDS.  Activations: unit = 4 rows x 256 B; LDS slot l of a unit is (row l / 16, chunk l % 16) and
     // holds global chunk (l % 16) ^ (row & 15).  Raw weights: unit = 8 row slots x 128 B; row slot sl holds row
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(512, 1) void wq_gemm4_kernel(const WqGemm4Args p)
     const __amdgpu_buffer_rsrc_t rsrc_w =
         make_rsrc(static_cast<const char *>(p.w) + (size_t)strip * ROW_B, (uint32_t)(p.K - 1) * p.ldw_bytes + strip_valid);
     const bool has_offset = p.offset != nullptr;
-    const uint32_t param_bytes = (uint32_t)(p.grouped ? units : 1) * (uint32_t)p.N * 2u;
+    const uint32_t param_bytes = (uint32_t)(p.grouped ? p.units : 1) * (uint32_t)p.N * 2u;
     const __amdgpu_buffer_rsrc_t rsrc_s = make_rsrc(p.scale, param_bytes);
     const __amdgpu_buffer_rsrc_t rsrc_o = make_rsrc(has_offset ? p.offset : p.scale, param_bytes);
     // a stage's 32 load units are dealt to the eight wavefronts; the parameters of a scale group (the strip's 256 scales
@@ -532,7 +532,9 @@ WqGemm4Plan make_wq_gemm4_plan(int64_t M, int64_t N, int64_t K, int w_bits, int6
     pl.strips = (int)((row_bytes + strip_bytes - 1) / strip_bytes);
     const int64_t stages = (K + bk - 1) / bk;
     const int64_t units = grouped ? K / group : stages;
-    // few tiles: split K in whole scale groups (per channel: in equal numbers of stages)
+    // few tiles: split K in whole scale groups; int4 per channel: in equal numbers of stages; int8: in numbers that differ by one at
+    // most, since a K that is not a multiple of 128 leaves counts that few splits divide (300x4288x2048, 67 stages: unsplit on 40
+    // workgroups 43.5 us, six ways 22.4; 128x5504x1024, 86 stages: two ways 33.7, eight ways 22.6)
     pl.bm = 64;
     pl.tiles_m = (int)((M + pl.bm - 1) / pl.bm);
     const int64_t tiles = (int64_t)pl.tiles_m * pl.strips;
@@ -544,10 +546,15 @@ WqGemm4Plan make_wq_gemm4_plan(int64_t M, int64_t N, int64_t K, int w_bits, int6
     if (room < kWorkspaceZeroBytes) S = 1;
     // the sums of S - 1 chunks per tile and one word per tile (the XCD of its collector)
     auto zone = [&](int64_t s) { return (uint64_t)(s - 1) * (uint64_t)tiles * (uint64_t)pl.bm * 256u * 4u + (uint64_t)tiles * 4u; };
-    while (S > 1 && (zone(S) > kWorkspaceZoneBytes || (!grouped && stages % S != 0))) S--;
+    while (S > 1 && zone(S) > kWorkspaceZoneBytes) S--;
+    if (!grouped) S = (stages + (stages + S - 1) / S - 1) / ((stages + S - 1) / S);   // no more chunks than their length asks for
+    int64_t even = S;
+    while (even > 1 && !grouped && stages % even != 0) even--;
+    if (w_bits == 4) S = even;
     pl.S = (int)S;
-    // per channel: one fold per workgroup, so a "group" is the workgroup's whole range
-    pl.gstages = (int)(grouped ? group / bk : stages / S);
+    pl.uneven = even == 1 && S > 1;
+    // per channel: one fold per workgroup, so a "group" is at least the workgroup's whole range
+    pl.gstages = (int)(grouped ? group / bk : (stages + S - 1) / S);
     pl.zone_bytes = pl.S > 1 ? (size_t)zone(pl.S) : 0;
     if (tiles * pl.S > 0x7fffffff) pl.ok = false;
     return pl;
@@ -574,6 +581,9 @@ int launch_wq_gemm4(const WqGemm4Plan &plan, const void *x, int act_f16, const v
     p.K = (int)K;
     p.gstages = plan.gstages;
     p.grouped = group_size > 0 && group_size != K;
+    const int stages = (int)((K + (w_bits == 4 ? 127 : 63)) / (w_bits == 4 ? 128 : 64));
+    p.unit_stages = p.grouped ? plan.gstages : 1;
+    p.units = stages / p.unit_stages;
     p.tiles_m = plan.tiles_m;
     p.strips = plan.strips;
     p.S = plan.S;

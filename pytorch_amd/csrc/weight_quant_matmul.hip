@@ -1033,6 +1033,8 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
         // int8 [K, N], more than 32 rows: the same register-expanding kernel
         WqGemm4Plan g8 = make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16);
         if (g8.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2))) {
+            // (a number of stages that has no even split needs no workspace: it is the remainder of a ragged K)
+            if (g8.uneven && room < kWorkspaceZeroBytes) g8 = make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
             const int st = fit_workspace(g8, kWorkspaceZeroBytes, [&]() {
                 return make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
             });

@@ -1562,6 +1562,21 @@ def test_w8a16_ragged_k_without_a_workspace(capi, golden, monkeypatch, M, K, N, 
     bf16_gate(out, torch.from_numpy(want))
 
 
+@pytest.mark.parametrize("M,K,N", [(40, 7232, 1020), (64, 9536, 260), (33, 3008, 252), (70, 4160, 516), (40, 448, 1020), (200, 1096, 508), (48, 4000, 100)])
+def test_w8a16_chunks_of_unequal_length(capi, golden, M, K, N):
+    """int8 [K, N], more than 32 rows: K split into chunks whose numbers of stages differ by one (113, 149, 47, 65, 7, 18 and 63 stages;
+    chunks of one stage leave a set of wavefronts without work), whole and partial last stages; the workspace is used twice."""
+    d = workloads.w8a16_inputs(seed=M + K, M=M, K=K, N=N)
+    _, want = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]), _bits(d["antiquant_offset"]))
+    pitch = (N + 15) // 16 * 16
+    w = torch.full((K, pitch), 77, dtype=torch.int8, device="cuda")[:, :N]
+    w.copy_(d["weight"])
+    args = d["x"].cuda(), w, d["antiquant_scale"].cuda(), d["antiquant_offset"].cuda()
+    first, second = capi.weight_quant_matmul(*args), capi.weight_quant_matmul(*args)
+    bf16_gate(first, torch.from_numpy(want))
+    assert torch.equal(first, second)
+
+
 def test_w4a16_repeated_launches_reuse_workspace(capi, golden):
     """The split-K exchange reuses one workspace and its arrival counters across launches: alternate two
     problems many times and check every result (a stale partial sum or counter would show up here)."""

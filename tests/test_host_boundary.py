@@ -533,7 +533,7 @@ def _weight_quant_status(M, N, K, bits, group, ldx, ldw_k, ldw_n, workspace_byte
                                        p[6] if need else None, need, None)
 
 
-_LAUNCH_ERROR, _WORKSPACE_ERROR = -5, -4
+_LAUNCH_ERROR, _WORKSPACE_ERROR, _ALIGNMENT_ERROR = -5, -4, -3
 
 
 @pytest.mark.parametrize("bits,M,K,N,group", [(8, 82, 664, 13696, 0), (8, 1253, 1152, 704, 0), (8, 228, 4160, 1808, 0), (8, 40, 1000, 1024, 0),
@@ -565,3 +565,20 @@ def test_weight_quant_int8_ragged_k_needs_no_workspace(M, K, N, pad):
     assert _weight_quant_status(200, 1024, 4096, 8, 0, 4096, 1, 4096, 0) == _WORKSPACE_ERROR
     assert _weight_quant_status(48, 1024, 4096, 8, 0, 4096, 1024, 1, 0) == _WORKSPACE_ERROR
     assert _weight_quant_status(48, 1024, 4000, 8, 0, 4000, 1024, 1, 0) == _WORKSPACE_ERROR
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 9536, 1020), (40, 7232, 1020), (64, 9040, 1020), (33, 3008, 252), (200, 1096, 508)])
+def test_weight_quant_int8_splits_any_number_of_stages(M, K, N):
+    """int8 [K, N], a K whose number of 64-row stages few or no splits divide, few tiles: K is split (a launch that splits refuses a misaligned workspace),
+    and without a workspace such a call runs as it did while no split divided its stages."""
+    from pytorch_amd import _capi
+    L, p = _capi.lib(), [i << 32 for i in range(1, 8)]
+    if torch.cuda.is_available():
+        pytest.skip("the addresses are not real")
+    need = L.mi355_weight_quant_matmul_workspace(M, N, K, 8, 0)
+    assert need > 0
+    call = lambda ws, bytes_: L.mi355_weight_quant_matmul(p[0], 0, p[1], 8, p[2], p[3], p[4], p[5], M, N, K, 0, 0, 1, K, N + 4, 1, N, ws, bytes_, None)  # noqa: E731
+    assert call(p[6] + 8, need) == _ALIGNMENT_ERROR and call(p[6], need) == _LAUNCH_ERROR
+    stages = (K + 63) // 64
+    if K % 32 or all(stages % s for s in range(2, 9)):
+        assert call(None, 0) == _LAUNCH_ERROR
