@@ -699,7 +699,10 @@ WqKmPlan make_kmajor_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, i
     if ((uint64_t)S * (uint64_t)M * (uint64_t)N * 4 >= (1ull << 32)) S = 1;
     if (S > 1 && (size_t)pl.tiles * pl.mchunks * sizeof(uint32_t) > kWorkspaceCounterBytes) S = 1;
     while (S > 1 && kWorkspaceZeroBytes + (uint64_t)S * (uint64_t)M * (uint64_t)N * 4 > room) S--;
-    if (wq_kmajor_decode_shape(M, N, K, group_size)) S = 1;   // the decode kernel splits K inside its workgroups
+    // The decode kernel splits K inside its workgroups.  Operands that it refuses for their alignment run here: unsplit where the output
+    // is wide and K short, but a narrow output is a handful of tiles (16x8192x1024: eight, 31.7 us unsplit, 11.1 split) and a long K many
+    // steps on each (5x9216x4096: 36.0 and 15.1 us), so those keep their split and the workspace for it.
+    if (N >= 2048 && wq_kmajor_decode_shape(M, N, K, group_size) && M <= 32 && pl.n_units <= (M <= 16 ? 64 : 32)) S = 1;
     pl.S = S;
     pl.partial_bytes = S > 1 ? (size_t)S * M * N * sizeof(float) : 0;
     pl.counter_bytes = S > 1 ? kWorkspaceZeroBytes : 0;
@@ -977,7 +980,8 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             return launch_wq_gemm(gk, x_bf16, f16 ? 1 : 0, w, 8, scale_bf16, offset_bf16, bias, out_bf16, M, N, K, ldx, ldw_n, ldo,
                                   workspace, stream);
         }
-        WqKmPlan km = make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
+        // (where the decode kernel refused the operands, a caller that brought no workspace is not refused: K is then not split)
+        WqKmPlan km = make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, wq_kmajor_decode_shape(M, N, K, group_size) ? room : ~(size_t)0);
         const bool params_ok = aligned(scale_bf16, 2) && (!offset_bf16 || aligned(offset_bf16, 2));
         if (km.fast && params_ok) {
             const int st = fit_workspace(km, km.counter_bytes + km.partial_bytes, [&]() { return make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, room); });

@@ -763,6 +763,25 @@ def test_w8a16_kmajor_decode_kernel(capi, golden, M, K, N, f16):
     bf16_gate(ref, tiled.float().cpu(), floor=ref.numel() < 8192)
 
 
+@pytest.mark.parametrize("M,K,N", [(16, 8192, 260), (1, 4096, 256), (32, 5120, 516), (5, 9216, 2052)])
+def test_w8a16_decode_shapes_with_scales_off_a_boundary(capi, golden, M, K, N):
+    """int8 weight stored [N, K], few rows, scales that start off an 8-byte boundary: the decode kernel refuses them, and the streaming
+    kernel runs with K split over workgroups; with a workspace of the size the query asks for, twice, and without one."""
+    d = workloads.w8a16_inputs(seed=M + K + N, M=M, K=K, N=N, weight_nk=True)
+    _, want = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]), _bits(d["antiquant_offset"]))
+    scale = torch.empty(N + 1, dtype=d["antiquant_scale"].dtype, device="cuda")[1:]
+    scale.copy_(d["antiquant_scale"])
+    args = d["x"].cuda(), d["weight"].cuda(), scale, d["antiquant_offset"].cuda()
+    first, second = capi.weight_quant_matmul(*args), capi.weight_quant_matmul(*args)
+    bf16_gate(first, torch.from_numpy(want), floor=first.numel() < 8192)
+    assert torch.equal(first, second)
+    x, w, sc, of = args
+    unsplit = torch.empty_like(first)
+    assert capi.lib().mi355_weight_quant_matmul(x.data_ptr(), 0, w.data_ptr(), 8, sc.data_ptr(), of.data_ptr(), None, unsplit.data_ptr(), M, N, K, 0, 0, 1,
+                                                K, 1, K, N, None, 0, torch.cuda.current_stream().cuda_stream) == 0
+    bf16_gate(unsplit, torch.from_numpy(want), floor=first.numel() < 8192)
+
+
 @pytest.mark.parametrize("M,K,N", [(5, 256, 130), (5, 256, 132), (32, 512, 6), (3, 128, 1)])
 def test_w8a16_kmajor_ragged_columns(capi, golden, M, K, N):
     """int8 weight stored [N, K] with N not a multiple of 4 (or of 8): the K-major streaming kernel stores quads of

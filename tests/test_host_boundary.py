@@ -582,3 +582,17 @@ def test_weight_quant_int8_splits_any_number_of_stages(M, K, N):
     stages = (K + 63) // 64
     if K % 32 or all(stages % s for s in range(2, 9)):
         assert call(None, 0) == _LAUNCH_ERROR
+
+
+@pytest.mark.parametrize("M,K,N", [(16, 8192, 1024), (1, 4096, 256), (32, 5120, 1028), (5, 9216, 4096), (30, 6144, 2048)])
+def test_weight_quant_int8_decode_shapes_keep_their_split(pa, M, K, N):
+    """int8 [N, K], few rows, narrow outputs or a long K: scales that the decode kernel refuses for their alignment run on the streaming
+    kernel, which then still splits K (a launch that splits refuses a misaligned workspace); without a workspace it runs unsplit."""
+    from pytorch_amd import _capi
+    if torch.cuda.is_available():
+        pytest.skip("the addresses are not real")
+    L, p = _capi.lib(), [i << 32 for i in range(1, 8)]
+    need = L.mi355_weight_quant_matmul_workspace(M, N, K, 8, 0)
+    call = lambda scale, ws, bytes_: L.mi355_weight_quant_matmul(p[0], 0, p[1], 8, scale, p[3], p[4], p[5], M, N, K, 0, 0, 1, K, 1, K, N, ws, bytes_, None)  # noqa: E731
+    assert need > 0 and call(p[2] + 2, p[6] + 8, need) == _ALIGNMENT_ERROR
+    assert [call(p[2] + 2, p[6], need), call(p[2] + 2, None, 0), call(p[2], p[6] + 8, need), call(p[2], None, 0)] == [_LAUNCH_ERROR] * 4
