@@ -300,9 +300,11 @@ int launch_qmm_decode(const QmmDecodeArgs &p, hipStream_t s)
     if (!qmm_decode_shape(p.M, p.N, p.K)) return MI355_ERR_UNSUPPORTED;
     if ((p.lda & 15) != 0 || (p.ldbt & 15) != 0 || !aligned(p.a, 16) || !aligned(p.bt, 16) || p.ldbt < p.K)
         return MI355_ERR_UNSUPPORTED;
-    // dequantisation parameters and results in pieces of four columns
-    if ((p.ldc & 3) != 0 || !aligned(p.out, p.out_i32 ? 16 : 8) || !aligned(p.qparam ? static_cast<const void *>(p.qparam) : static_cast<const void *>(p.scale), 16) ||
-        (p.bias && !aligned(p.bias, p.bias_kind == MI355_BIAS_BF16 ? 8 : 16)))
+    // Results go in pieces of four columns.  Parameters come in such pieces too, by buffer loads, which need whole dwords and no more: a
+    // slice of a longer scale vector may start anywhere (the tiled kernel, unsplit where this kernel's shapes have no scratch, takes
+    // 46.7 us for 32x14336x4096, this one 15.1).
+    if ((p.ldc & 3) != 0 || !aligned(p.out, p.out_i32 ? 16 : 8) || !aligned(p.qparam ? static_cast<const void *>(p.qparam) : static_cast<const void *>(p.scale), 4) ||
+        (p.bias && !aligned(p.bias, 4)))
         return MI355_ERR_UNSUPPORTED;
     // 32-bit buffer offsets over the whole weight and all activation rows
     if ((uint64_t)(p.N + 16) * (uint64_t)p.ldbt + (uint64_t)p.K >= (1ull << 31) || (uint64_t)p.M * (uint64_t)p.lda + (uint64_t)p.K >= (1ull << 31))

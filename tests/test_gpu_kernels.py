@@ -560,6 +560,34 @@ def test_quant_matmul_decode_kernel(capi, golden, M, K, N):
         capi.set_tuning("MI355_QMM_DECODE_OFF", 0)
 
 
+@pytest.mark.parametrize("shift", [1, 2, 3])
+@pytest.mark.parametrize("M,K,N", [(16, 4096, 2048), (3, 1152, 4100), (32, 14336, 2052), (40, 9344, 3072)])
+def test_quant_matmul_decode_kernel_with_parameters_off_a_boundary(capi, golden, M, K, N, shift):
+    """Scale, bias and packed parameters cut out of longer vectors, 1 to 3 elements past a 16-byte boundary (the decode kernel loads four
+    columns' worth at a time, by whole dwords: a bf16 bias an odd number of elements off goes elsewhere); outputs bit-identical to the oracle."""
+    d = workloads.quant_matmul_inputs(seed=M + K + N, M=M, K=K, N=N, weight_nk=True, bias=True)
+    g = torch.Generator().manual_seed(M + N)
+    bias_i32, bias_f32 = torch.randint(-(1 << 20), 1 << 20, (N,), generator=g, dtype=torch.int32), torch.randn(N, generator=g)
+    x1, x2, ps = d["x1"].cuda(), d["x2"].cuda(), d["pertoken_scale"].cuda()
+
+    def off(t):
+        out = torch.full((N + shift + 4,), 7, dtype=t.dtype, device="cuda")[shift:shift + N]
+        return out.copy_(t)
+
+    sc = off(d["scale"])
+    acc = golden.int8_gemm(d["x1"].numpy(), d["x2"].numpy())
+    for bias, dt, name in [(d["bias"], torch.bfloat16, "bf16"), (bias_i32, torch.bfloat16, "bf16"), (bias_f32, torch.float16, "fp16"), (None, torch.bfloat16, "bf16")]:
+        out = capi.quant_matmul(x1, x2, sc, ps, None if bias is None else off(bias), out_dtype=dt)
+        bias_np = None if bias is None else (_bits(bias) if bias.dtype == torch.bfloat16 else bias.numpy())
+        want = golden.quant_matmul_epilogue_ex(acc, d["scale"].numpy(), d["pertoken_scale"].numpy(), bias_np, out=name)
+        assert np.array_equal(out.cpu().view(torch.int16).numpy().view(np.uint16), want), (name, None if bias is None else bias.dtype)
+    got = capi.quant_matmul_qparam(x1, x2, off(capi.trans_quant_param(d["scale"].cuda())), off(bias_i32), out_dtype=torch.float16)
+    want = golden.quant_matmul_epilogue_ex(acc, d["scale"].numpy(), None, bias_i32.numpy(), out="fp16")
+    assert np.array_equal(got.cpu().view(torch.int16).numpy().view(np.uint16), want)
+    got = capi.quant_matmul(x1, x2, None, None, off(bias_i32), out_dtype=torch.int32)
+    assert np.array_equal(got.cpu().numpy(), (acc.astype(np.int64) + bias_i32.numpy()).astype(np.int32))
+
+
 @pytest.mark.parametrize("weight_nk", [True, False])
 @pytest.mark.parametrize("M,K,N", [(5, 1040, 2052), (20, 2160, 2048), (40, 1936, 2064),       # decode kernel, partial last step
                                    (64, 144, 260), (100, 4112, 520), (128, 1264, 2000),         # streaming loop, small tiles, split K
