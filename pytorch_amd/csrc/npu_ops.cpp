@@ -258,7 +258,20 @@ void check_workspace(const Tensor &ws, void *stream, const char *when)
                 "; the outputs of that launch hold NaN, the workspace has been cleared and is usable again)");
 }
 
-Tensor zeroed_workspace(const Tensor &like, size_t bytes)
+// A new buffer with the zero area cleared, which is all that a kernel finds in it.
+Tensor new_workspace(const Tensor &like, int64_t bytes)
+{
+    Tensor ws = at::empty({bytes}, like.options().dtype(at::kChar));
+    ws.narrow(0, 0, std::min<int64_t>(bytes, (int64_t)MI355_WORKSPACE_ZERO_BYTES)).zero_();
+    return ws;
+}
+
+// `large_for_call`: the request holds a copy of operands of any size, so a large one is given back when the call returns instead of
+// staying with the stream for good (and counting twice once it is outgrown).  The fill of its zero area adds 5 us
+// (16x9999x8192 59.6 -> 64.2 us, 1784x9313x8192 148.2 -> 153.3).
+constexpr size_t kKeptWorkspaceBytes = (size_t)MI355_WORKSPACE_ZERO_BYTES + ((size_t)64 << 20);
+
+Tensor zeroed_workspace(const Tensor &like, size_t bytes, bool large_for_call = false)
 {
     WorkspaceCache &wc = workspace_cache();
     std::lock_guard<std::mutex> lock(wc.mu);
@@ -273,12 +286,13 @@ Tensor zeroed_workspace(const Tensor &like, size_t bytes)
         if (eager != wc.eager.end() && eager->second.defined() && (size_t)eager->second.numel() >= bytes) return eager->second;
         WorkspaceCache::Captured &c = wc.captured[key];
         if (!c.ws.defined() || c.id != capture_id || (size_t)c.ws.numel() < bytes) {
-            c.ws = at::zeros({want}, like.options().dtype(at::kChar));      // the fill is recorded into this capture
+            c.ws = new_workspace(like, want);                               // the fill is recorded into this capture
             c.id = capture_id;
         }
         return c.ws;
     }
     wc.captured.erase(key);
+    if (large_for_call && bytes > kKeptWorkspaceBytes) return new_workspace(like, want);
     Tensor &ws = wc.eager[key];
     if (!ws.defined() || (size_t)ws.numel() < bytes) {
         if (ws.defined()) {
@@ -512,7 +526,7 @@ Tensor quant_matmul_hip(const Tensor &x1, const Tensor &x2, const Tensor &scale,
         if (w.stride(0) == 1 && !rows_aligned(w, w.stride(1))) w = aligned_rows(w.t(), p.K).t();
         const int64_t m = a.size(0);
         const size_t ws_bytes = mi355_quant_matmul_workspace(m, p.N, p.K, w.stride(0), w.stride(1));
-        const Tensor ws = ws_bytes ? zeroed_workspace(xa, ws_bytes) : Tensor();
+        const Tensor ws = ws_bytes ? zeroed_workspace(xa, ws_bytes, (p.K & 15) != 0) : Tensor();   // such a K: padded copies of the operands
         void *o = static_cast<char *>(out.data_ptr()) + row0 * p.N * (int64_t)out.element_size();
         const int st = qp.defined()
             ? mi355_quant_matmul_qparam(static_cast<int8_t *>(a.data_ptr()), static_cast<int8_t *>(w.data_ptr()), static_cast<uint64_t *>(qp.data_ptr()),

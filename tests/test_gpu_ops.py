@@ -618,6 +618,35 @@ def test_workspace_outlives_growth_after_capture(pa):
     torch.cuda.synchronize()
 
 
+def test_large_padded_operands_are_not_kept(pa):
+    """A K that is not a multiple of 16 copies the weight into padded rows.  Where that takes 80 MB the stream does not keep them when
+    the call returns, and a captured call, which has a workspace of its own, replays to the same bits."""
+    g = torch.Generator().manual_seed(29)
+    M, K, N = 40, 4001, 20000
+    x = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8).cuda()
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).cuda()
+    sc, ps = (torch.rand(N, generator=g) * 1e-2).cuda(), (torch.rand(M, generator=g) * 1e-2).cuda()
+    op = lambda: pa.npu_quant_matmul(x, w.t(), sc, pertoken_scale=ps, output_dtype=torch.bfloat16)
+    acc = (x.cpu().double() @ w.cpu().double().t()).float()                # below 2^31: exact in float64
+    want = ((acc * ps.cpu()[:, None]) * sc.cpu()).bfloat16()
+    stream = torch.cuda.Stream()                       # fresh stream: no workspace is cached for it
+    with torch.cuda.stream(stream):
+        before = torch.cuda.memory_allocated()
+        for it in range(3):
+            assert torch.equal(op().cpu(), want), it
+        assert torch.cuda.memory_allocated() - before < N * K // 2
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = op()
+        for it in range(3):
+            out.zero_()
+            graph.replay()
+            stream.synchronize()
+            assert torch.equal(out.cpu(), want), f"replay {it}"
+            assert torch.equal(op().cpu(), want)
+    torch.cuda.synchronize()
+
+
 def test_split_k_graph_survives_workspace_growth(pa):
     """The same with a first product whose graph uses the workspace: 258 columns are not whole pieces of four, so the tiled kernel
     runs with K split over workgroups that meet at counters there."""
