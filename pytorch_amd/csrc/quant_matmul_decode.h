@@ -24,8 +24,11 @@ struct QmmDecodeArgs {
     int scale_len;             // 1 or N
 };
 
-// The part of the decision that depends on the shape alone (the planner uses it: the kernel needs no workspace).
+// The shapes that the kernel takes (it needs no workspace).
 __attribute__((visibility("hidden"))) bool qmm_decode_shape(int64_t M, int64_t N, int64_t K);
+
+// Estimated time in us of such a shape where K takes several passes; 0 where one is enough, which is always the faster form.
+__attribute__((visibility("hidden"))) double qmm_decode_passes_us(int64_t M, int64_t N, int64_t K);
 
 // MI355_ERR_UNSUPPORTED when pointers or pitches do not fit the kernel: the caller then takes the tiled kernel.
 __attribute__((visibility("hidden"))) int launch_qmm_decode(const QmmDecodeArgs &p, hipStream_t stream);

@@ -266,7 +266,7 @@ int launch(const QmmDecodeArgs &p, hipStream_t s)
     return check_launch();
 }
 
-// Tiles of 16 rows per workgroup (1, 2 or 4), 0: the tiled kernel is the faster one.
+// Tiles of 16 rows per workgroup (1, 2 or 4), 0: not a shape for this kernel.
 int row_tiles(int64_t M, int64_t N, int64_t K)
 {
     // (parameters and results go in pieces of four columns; any other width takes the tiled kernel and its split of K)
@@ -279,8 +279,7 @@ int row_tiles(int64_t M, int64_t N, int64_t K)
         const int64_t chunks = (M + 16 * mt - 1) / (16 * mt);
         if (chunks > 1 && (strips * chunks > kMaxWorkgroups || strips * chunks * (16 + 16 * mt) * K > kMaxChunkBytes)) continue;
         // The activations of a wavefront's eighth of K stay in registers: up to 16 steps with one tile of 16 rows, 8 with two,
-        // 4 with four; a longer K takes passes.  A pass of four tiles reads 64 x 4096 bytes per workgroup from the L2 (5 us when
-        // every CU does), so there are at most two or three of them (14336x4096 at 64 rows, four passes: 24 us; tiled: 18.7).
+        // 4 with four; a longer K takes passes.
         if (steps > 16 / mt && lds_need(mt, N, true) > kMaxLds) continue;
         if (mt == 4 && steps > 4 && !(steps <= 8 && N <= 4096) && !(steps <= 12 && N <= 3072)) continue;
         // With four tiles and more than 1024 strips the tiled kernel's streaming loop is faster (measured at K = 4096:
@@ -294,6 +293,20 @@ int row_tiles(int64_t M, int64_t N, int64_t K)
 } // namespace
 
 bool qmm_decode_shape(int64_t M, int64_t N, int64_t K) { return knob(kKnobQmmDecodeOff) != 1 && row_tiles(M, N, K) > 0; }
+
+// Every pass exposes a round trip for its activations and fills its weight ring anew.  Fitted to 680 shapes with several passes, M = 1
+// .. 256, K = 8192 .. 28160, N = 256 .. 28672, 3.3 % off on average; passes taken wherever they fit were 7 % behind the better of the
+// two kernels on average and 46 % at worst (32x16640x4480: 28.6 us, tiled 20.5).  Four tiles never pay in passes: 109 of 110 shapes
+// of two passes and all of three were slower, by 8 and 18 % on average.
+double qmm_decode_passes_us(int64_t M, int64_t N, int64_t K)
+{
+    const int mt = row_tiles(M, N, K);
+    const int64_t steps = ((K + kStep - 1) / kStep + 7) / 8, per_pass = mt > 0 ? 16 / mt : steps;
+    if (steps <= per_pass) return 0.0;
+    if (mt == 4) return 1e30;
+    const int64_t passes = (steps + per_pass - 1) / per_pass, strips = ((N + 15) / 16 + kMaxWorkgroups - 1) / kMaxWorkgroups;
+    return 1.2 + 3.0 * (double)passes + (double)strips * (1.6 + 0.31 * (double)steps) + (double)N * (double)K / 17.9e6;
+}
 
 int launch_qmm_decode(const QmmDecodeArgs &p, hipStream_t s)
 {

@@ -511,7 +511,7 @@ QMM_DECODE_CASES = [(1, 4096, 4096), (7, 1024, 2048), (16, 1152, 2056), (5, 1433
 
 
 @pytest.mark.parametrize("M,K,N", QMM_DECODE_CASES)
-def test_quant_matmul_decode_kernel(capi, golden, M, K, N):
+def test_quant_matmul_decode_kernel(capi, golden, monkeypatch, M, K, N):
     """Few rows and a weight stored [N, K]: the kernel that splits K over the wavefronts of a workgroup and walks
     over strips of 16 columns (one, two and four tiles of 16 rows; 1 to 16 steps per wavefront, even and uneven; strips
     that end past N; more strips than workgroups).  Outputs bit-identical to the oracle for every bias kind, both output
@@ -522,7 +522,7 @@ def test_quant_matmul_decode_kernel(capi, golden, M, K, N):
     bias_f32 = torch.randn(N, generator=g)
     x1, x2, sc, ps = d["x1"].cuda(), d["x2"].cuda(), d["scale"].cuda(), d["pertoken_scale"].cuda()
     if M <= 64 and N >= 2048:
-        assert capi.lib().mi355_quant_matmul_workspace(M, N, K, 1, K) == 0      # no split of K over workgroups
+        monkeypatch.setattr(capi, "_wq_workspace", lambda device, nbytes: None)      # no split of K over workgroups
     acc = golden.int8_gemm(d["x1"].numpy(), d["x2"].numpy())
     cases = [(d["bias"], torch.bfloat16, "bf16", True), (bias_i32, torch.bfloat16, "bf16", True), (bias_f32, torch.float16, "fp16", True),
              (None, torch.float16, "fp16", True), (None, torch.bfloat16, "bf16", False), (bias_f32, torch.bfloat16, "bf16", False)]
@@ -552,6 +552,7 @@ def test_quant_matmul_decode_kernel(capi, golden, M, K, N):
     assert np.array_equal(capi.quant_matmul(x1, x2, None, out_dtype=torch.int32).cpu().numpy(), acc)
     got = capi.quant_matmul(x1, x2, sc, ps, bias_i32.cuda(), out_dtype=torch.int32)
     assert np.array_equal(got.cpu().numpy(), (acc.astype(np.int64) + bias_i32.numpy().astype(np.int64)).astype(np.int32))
+    monkeypatch.undo()
     capi.set_tuning("MI355_QMM_DECODE_OFF", 1)
     try:
         assert torch.equal(capi.quant_matmul(x1, x2, sc, ps, d["bias"].cuda()), ref)
@@ -561,7 +562,7 @@ def test_quant_matmul_decode_kernel(capi, golden, M, K, N):
 
 
 @pytest.mark.parametrize("shift", [1, 2, 3])
-@pytest.mark.parametrize("M,K,N", [(16, 4096, 2048), (3, 1152, 4100), (32, 14336, 2052), (40, 9344, 3072)])
+@pytest.mark.parametrize("M,K,N", [(16, 4096, 2048), (3, 1152, 4100), (32, 14336, 2052), (40, 3200, 3072)])
 def test_quant_matmul_decode_kernel_with_parameters_off_a_boundary(capi, golden, M, K, N, shift):
     """Scale, bias and packed parameters cut out of longer vectors, 1 to 3 elements past a 16-byte boundary (the decode kernel loads four
     columns' worth at a time, by whole dwords: a bf16 bias an odd number of elements off goes elsewhere); outputs bit-identical to the oracle."""
@@ -1674,3 +1675,37 @@ def test_weight_quant_exchange_timeout_is_reported(capi, golden, M):
     assert int(ws[:capi.ZERO_AREA_BYTES].count_nonzero()) == 0
     again = capi.weight_quant_matmul(x, w, sc, of, group_size=128)
     assert torch.equal(again, good)
+
+
+def _leaves_sums_in_the_workspace(capi, monkeypatch, call):
+    """The call's result and whether it exchanged partial sums through the workspace (K split over workgroups) or not."""
+    made = []
+
+    def workspace(device, nbytes):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        ws[capi.ZERO_AREA_BYTES:] = 0x55
+        made.append(ws)
+        return ws
+
+    monkeypatch.setattr(capi, "_wq_workspace", workspace)
+    out = call()
+    return out, any(bool((ws[capi.ZERO_AREA_BYTES:] != 0x55).any()) for ws in made)
+
+
+@pytest.mark.parametrize("M,K,N,split", [(32, 16640, 4480, True), (6, 21248, 4224, True), (40, 10240, 2048, True), (20, 10240, 1552, False),
+                                         (60, 4096, 2048, False)])
+def test_quant_matmul_passes_over_a_long_k(capi, monkeypatch, M, K, N, split):
+    """Few rows and a K that the decode kernel walks over in passes: it runs where that is the faster form, K split over workgroups
+    elsewhere, and without a workspace the decode kernel takes all of them; bit-identical to exact integer sums."""
+    g = torch.Generator().manual_seed(M + K + N)
+    x1 = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8)
+    x2 = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    want = (x1.double() @ x2.double().t()).to(torch.int32)
+    a, w = x1.cuda(), x2.cuda().t()
+    out, used = _leaves_sums_in_the_workspace(capi, monkeypatch, lambda: capi.quant_matmul(a, w, None, out_dtype=torch.int32))
+    assert torch.equal(out.cpu(), want) and used is split
+    if N >= 2048:
+        bare = torch.empty_like(out)
+        assert capi.lib().mi355_quant_matmul(a.data_ptr(), w.data_ptr(), None, None, 0, None, 0, bare.data_ptr(), 1, M, N, K, K, 1, K, N, None, 0,
+                                             torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(bare, out)

@@ -596,3 +596,17 @@ def test_weight_quant_int8_decode_shapes_keep_their_split(pa, M, K, N):
     call = lambda scale, ws, bytes_: L.mi355_weight_quant_matmul(p[0], 0, p[1], 8, scale, p[3], p[4], p[5], M, N, K, 0, 0, 1, K, 1, K, N, ws, bytes_, None)  # noqa: E731
     assert need > 0 and call(p[2] + 2, p[6] + 8, need) == _ALIGNMENT_ERROR
     assert [call(p[2] + 2, p[6], need), call(p[2] + 2, None, 0), call(p[2], p[6] + 8, need), call(p[2], None, 0)] == [_LAUNCH_ERROR] * 4
+
+
+@pytest.mark.parametrize("M,K,N", [(32, 16640, 4480), (6, 21248, 4224), (3, 18432, 10688), (63, 6144, 2752), (40, 10240, 2048)])
+def test_quant_matmul_long_k_keeps_its_split(M, K, N):
+    """Shapes whose K takes the decode kernel several passes, where the tiled kernel with K split is the faster one: the query asks for
+    the workspace of the split, and a call without one runs all the same, as it has while the decode kernel took them."""
+    from pytorch_amd import _capi
+    if torch.cuda.is_available():
+        pytest.skip("the addresses are not real")
+    L, p = _capi.lib(), [i << 32 for i in range(1, 6)]
+    need = L.mi355_quant_matmul_workspace(M, N, K, 1, K)
+    call = lambda ws, bytes_: L.mi355_quant_matmul(p[0], p[1], None, p[2], N, None, 0, p[3], 0, M, N, K, K, 1, K, N, ws, bytes_, None)  # noqa: E731
+    assert need > 0
+    assert [call(p[4], need), call(None, 0), call(p[4], need - 1)] == [_LAUNCH_ERROR] * 3
