@@ -252,7 +252,7 @@ int launch(const WqKmDecodeArgs &p, hipStream_t s)
     return check_launch();
 }
 
-// Tiles of 16 rows per workgroup (1, 2 or 4), 0: another kernel is the faster one.
+// Tiles of 16 rows per workgroup (1, 2 or 4), 0: not a shape for this kernel.
 int row_tiles(int64_t M, int64_t N, int64_t K)
 {
     if (M < 1 || M > 128 || K % 16 != 0 || K < 8 * kStep || N % 4 != 0) return 0;
@@ -278,7 +278,7 @@ int launch_act(const WqKmDecodeArgs &p, hipStream_t s)
     const int mt = row_tiles(p.M, p.N, p.K);
     if (mt == 1) return ns <= 4 ? launch<1, 4, 4, ACT, false>(p, s) : ns <= 8 ? launch<1, 8, 4, ACT, false>(p, s) : launch<1, 8, 4, ACT, true>(p, s);
     if (mt == 2) return ns <= 4 ? launch<2, 4, 4, ACT, false>(p, s) : launch<2, 4, 4, ACT, true>(p, s);
-    return ns <= 2 ? launch<4, 2, 2, ACT, false>(p, s) : launch<4, 2, 2, ACT, true>(p, s);
+    return launch<4, 2, 2, ACT, false>(p, s);              // (the sums of four tiles do not fit the LDS between passes)
 }
 
 } // namespace
@@ -288,6 +288,20 @@ bool wq_kmajor_decode_shape(int64_t M, int64_t N, int64_t K, int64_t group_size)
     if (knob(kKnobWqDecodeOff) == 1 || knob(kKnobWqSplit) != 0) return false;
     if (group_size > 0 && group_size != K) return false;                  // one scale per column
     return row_tiles(M, N, K) > 0;
+}
+
+// Fitted to 912 shapes of at most 32 rows with several passes, K = 4352 .. 28416, N = 256 .. 16384, 5 % off on average.  Passes taken
+// wherever they fit were 14 % behind the better kernel on average and 89 % at worst (5x25600x768: 24.4 us, K split over
+// workgroups 14.9).  From 33 rows up the other kernel is the tiled one, which two passes (two tiles: three) beat by 17 % on average of 70
+// shapes and more lose to by 5 % (12 shapes).
+double wq_kmajor_decode_passes_us(int64_t M, int64_t N, int64_t K)
+{
+    const int mt = row_tiles(M, N, K);
+    const int64_t steps = ((K + kStep - 1) / kStep + 7) / 8, per_pass = mt > 0 ? 8 / mt : steps;
+    const int64_t passes = (steps + per_pass - 1) / per_pass, strips = ((N + 15) / 16 + kMaxWorkgroups - 1) / kMaxWorkgroups;
+    if (passes <= 1) return 0.0;
+    if (M > 32) return passes <= 1 + mt ? 0.0 : 1e30;
+    return 0.6 + 3.8 * (double)passes + (double)strips * (2.4 + 0.22 * (double)steps) + (double)N * (double)K / 18e6;
 }
 
 int launch_wq_kmajor_decode(const WqKmDecodeArgs &p, int act_f16, hipStream_t s)

@@ -671,6 +671,7 @@ struct WqKmPlan {
     int mt, mchunks, tiles, S, unit_steps, n_units;
     bool grouped;
     size_t partial_bytes, counter_bytes, lds_bytes;
+    double us;                             // estimated time, at most 32 rows
 };
 
 WqKmPlan make_kmajor_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw_n, int64_t ldx, const void *x,
@@ -707,6 +708,10 @@ WqKmPlan make_kmajor_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, i
     pl.partial_bytes = S > 1 ? (size_t)S * M * N * sizeof(float) : 0;
     pl.counter_bytes = S > 1 ? kWorkspaceZeroBytes : 0;
     pl.lds_bytes = 16 + (size_t)2 * 32768 + 8 * 2 * 2048;   // two activation chunks + the turn-around tiles
+    // fitted to the same shapes as the estimate of the decode kernel's passes, 6 % off on average; tiles are dealt to the XCDs in eights
+    const int rounds = ((pl.tiles + 7) / 8 * S * pl.mchunks + 31) / 32;
+    pl.us = 1.3 + rounds * (4.2 + 0.4 * ((pl.n_units * pl.unit_steps + S - 1) / S)) + 0.15 * S + (double)N * (double)K / 14.2e6 +
+            (double)S * (double)M * (double)N / 142e3;
     return pl;
 }
 
@@ -756,6 +761,9 @@ enum { kPreferDecode, kPreferGemm4, kPreferGemm, kPreferStream };
 // gathered into row-major [G, N]) for the register-expanding GEMM.  Layout of the workspace: the zero area, the weight
 // ([K, repack_pitch_words(N)] words), scales, offsets.
 constexpr int64_t kRepackRows = 256;
+// A decode kernel that needs several passes over K runs unless its estimate is this much above the other kernel's: about the error of
+// both.  Over 912 shapes of int8 [N, K] 0.8 % behind the better of the two kernels on average.
+constexpr double kPassesMargin = 1.05;
 int64_t repack_pitch_words(int64_t N) { return (N / 8 + 3) / 4 * 4; }
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 size_t repack_weight_bytes(int64_t N, int64_t K) { return align256((size_t)K * (size_t)repack_pitch_words(N) * 4); }
@@ -879,6 +887,7 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
     // multiple of 128 also runs without one (a step of 32 is enough where the streaming kernel reads the weight).
     const bool n_major = w_bits == 4 || (ldw_n == 1 && ldw_k >= N);
     const size_t room = workspace ? workspace_bytes : 0;
+    const auto workspace_holds = [&](size_t bytes) { return workspace && workspace_bytes >= bytes && aligned(workspace, 16); };
     const auto must_have = [&]() {
         if (room >= mi355_weight_quant_matmul_workspace(M, N, K, w_bits, group_size)) return false;
         if (w_bits != 8 || group != K || K % 128 == 0) return true;
@@ -942,7 +951,19 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
     if (!params_rowmajor) return generic();
     if (w_bits == 8 && ldw_k == 1 && ldw_n != 1) {
         // K-major: the transposed view of an [N, K] weight
-        if (wq_kmajor_decode_shape(M, N, K, group_size)) {
+        const bool out_ok = aligned(out_bf16, 2) && (!bias || aligned(bias, 2));
+        bool decode = wq_kmajor_decode_shape(M, N, K, group_size);
+        if (const double passes_us = decode ? wq_kmajor_decode_passes_us(M, N, K) : 0.0; passes_us > 0.0) {
+            // K takes several passes there: the kernel with the smaller estimate runs, or this one where there is no workspace for it
+            if (M > 32) {
+                const WqKmGemmPlan other = make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
+                decode = !other.ok || !out_ok || (other.S > 1 && !workspace_holds(other.counter_bytes + other.partial_bytes));
+            } else {
+                const WqKmPlan other = make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
+                decode = !other.fast || passes_us < kPassesMargin * other.us || (other.S > 1 && !workspace_holds(other.counter_bytes + other.partial_bytes));
+            }
+        }
+        if (decode) {
             // few rows, one scale per column: the barrier-free kernel that splits K inside the workgroup
             WqKmDecodeArgs d;
             d.x = static_cast<const uint16_t *>(x_bf16);
@@ -960,7 +981,6 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             const int st = launch_wq_kmajor_decode(d, f16 ? 1 : 0, s);
             if (st != MI355_ERR_UNSUPPORTED) return st;
         }
-        const bool out_ok = aligned(out_bf16, 2) && (!bias || aligned(bias, 2));
         WqKmGemmPlan kg = make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
         if (kg.ok && out_ok) {
             const int st = fit_workspace(kg, kg.counter_bytes + kg.partial_bytes, [&]() {
@@ -1051,7 +1071,6 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
     // A kernel that the workspace query did not plan for (it only runs because a pointer kept the preferred one away) goes
     // on to the next one when its own request is not met; the preferred one reports the missing workspace.
     const int preferred = n_major ? preferred_n_major_kernel(M, N, K, w_bits, group_size, ldw_k, ldx) : kPreferStream;
-    const auto workspace_holds = [&](size_t bytes) { return workspace && workspace_bytes >= bytes && aligned(workspace, 16); };
     WqGemmPlan gp = make_wq_gemm_plan(M, N, K, w_bits, group_size, n_major ? 1 : 0, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16);
     const bool gemm_runs = gp.ok && aligned(out_bf16, 2) && (!bias || aligned(bias, 2));
     if (gemm_runs && preferred >= kPreferGemm) {

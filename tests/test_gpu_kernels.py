@@ -1709,3 +1709,19 @@ def test_quant_matmul_passes_over_a_long_k(capi, monkeypatch, M, K, N, split):
         assert capi.lib().mi355_quant_matmul(a.data_ptr(), w.data_ptr(), None, None, 0, None, 0, bare.data_ptr(), 1, M, N, K, K, 1, K, N, None, 0,
                                              torch.cuda.current_stream().cuda_stream) == 0
         assert torch.equal(bare, out)
+
+
+@pytest.mark.parametrize("M,K,N,split", [(5, 25600, 768, True), (3, 17408, 320, True), (20, 20480, 1032, True), (57, 17408, 704, True), (12, 9472, 2240, False),
+                                         (16, 10240, 4096, False), (36, 9216, 576, False)])
+def test_w8a16_passes_over_a_long_k(capi, golden, monkeypatch, M, K, N, split):
+    """The same for an int8 weight stored [N, K]."""
+    d = workloads.w8a16_inputs(seed=M + K + N, M=M, K=K, N=N, weight_nk=True)
+    _, want = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]), _bits(d["antiquant_offset"]))
+    x, w, sc, of = (d[k].cuda() for k in ("x", "weight", "antiquant_scale", "antiquant_offset"))
+    out, used = _leaves_sums_in_the_workspace(capi, monkeypatch, lambda: capi.weight_quant_matmul(x, w, sc, of))
+    bf16_gate(out, torch.from_numpy(want), floor=out.numel() < 8192)
+    assert used is split
+    bare = torch.empty_like(out)
+    assert capi.lib().mi355_weight_quant_matmul(x.data_ptr(), 0, w.data_ptr(), 8, sc.data_ptr(), of.data_ptr(), None, bare.data_ptr(), M, N, K, 0, 0, 1,
+                                                K, 1, K, N, None, 0, torch.cuda.current_stream().cuda_stream) == 0
+    bf16_gate(bare, torch.from_numpy(want), floor=out.numel() < 8192)
