@@ -17,6 +17,7 @@ struct WqKpackedPlan {
     int unit_sub;            // sub-steps of 128 k per scale group (grouped only)
     bool grouped;
     size_t lds_bytes, counter_bytes, partial_bytes;   // workspace when S > 1: [arrival counters | partial sums]
+    double us;               // estimated time, at most 32 rows
 };
 
 // `ldw_n`: int32 words between the rows of two consecutive output columns

@@ -19,8 +19,11 @@ struct WqKpDecodeArgs {
     int M, N, K;
 };
 
-// The part of the decision that depends on the shape alone (the kernel needs no workspace).
+// The shapes that the kernel takes (it needs no workspace).
 __attribute__((visibility("hidden"))) bool wq_kpacked_decode_shape(int64_t M, int64_t N, int64_t K, int64_t group_size);
+
+// Estimated time in us of such a shape where K takes several passes; 0 where the kernel is the faster one whatever the other's plan.
+__attribute__((visibility("hidden"))) double wq_kpacked_decode_passes_us(int64_t M, int64_t N, int64_t K);
 
 // MI355_ERR_UNSUPPORTED when pointers or pitches do not fit the kernel: the caller then takes the other K-packed kernel.
 __attribute__((visibility("hidden"))) int launch_wq_kpacked_decode(const WqKpDecodeArgs &p, int act_f16, hipStream_t stream);

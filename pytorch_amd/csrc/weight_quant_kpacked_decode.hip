@@ -305,7 +305,7 @@ int launch(const WqKpDecodeArgs &p, hipStream_t s)
     return check_launch();
 }
 
-// Tiles of 16 rows per workgroup (1 or 2), 0: another kernel is the faster one.
+// Tiles of 16 rows per workgroup (1 or 2), 0: not a shape for this kernel.
 int row_tiles(int64_t M, int64_t N, int64_t K)
 {
     if (M < 1 || M > 128 || K % (2 * kStep) != 0 || N % 4 != 0) return 0;
@@ -328,6 +328,7 @@ template <int ACT>
 int launch_act(const WqKpDecodeArgs &p, hipStream_t s)
 {
     const int ns = (p.K / (2 * kStep) + 7) / 8;
+    // (two tiles in passes spill 7 to 9 registers; still 16.5 us for 30x6144x4096, where the other kernel takes 18.9)
     if (row_tiles(p.M, p.N, p.K) == 2) return ns <= 2 ? launch<2, 2, 1, 2, ACT>(p, s) : launch<2, 2, 1, 2, ACT, true>(p, s);
     if (ns > 4) return launch<1, 2, 1, 2, ACT, true>(p, s);               // (four steps per pass spill)
     if (ns > 2) return launch<1, 4, 1, 4, ACT>(p, s);
@@ -343,6 +344,23 @@ bool wq_kpacked_decode_shape(int64_t M, int64_t N, int64_t K, int64_t group_size
 {
     if (knob(kKnobWqDecodeOff) == 1 || knob(kKnobWqSplit) != 0) return false;
     return group_size == 128 && row_tiles(M, N, K) > 0;
+}
+
+// Fitted to 1006 shapes of at most 32 rows with several passes, K = 4352 .. 28672, N = 320 .. 28352, 6 % off on average.  Passes taken
+// wherever they fit were 6 % behind the better kernel on average and 87 % at worst (32x14336x4096: 29.3 us, the other kernel
+// 21.3).  From 33 rows up one tile is the faster form up to the seven passes of K = 28672 and two tiles up to three (four: 11 % slower on
+// average).
+double wq_kpacked_decode_passes_us(int64_t M, int64_t N, int64_t K)
+{
+    const int mt = row_tiles(M, N, K);
+    const int64_t steps = (K / (2 * kStep) + 7) / 8;
+    if (mt == 0 || steps <= 4 / mt) return 0.0;
+    const int64_t passes = (steps + 1) / 2, column_tiles = (N + 15) / 16, strips = (column_tiles + kMaxWorkgroups - 1) / kMaxWorkgroups;
+    if (M > 32) return mt == 1 || passes <= 3 ? 0.0 : 1e30;
+    const int64_t chunks = (M + 16 * mt - 1) / (16 * mt);
+    const double filled = (double)(column_tiles < kMaxWorkgroups ? column_tiles : kMaxWorkgroups) * (double)chunks / kMaxWorkgroups;
+    return 2.4 * (double)chunks + (double)passes * ((mt == 1 ? 1.5 : 4.7) + 0.2 * filled * mt) +
+           (double)strips * (0.6 + (mt == 1 ? 0.55 : 0.46) * (double)steps) + (double)N * (double)K / 52e6;
 }
 
 int launch_wq_kpacked_decode(const WqKpDecodeArgs &p, int act_f16, hipStream_t s)

@@ -762,7 +762,7 @@ enum { kPreferDecode, kPreferGemm4, kPreferGemm, kPreferStream };
 // ([K, repack_pitch_words(N)] words), scales, offsets.
 constexpr int64_t kRepackRows = 256;
 // A decode kernel that needs several passes over K runs unless its estimate is this much above the other kernel's: about the error of
-// both.  Over 912 shapes of int8 [N, K] 0.8 % behind the better of the two kernels on average.
+// both.  Over 912 shapes of int8 [N, K] 0.8 % behind the better of the two kernels on average, over 1006 of int4 [N, K / 8] 0.7 %.
 constexpr double kPassesMargin = 1.05;
 int64_t repack_pitch_words(int64_t N) { return (N / 8 + 3) / 4 * 4; }
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
@@ -917,8 +917,15 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             return launch_wq_gemm4(g4, x_bf16, f16 ? 1 : 0, w_kn, 4, scale_gn, offset_gn, bias, out_bf16, M, N, K, group_size, ldx, pitch,
                                    ldo, workspace, stream);
         }
-        if (wq_kpacked_decode_shape(M, N, K, group_size) && ldw_n < (1ll << 29)) {
-            // at most 32 rows, groups of 128: the barrier-free kernel that splits K inside the workgroup
+        const WqKpackedPlan kp = make_wq_kpacked_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
+        const bool ptrs_ok = aligned(scale_bf16, 2) && (!offset_bf16 || aligned(offset_bf16, 2)) && aligned(out_bf16, 2) &&
+                             (!bias || aligned(bias, 2));
+        bool decode = wq_kpacked_decode_shape(M, N, K, group_size) && ldw_n < (1ll << 29);
+        if (const double passes_us = decode ? wq_kpacked_decode_passes_us(M, N, K) : 0.0; passes_us > 0.0)
+            // K takes several passes there: the kernel with the smaller estimate runs, or this one where there is no workspace for it
+            decode = !kp.ok || !ptrs_ok || passes_us < kPassesMargin * kp.us || (kp.S > 1 && !workspace_holds(kp.counter_bytes + kp.partial_bytes));
+        if (decode) {
+            // few rows, groups of 128: the barrier-free kernel that splits K inside the workgroup
             WqKpDecodeArgs d;
             d.x = static_cast<const uint16_t *>(x_bf16);
             d.w = w;
@@ -937,9 +944,6 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             const int st = launch_wq_kpacked_decode(d, f16 ? 1 : 0, static_cast<hipStream_t>(stream));
             if (st != MI355_ERR_UNSUPPORTED) return st;
         }
-        const WqKpackedPlan kp = make_wq_kpacked_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
-        const bool ptrs_ok = aligned(scale_bf16, 2) && (!offset_bf16 || aligned(offset_bf16, 2)) && aligned(out_bf16, 2) &&
-                             (!bias || aligned(bias, 2));
         if (!kp.ok || !ptrs_ok) return generic();
         if (kp.S > 1) {
             if (!workspace || workspace_bytes < kp.counter_bytes + kp.partial_bytes) return MI355_ERR_WORKSPACE;

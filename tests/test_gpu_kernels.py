@@ -1725,3 +1725,20 @@ def test_w8a16_passes_over_a_long_k(capi, golden, monkeypatch, M, K, N, split):
     assert capi.lib().mi355_weight_quant_matmul(x.data_ptr(), 0, w.data_ptr(), 8, sc.data_ptr(), of.data_ptr(), None, bare.data_ptr(), M, N, K, 0, 0, 1,
                                                 K, 1, K, N, None, 0, torch.cuda.current_stream().cuda_stream) == 0
     bf16_gate(bare, torch.from_numpy(want), floor=out.numel() < 8192)
+
+
+@pytest.mark.parametrize("M,K,N,split", [(5, 25600, 768, True), (2, 27648, 640, True), (32, 14336, 2816, True), (100, 13824, 640, True), (3, 12288, 1024, False),
+                                         (32, 6144, 1024, False), (40, 14336, 512, False)])
+def test_w4a16_words_along_k_passes_over_a_long_k(capi, golden, monkeypatch, M, K, N, split):
+    """The same for an int4 weight stored [N, K/8], scale groups of 128."""
+    d = workloads.w4a16_inputs(seed=M + K + N, M=M, K=K, N=N)
+    _, want = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]), _bits(d["antiquant_offset"]), group_size=128)
+    w = torch.from_numpy(golden.pack_int4(np.ascontiguousarray(d["weight_int4_values"].numpy().T))).cuda().t()
+    x, sc, of = (d[k].cuda() for k in ("x", "antiquant_scale", "antiquant_offset"))
+    out, used = _leaves_sums_in_the_workspace(capi, monkeypatch, lambda: capi.weight_quant_matmul(x, w, sc, of, group_size=128))
+    bf16_gate(out, torch.from_numpy(want), floor=out.numel() < 8192)
+    assert used is split
+    bare = torch.empty_like(out)
+    assert capi.lib().mi355_weight_quant_matmul(x.data_ptr(), 0, w.data_ptr(), 4, sc.data_ptr(), of.data_ptr(), None, bare.data_ptr(), M, N, K, 128, N, 1,
+                                                K, 1, K // 8, N, None, 0, torch.cuda.current_stream().cuda_stream) == 0
+    bf16_gate(bare, torch.from_numpy(want), floor=out.numel() < 8192)
