@@ -205,16 +205,22 @@ __global__ __launch_bounds__(W * KS * 64) void wq_stream_kernel(const WqArgs p)
         // rows are dealt to the wavefronts, the lanes walk along a row; the loads of a lane are independent of
         // its LDS stores, so they all go out before the first one is needed
         const uint16_t *xsrc = p.x + (int64_t)m_base * p.ldx + (int64_t)cstep0 * 32;
-        for (int r = wave; r < rows_valid; r += W * KS) {
-            const uint16_t *xrow = xsrc + (int64_t)r * p.ldx;
-            char *dst = xs + (((r >> 4) * 64 + (r & 15)) << 4);
+        const auto stage = [&](auto past_k) {
+            for (int r = wave; r < rows_valid; r += W * KS) {
+                const uint16_t *xrow = xsrc + (int64_t)r * p.ldx;
+                char *dst = xs + (((r >> 4) * 64 + (r & 15)) << 4);
 #pragma unroll 4
-            for (int q = lane; q < pieces; q += 64) {
-                // (past K: zeros)
-                const u32x4 v = cstep0 * 32 + q * 8 < p.K ? *reinterpret_cast<const u32x4 *>(xrow + q * 8) : u32x4{0u, 0u, 0u, 0u};
-                *reinterpret_cast<u32x4 *>(dst + ((((q >> 2) * MT) * 64 + (q & 3) * 16) << 4)) = v;
+                for (int q = lane; q < pieces; q += 64) {
+                    u32x4 v{0u, 0u, 0u, 0u};
+                    if (!decltype(past_k)::value || cstep0 * 32 + q * 8 < p.K) v = *reinterpret_cast<const u32x4 *>(xrow + q * 8);
+                    *reinterpret_cast<u32x4 *>(dst + ((((q >> 2) * MT) * 64 + (q & 3) * 16) << 4)) = v;
+                }
             }
-        }
+        };
+        // only the chunk that reaches past the end of K (a scalar test) compares its pieces with it and puts zeros there: the
+        // comparison keeps the loads from going out together (22x6656x7232: 25.8 us where every chunk does, 23.2 without)
+        if (cstep0 * 32 + pieces * 8 > p.K) stage(std::true_type{});
+        else stage(std::false_type{});
     }
     __syncthreads();
     const char *xw = xs + ((size_t)(step0 - cstep0) * MT * 64 + lane) * 16;   // this wavefront's first fragment
