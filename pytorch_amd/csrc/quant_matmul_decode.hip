@@ -89,7 +89,7 @@ __global__ __launch_bounds__(512) void qmm_decode_kernel(const QmmDecodeArgs p)
 
     // The wavefront's slice of the activations of a pass, in operand order: every strip multiplies the same fragments.
     i32x4v xf[NS][MT][2];
-    auto load_x = [&](int pass) {
+    auto load_steps = [&](int pass, auto past_k) {
 #pragma unroll
         for (int j = 0; j < NS; j++) {
             const int st = pass * NS + j;
@@ -98,8 +98,15 @@ __global__ __launch_bounds__(512) void qmm_decode_kernel(const QmmDecodeArgs p)
 #pragma unroll
                 for (int h = 0; h < 2; h++)
                     xf[j][mt][h] = __builtin_bit_cast(i32x4v, __builtin_amdgcn_raw_buffer_load_b128(
-                        rsrc_x, st < ns && (s0 + st) * kStep < kpos[h] ? voff_x[mt][h] : kOutOfRange, (uint32_t)(s0 + st) * kStep, 0));
+                        rsrc_x, st < ns && (!decltype(past_k)::value || (s0 + st) * kStep < kpos[h]) ? voff_x[mt][h] : kOutOfRange, (uint32_t)(s0 + st) * kStep, 0));
         }
+    };
+    // With 16 steps only the wavefront whose range reaches past the end of K (a scalar test) compares its pieces with it
+    // (2x12032x3264: 11.6 us where all do, 10.9 without); with fewer the second copy of the loads costs more than it saves
+    // (17x3712x4144: 7.3 and 7.6 us).
+    auto load_x = [&](int pass) {
+        if (NS < 16 || (s0 + ns) * kStep > p.K) load_steps(pass, std::true_type{});
+        else load_steps(pass, std::false_type{});
     };
     // turn the activation fragments around (a wavefront's LDS operations complete in order)
     auto turn_x = [&]() {
