@@ -978,12 +978,13 @@ int launch_qmm(QmmArgs p, hipStream_t s)
     return check_launch();
 }
 
-// Tile shapes (rows x columns of the workgroup tile) the library instantiates, with measured times at K = 4096
-// on operands that are not cache resident: `slots` workgroups are resident at once (256 CUs x 1 or 2), a launch
-// that fits in one round of them takes `single_us` in all, longer launches take `round_us` per round.
+// Tile shapes (rows x columns of the workgroup tile) the library instantiates, with the coefficients of the estimate below at K = 4096 on
+// operands that are not cache resident: `slots` workgroups are resident at once (256 CUs x 1 or 2), a launch that fits in one round of
+// them costs `single_us` in all, a longer one `round_us` per round.  They are fitted together with the constants, not measured one by
+// one: of a tile whose choices lie mostly on one side the other coefficient can be off.
 // `whole`: the variant of a 128-row tile that keeps three whole stages (as many activation slots as weight slots) and
 // has a CU to itself: its activation refills get two K steps to land instead of one, which is what a tile needs when no
-// second workgroup on the CU covers the wait (128x192 at K = 4096: 37.2 -> 31.6 us per round, 128x128: 33.0 -> 24.7).
+// second workgroup on the CU covers the wait (launches of one round at K = 4096: 128x192 37.2 -> 31.6 us, 128x128 33.0 -> 24.7).
 struct TileChoice {
     int bm, bn, slots;
     double single_us, round_us;
@@ -1029,7 +1030,9 @@ double choose_tile_and_split(int64_t M, int64_t N, int64_t K, bool may_split, si
     for (const TileChoice &c : kTiles) {
         if (forced_tile && (c.bm != forced_tile / 1000 || c.bn != forced_tile % 1000)) continue;
         if (c.whole && knob(kKnobQmmLoop) == 1) continue;   // MI355_QMM_LOOP = 1: only the generic loop with its usual rings
-        if (!c.whole && knob(kKnobQmmLoop) == 4 && c.bm == 128 && (c.bn == 128 || c.bn == 192)) continue;   // 4: only their whole-stage variants
+        // The 128-row tiles that have a whole-stage variant run that one (and the others with the knob at 1 only): two workgroups to a CU are
+        // not the best plan of any of 1054 shapes, and the estimate has them too low (943x4352x6656: 64 us, 128x256 tiles 38).
+        if (!c.whole && knob(kKnobQmmLoop) != 1 && c.bm == 128 && (c.bn == 128 || c.bn == 192)) continue;
         const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
         for (const int S : {1, 2, 3, 4, 6, 8, 12, 16}) {
             if (forced_split >= 1 && forced_split <= kt && may_split) {
@@ -1290,7 +1293,7 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
     if (c.bm == bm_ && c.bn == bn_) return launch_qmm<wgm_, wgn_, bm_ / (16 * wgm_), bn_ / (16 * wgn_)>(p, s);
     MI355_QMM_CASE(256, 256, 2, 4)
     {
-        const int lk = knob(kKnobQmmLoop);                 // 0: automatic; 1: the generic loop; 2, 3: the wide loop with refills in a block / spread; 4: see the planner
+        const int lk = knob(kKnobQmmLoop);                 // 0: automatic; 1: the generic loop; 2, 3: the wide loop with refills in a block / spread
         if (lk != 1) {
             if (c.bm == 256 && c.bn == 224) {
                 if (lk == 2) return launch_qmm<4, 2, 4, 7, 0, 1>(p, s);
