@@ -548,22 +548,24 @@ WqGemm4Plan make_wq_gemm4_plan(int64_t M, int64_t N, int64_t K, int w_bits, int6
     auto zone = [&](int64_t s) { return (uint64_t)(s - 1) * (uint64_t)tiles * (uint64_t)pl.bm * 256u * 4u + (uint64_t)tiles * 4u; };
     while (S > 1 && zone(S) > kWorkspaceZoneBytes) S--;
     int64_t even = S;
-    while (even > 1 && !grouped && stages % even != 0) even--;
+    while (even > 1 && !grouped && (uint32_t)stages % (uint32_t)even != 0) even--;
     if (w_bits == 8 && !grouped && knob(kKnobWqgSplit) == 0) {
         // The split with the smallest estimate, if that is clearly below the one into equal chunks.  Strips are dealt to the XCDs in
         // eights, so a split that fits 256 workgroups can still be a second round (62x8448x8768: seven ways 40 x 7 slots, 47.7 us; six
         // ways 33.4).  Fitted to every split of 1655 shapes, 4 % off: the choice is 2.7 % behind the best on average, equal chunks 33 %, and
         // never more than 1 % behind those.
-        const double wgs = (double)((pl.strips + 7) / 8 * pl.tiles_m);
-        const auto us = [&](int64_t s) {
-            const int64_t rounds = ((int64_t)wgs * s + 31) / 32, per = (stages + s - 1) / s;
-            return 1.1 + (double)N * (double)K / 27.5e6 + (double)rounds * (3.9 + 0.64 * (double)per) + (s > 1 ? 2.7 : 0.0) +
-                   (double)(s - 1) * (0.83 + 4.6 * (double)tiles / 256.0);
-        };
-        int64_t best = S;
-        while (S-- > 1)
-            if (us(S) < us(best)) best = S;
-        S = 1.05 * us(best) < us(even) ? best : even;
+        const int per_xcd = (pl.strips + 7) / 8 * pl.tiles_m, st = (int)stages, limit = (int)S;
+        const double fixed = 1.1 + (double)N * (double)K / 27.5e6, exchange = 0.83 + 4.6 * (double)tiles / 256.0;
+        double best_us = 1e300, even_us = 0.0;
+        for (int s = 1; s <= limit; s++) {
+            const double us = fixed + (double)((per_xcd * s + 31) >> 5) * (3.9 + 0.64 * (double)((st + s - 1) / s)) + (s > 1 ? 2.7 : 0.0) + (double)(s - 1) * exchange;
+            if (s == even) even_us = us;
+            if (us < best_us) {
+                best_us = us;
+                S = s;
+            }
+        }
+        if (1.05 * best_us >= even_us) S = even;
     } else if (w_bits == 4) {
         S = even;
     }

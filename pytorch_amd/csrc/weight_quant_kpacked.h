@@ -17,13 +17,15 @@ struct WqKpackedPlan {
     int unit_sub;            // sub-steps of 128 k per scale group (grouped only)
     bool grouped;
     size_t lds_bytes, counter_bytes, partial_bytes;   // workspace when S > 1: [arrival counters | partial sums]
-    double us;               // estimated time, at most 32 rows
 };
 
 // `ldw_n`: int32 words between the rows of two consecutive output columns
 __attribute__((visibility("hidden"))) WqKpackedPlan make_wq_kpacked_plan(int64_t M, int64_t N, int64_t K, int64_t group_size,
                                                                          int64_t ldw_n, int64_t ldx, const void *x,
                                                                          const void *w);
+
+// Estimated time in us, for at most 32 rows and groups of 128.
+__attribute__((visibility("hidden"))) double wq_kpacked_us(const WqKpackedPlan &plan, int64_t M, int64_t N, int64_t K);
 
 // scale / offset element (group, column) at index group * ld_param_g + column * ld_param_n, any strides;
 // `workspace` holds counter_bytes + partial_bytes when plan.S > 1

@@ -478,11 +478,15 @@ WqKpackedPlan make_wq_kpacked_plan(int64_t M, int64_t N, int64_t K, int64_t grou
     pl.lds_bytes = lds_need(S);
     pl.partial_bytes = S > 1 ? (size_t)S * M * N * sizeof(float) : 0;
     pl.counter_bytes = S > 1 ? kWorkspaceZeroBytes : 0;
-    // fitted to the same shapes as the estimate of the decode kernel's passes, 5 % off on average; tiles are dealt to the XCDs in eights
-    const int rounds = ((pl.tiles + 7) / 8 * S * pl.mchunks + 31) / 32;
-    pl.us = 1.0 + rounds * ((pl.nw == 8 ? 0.0 : pl.mt == 1 ? 7.0 : 10.5) + (pl.nw == 8 ? 0.75 : 0.33) * (double)(K / 256) / S) + 0.27 * S +
-            (double)N * (double)K / 17.7e6 + (double)S * (double)M * (double)N / 150e3;
     return pl;
+}
+
+double wq_kpacked_us(const WqKpackedPlan &pl, int64_t M, int64_t N, int64_t K)
+{
+    // fitted to the same shapes as the estimate of the decode kernel's passes, 5 % off on average; tiles are dealt to the XCDs in eights
+    const int rounds = ((pl.tiles + 7) / 8 * pl.S * pl.mchunks + 31) / 32;
+    return 1.0 + rounds * ((pl.nw == 8 ? 0.0 : pl.mt == 1 ? 7.0 : 10.5) + (pl.nw == 8 ? 0.75 : 0.33) * (double)(K / 256) / pl.S) + 0.27 * pl.S +
+           (double)N * (double)K / 17.7e6 + (double)pl.S * (double)M * (double)N / 150e3;
 }
 
 int launch_wq_kpacked(const WqKpackedPlan &pl, const void *x, int act_f16, const void *w, const void *scale, const void *offset,

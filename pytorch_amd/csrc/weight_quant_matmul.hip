@@ -677,7 +677,6 @@ struct WqKmPlan {
     int mt, mchunks, tiles, S, unit_steps, n_units;
     bool grouped;
     size_t partial_bytes, counter_bytes, lds_bytes;
-    double us;                             // estimated time, at most 32 rows
 };
 
 WqKmPlan make_kmajor_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw_n, int64_t ldx, const void *x,
@@ -714,11 +713,16 @@ WqKmPlan make_kmajor_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, i
     pl.partial_bytes = S > 1 ? (size_t)S * M * N * sizeof(float) : 0;
     pl.counter_bytes = S > 1 ? kWorkspaceZeroBytes : 0;
     pl.lds_bytes = 16 + (size_t)2 * 32768 + 8 * 2 * 2048;   // two activation chunks + the turn-around tiles
-    // fitted to the same shapes as the estimate of the decode kernel's passes, 6 % off on average; tiles are dealt to the XCDs in eights
-    const int rounds = ((pl.tiles + 7) / 8 * S * pl.mchunks + 31) / 32;
-    pl.us = 1.3 + rounds * (4.2 + 0.4 * ((pl.n_units * pl.unit_steps + S - 1) / S)) + 0.15 * S + (double)N * (double)K / 14.2e6 +
-            (double)S * (double)M * (double)N / 142e3;
     return pl;
+}
+
+// Estimated time in us for at most 32 rows and one scale per column, fitted to the same shapes as the estimate of the decode kernel's
+// passes, 6 % off on average; tiles are dealt to the XCDs in eights.
+double kmajor_us(const WqKmPlan &pl, int64_t M, int64_t N, int64_t K)
+{
+    const int rounds = ((pl.tiles + 7) / 8 * pl.S * pl.mchunks + 31) / 32;
+    return 1.3 + rounds * (4.2 + 0.4 * ((pl.n_units + pl.S - 1) / pl.S)) + 0.15 * pl.S + (double)N * (double)K / 14.2e6 +
+           (double)pl.S * (double)M * (double)N / 142e3;
 }
 
 template <int MT, bool GROUPED, int ACT>
@@ -789,7 +793,7 @@ bool repack_applies(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t
 int preferred_n_major_kernel(int64_t M, int64_t N, int64_t K, int w_bits, int64_t group_size, int64_t ldw_k, int64_t ldx)
 {
     if (w_bits == 4 && make_wq_decode_plan(M, N, K, 4, group_size, ldw_k, ldx, nullptr, nullptr, nullptr, nullptr).ok) return kPreferDecode;
-    if (make_wq_gemm4_plan(M, N, K, w_bits, group_size, ldw_k, ldx, nullptr, nullptr, nullptr, nullptr).ok) return kPreferGemm4;
+    if (make_wq_gemm4_plan(M, N, K, w_bits, group_size, ldw_k, ldx, nullptr, nullptr, nullptr, nullptr, 0).ok) return kPreferGemm4;   // (no split to look for)
     if (make_wq_gemm_plan(M, N, K, w_bits, group_size, 1, ldw_k, ldx, nullptr, nullptr, nullptr, nullptr).ok) return kPreferGemm;
     return kPreferStream;
 }
@@ -842,8 +846,10 @@ extern "C" size_t mi355_weight_quant_matmul_workspace(int64_t M, int64_t N, int6
                 if (kp.ok && kp.partial_bytes + kp.counter_bytes > need) need = kp.partial_bytes + kp.counter_bytes;
             }
         } else {                            // the K-major layout may split differently
-            const WqGemm4Plan g8 = make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_n_major, ldx, nullptr, nullptr, nullptr, nullptr);
-            if (g8.ok && g8.S > 1 && kWorkspaceZeroBytes > need) need = kWorkspaceZeroBytes;
+            if (need < kWorkspaceZeroBytes) {
+                const WqGemm4Plan g8 = make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_n_major, ldx, nullptr, nullptr, nullptr, nullptr);
+                if (g8.ok && g8.S > 1) need = kWorkspaceZeroBytes;
+            }
             const WqKmPlan km = make_kmajor_plan(M, N, K, group_size, ldw_k_major, ldx, nullptr, nullptr);
             if (km.fast && km.partial_bytes + km.counter_bytes > need) need = km.partial_bytes + km.counter_bytes;
         }
@@ -923,13 +929,16 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             return launch_wq_gemm4(g4, x_bf16, f16 ? 1 : 0, w_kn, 4, scale_gn, offset_gn, bias, out_bf16, M, N, K, group_size, ldx, pitch,
                                    ldo, workspace, stream);
         }
-        const WqKpackedPlan kp = make_wq_kpacked_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
+        const auto plan = [&]() { return make_wq_kpacked_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w); };
         const bool ptrs_ok = aligned(scale_bf16, 2) && (!offset_bf16 || aligned(offset_bf16, 2)) && aligned(out_bf16, 2) &&
                              (!bias || aligned(bias, 2));
         bool decode = wq_kpacked_decode_shape(M, N, K, group_size) && ldw_n < (1ll << 29);
-        if (const double passes_us = decode ? wq_kpacked_decode_passes_us(M, N, K) : 0.0; passes_us > 0.0)
+        if (const double passes_us = decode ? wq_kpacked_decode_passes_us(M, N, K) : 0.0; passes_us > 0.0) {
             // K takes several passes there: the kernel with the smaller estimate runs, or this one where there is no workspace for it
-            decode = !kp.ok || !ptrs_ok || passes_us < kPassesMargin * kp.us || (kp.S > 1 && !workspace_holds(kp.counter_bytes + kp.partial_bytes));
+            const WqKpackedPlan other = plan();
+            decode = !other.ok || !ptrs_ok || passes_us < kPassesMargin * wq_kpacked_us(other, M, N, K) ||
+                     (other.S > 1 && !workspace_holds(other.counter_bytes + other.partial_bytes));
+        }
         if (decode) {
             // few rows, groups of 128: the barrier-free kernel that splits K inside the workgroup
             WqKpDecodeArgs d;
@@ -950,6 +959,7 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
             const int st = launch_wq_kpacked_decode(d, f16 ? 1 : 0, static_cast<hipStream_t>(stream));
             if (st != MI355_ERR_UNSUPPORTED) return st;
         }
+        const WqKpackedPlan kp = plan();
         if (!kp.ok || !ptrs_ok) return generic();
         if (kp.S > 1) {
             if (!workspace || workspace_bytes < kp.counter_bytes + kp.partial_bytes) return MI355_ERR_WORKSPACE;
@@ -970,7 +980,7 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
                 decode = !other.ok || !out_ok || (other.S > 1 && !workspace_holds(other.counter_bytes + other.partial_bytes));
             } else {
                 const WqKmPlan other = make_kmajor_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w);
-                decode = !other.fast || passes_us < kPassesMargin * other.us || (other.S > 1 && !workspace_holds(other.counter_bytes + other.partial_bytes));
+                decode = !other.fast || passes_us < kPassesMargin * kmajor_us(other, M, N, K) || (other.S > 1 && !workspace_holds(other.counter_bytes + other.partial_bytes));
             }
         }
         if (decode) {
