@@ -1054,7 +1054,7 @@ double choose_tile_and_split(int64_t M, int64_t N, int64_t K, bool may_split, si
             const double at_4096 = rounds == 1 ? c.single_us : (double)rounds * c.round_us;
             double loop_us = (at_4096 - kBaseUs) * ((double)kt / s_eff) / 32.0;
             // tiles that run two to a CU: with more than 256 and fewer than 512 workgroups the CUs that hold two set the
-            // time, as if all did (128x128 split six ways, 384 workgroups: 42 us where eight ways, 512, take 38)
+            // time, as if all did (seen with 128x128 tiles: split six ways, 384 workgroups, 42 us where eight ways, 512, take 38)
             if (c.slots == 512 && rounds == 1 && wgs > 256) loop_us *= 512.0 / (double)wgs;
             // ... and with at most 256 every workgroup has a CU to itself
             if (c.slots == 512 && wgs <= 256) loop_us *= c.bm == 64 ? kStreamAloneOnCu : kAloneOnCu;
