@@ -23,6 +23,7 @@
 #include "common.h"
 #include "quant_matmul_decode.h"
 #include "quant_matmul_wide.h"
+#include "quant_matmul_pingpong.h"
 #include <stdio.h>
 #include <type_traits>
 #include <stdlib.h>
@@ -107,7 +108,7 @@ __device__ __forceinline__ int32_t requant1(int32_t a, int32_t bi, float sc, flo
 // WGM x WGN wavefronts per workgroup, each owning (16*WTM) x (16*WTN) of the output tile.
 // LOOP 0: the generic K loop below; 3: the same with as many activation slots as weight slots (whole stages requested
 // NS steps ahead); 1, 2: the loop of quant_matmul_wide.h (4 x 2 wavefronts of 64 rows) with its
-// instruction order 0 (refills in a block) or 1 (refills spread over the step); 4: 2 and a partial last step of K (in one kernel
+// instruction order 0 (refills in a block) or 1 (refills spread over the step); 5: the loop of quant_matmul_pingpong.h; 4: 2 and a partial last step of K (in one kernel
 // with the loop, the step that few launches take costs 2048x4096x28672 0.5 %)
 // EPI (the widest wavefront tile only, see LEAN below): which variants of the LDS-parameter epilogue this instantiation holds
 template <int WGM, int WGN, int WTM, int WTN, int NS, int LOOP = 0, int EPI = 0>
@@ -124,8 +125,9 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     constexpr int ORDER = LOOP == 1 ? 0 : 1;                 // instruction order of the wide loop
     constexpr bool WHOLE = NS >= 4 || LOOP == 3;             // whole stages: activations get NS slots as well
     // the epilogues that take their parameters from LDS (quant_matmul_wide.h: wavefronts of 64 rows): the wide loop's tiles
-    // and the whole-stage 128-row tiles, which keep the vectors behind their ring
-    constexpr bool LDSP = WIDE || (LOOP == 3 && WTM == 4);
+    // and the whole-stage 128-row tiles and the alternating loop's, which keep the vectors (256 entries) behind their ring
+    constexpr bool PP = LOOP == 5;
+    constexpr bool LDSP = WIDE || (LOOP == 3 && WTM == 4) || (PP && BN <= 256);
     constexpr int NSA = WHOLE ? NS : 2;                      // activation slots; NS weight slots follow them in LDS
     constexpr uint32_t kOutOfRange = 0x80000000u;            // lane offset beyond every buffer: the load writes zeros
     static_assert(UNITS_A % NW == 0, "A units must divide evenly over the wavefronts");
@@ -208,7 +210,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     // (the widest wavefront tile holds few variants of it at a time: every further one costs the K loop registers it does not
     // have - 2048x4096x28672 went from 203 to 219 us with all of them in one kernel.  EPI 0: no bias or a bf16 one; 1: an
     // int32 or float32 bias; 2: packed parameter words with no bias or an int32 one.)
-    constexpr bool LEAN = WTN >= 7;
+    constexpr bool LEAN = WTN >= 7 || WTM == 8;
     const bool lean_bias = EPI == 0 ? p.bias_kind == MI355_BIAS_NONE || p.bias_kind == MI355_BIAS_BF16
                                     : EPI == 1 && (p.bias_kind == MI355_BIAS_INT32 || p.bias_kind == MI355_BIAS_FP32);
     const bool lean_qp = EPI == 2 && (p.bias_kind == MI355_BIAS_NONE || p.bias_kind == MI355_BIAS_INT32);
@@ -220,12 +222,12 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     const bool fast_epilogue_qp = LDSP && (!LEAN || lean_qp) && !p.out_i32 && !p.out_i8 && p.qparam && !p.pertoken && p.scale_len == p.N && (p.ldc & 7) == 0 &&
                                   aligned_dev(p.out, 16) && aligned_dev(p.qparam, 16) && (!p.bias || aligned_dev(p.bias, 16));
     // ... and so does the one for the re-quantised int8 output with per-channel parameter words
-    const bool fast_epilogue_i8 = LDSP && p.out_i8 && p.qparam && p.scale_len == p.N &&
+    const bool fast_epilogue_i8 = LDSP && WTM == 4 && p.out_i8 && p.qparam && p.scale_len == p.N &&
                                   (p.bias_kind == MI355_BIAS_NONE || p.bias_kind == MI355_BIAS_INT32) && (p.ldc & 15) == 0 &&
                                   aligned_dev(p.out, 16) && aligned_dev(p.qparam, 16) && (!p.bias || aligned_dev(p.bias, 16));
 
     // requested by one wavefront in front of its first stage (loads retire in order: they have landed when stage 0 has)
-    constexpr int PARAM_BASE = WIDE ? wide::Geometry<WTN>::PARAM_BASE : NSA * A_BYTES + (NS > 0 ? NS : 1) * B_BYTES;
+    constexpr int PARAM_BASE = WIDE ? wide::Geometry<WTN>::PARAM_BASE : PP ? pingpong::Geometry<WGM, WGN, WTM, WTN>::PARAM_BASE : NSA * A_BYTES + (NS > 0 ? NS : 1) * B_BYTES;
     if constexpr (LDSP) {
         if (fast_epilogue && wave == 0)
             wide::request_params(lds, PARAM_BASE, p.pertoken, p.scale, p.scale_len == 1, p.bias, p.bias_kind == MI355_BIAS_BF16 ? 2 : 4,
@@ -280,6 +282,27 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
         MI355_TS(2)
         __syncthreads();
         MI355_TS(3)
+    } else if constexpr (PP) {
+        using G = pingpong::Geometry<WGM, WGN, WTM, WTN>;
+        const int frow = lane & 15;
+        const uint32_t sw0 = (uint32_t)(((lane >> 4) ^ ((frow >> 1) & 7)) * 16);
+        pingpong::LoopState st;
+        st.rsrc_a = rsrc_a;
+        st.rsrc_b = rsrc_b;
+        st.voff_a = voff_a;
+        st.voff_b = voff_b;
+        st.gchunk = gchunk;
+        st.stride_a = unit_stride_a;
+        st.stride_b = unit_stride_b;
+        st.k0 = (uint32_t)kt0 * BK;
+        st.KT = KT;
+        st.kbytes = kbytes;
+        st.va = (uint32_t)((wm * WTM * 16 + frow) * BK) + sw0;
+        st.vax = (uint32_t)((wm * WTM * 16 + frow) * BK) + (sw0 ^ 64u);
+        st.vb = (uint32_t)(G::B_BASE + (wn * WTN * 16 + frow) * BK) + sw0;
+        st.vbx = (uint32_t)(G::B_BASE + (wn * WTN * 16 + frow) * BK) + (sw0 ^ 64u);
+        pingpong::k_loop<WGM, WGN, WTM, WTN>(acc, lds, st, wave);
+        __syncthreads();
     } else if constexpr (NS == 0) {
         // ---- streaming K loop (at most 64 rows, few workgroups per CU: the weights are a pure HBM stream).  No workgroup
         // ring and no barrier per K step: a wavefront owns its 16 weight rows (= 16 output columns) for the whole K range
@@ -551,6 +574,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     }
 
     if constexpr (LDSP) {
+        // the epilogues take 64 rows of a wavefront at a time (256x256 tile: 6.3 us behind the loop with the general one)
         if (fast_epilogue_i8) {
             wide::EpilogueArgs e;
             e.param_base = PARAM_BASE;
@@ -563,9 +587,9 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             e.has_bias = p.bias_kind == MI355_BIAS_INT32;
             e.out_f16 = 0;
             e.stream_out = p.stream_out;
-            e.wm = wm;
+            e.wm = wm * (WTM / 4);                            // in blocks of 64 rows
             e.wn = wn;
-            wide::epilogue_fast_i8<WTN>(acc, lds, e, wave, lane);
+            if constexpr (WTM == 4) wide::epilogue_fast_i8<WTN>(acc, lds, e, wave, lane);
             return;
         }
         if (fast_epilogue || fast_epilogue_qp) {
@@ -581,9 +605,13 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             e.has_bias = p.bias ? p.bias_kind : MI355_BIAS_NONE;
             e.out_f16 = p.out_f16;
             e.stream_out = p.stream_out;
-            e.wm = wm;
+            e.wm = wm * (WTM / 4);                            // in blocks of 64 rows
             e.wn = wn;
             wide::epilogue_fast<WTN, EPI>(acc, lds, e, wave, lane);
+            if constexpr (WTM == 8) {
+                e.wm++;
+                wide::epilogue_fast<WTN, EPI, 4>(acc, lds, e, wave, lane);
+            }
             MI355_TS(4)
             return;
         }
@@ -962,7 +990,7 @@ int launch_qmm(QmmArgs p, hipStream_t s)
     constexpr int NS = DEEP < 0 ? 0 : DEEP ? DEEP : 2 * a_bytes + 2 * b_bytes <= 80 * 1024 && staging_bytes <= 80 * 1024 ? 2 : 3;
     // DEEP < 0: the streaming K loop (two activation chunks of 32 KiB and a ring of five 2 KiB weight steps per wavefront)
     constexpr size_t stage_bytes = DEEP < 0 ? (size_t)2 * 32768 + 8 * 5 * 2048 : (DEEP ? DEEP : 2) * a_bytes + NS * b_bytes;
-    constexpr size_t ring_bytes = LOOP == 1 || LOOP == 2 || LOOP == 4 ? (size_t)wide::Geometry<WTN>::LDS_BYTES : stage_bytes + (LOOP == 3 ? 3072 : 0);
+    constexpr size_t ring_bytes = LOOP == 5 ? (size_t)pingpong::Geometry<WGM, WGN, WTM, WTN>::LDS_BYTES : LOOP == 1 || LOOP == 2 || LOOP == 4 ? (size_t)wide::Geometry<WTN>::LDS_BYTES : stage_bytes + (LOOP == 3 ? 3072 : 0);
     constexpr size_t lds_bytes = ring_bytes > staging_bytes ? ring_bytes : staging_bytes;
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
     p.tiles_m = (p.M + BM - 1) / BM;
@@ -990,8 +1018,8 @@ struct TileChoice {
     double single_us, round_us;
     int whole;
 };
-constexpr TileChoice kTiles[] = {{256, 256, 256, 48.6, 50.0, 0}, {256, 224, 256, 40.1, 42.9, 0}, {256, 192, 256, 39.0, 37.1, 0},
-                                 {128, 320, 256, 41.8, 38.3, 0}, {128, 256, 256, 38.3, 36.2, 0}, {128, 192, 512, 38.1, 53.9, 0},
+constexpr TileChoice kTiles[] = {{256, 256, 256, 45.8, 44.6, 0}, {256, 224, 256, 40.1, 42.9, 0}, {256, 192, 256, 39.0, 37.1, 0},
+                                 {128, 320, 256, 39.0, 38.3, 0}, {128, 256, 256, 30.5, 36.2, 0}, {128, 192, 512, 38.1, 53.9, 0},
                                  {128, 128, 512, 31.4, 35.7, 0}, {64, 256, 512, 36.8, 47.9, 0},  {64, 128, 512, 25.1, 20.6, 0},
                                  {128, 192, 256, 30.5, 26.2, 1}, {128, 128, 256, 22.7, 19.2, 1}};
 
@@ -1011,8 +1039,9 @@ struct QmmPlan {
 // wgs x bm x bn x 4 bytes of partial sums out and in again, the S - 1 foreign chunks of a tile through the one workgroup
 // that collects them (128x256 tiles split twelve ways: 39 us where a four-way split of 64x128 tiles takes 25).
 // Table and constants are fitted to sweeps over every tile and split of 290 shapes, M = 33 .. 2048, K = 1024 .. 14336, N = 1024
-// .. 28672 drawn evenly over their logarithms: the estimate's choice is 0.7 % slower than the measured best on average and
-// 17 % at worst (4 % and 25 % with constants fitted to layer projections of K = 4096 .. 14336 only).
+// .. 28672 drawn evenly over their logarithms; those of the three tiles that run the loop of quant_matmul_pingpong.h to 670 further ones
+// from 129 rows up: the estimate's choice is 1.1 % slower than the measured best there on average and 21 % at worst (1.4 and 27 % with
+// the coefficients those tiles had before that loop).
 constexpr size_t kMaxPartialBytes = (size_t)128 << 20;
 constexpr uint64_t kStreamOutMaxBytes = (uint64_t)32 << 20;     // the L2s of the eight XCDs together
 constexpr double kBaseUs = 4.0, kL2BytesPerUs = 13.1e6, kExchangeUs = 2.9, kExchangeBytesPerUs = 6.0e6, kCollectorBytesPerUs = 163e3;
@@ -1291,7 +1320,7 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
 #endif
 #define MI355_QMM_CASE(bm_, bn_, wgm_, wgn_)  \
     if (c.bm == bm_ && c.bn == bn_) return launch_qmm<wgm_, wgn_, bm_ / (16 * wgm_), bn_ / (16 * wgn_)>(p, s);
-    MI355_QMM_CASE(256, 256, 2, 4)
+    if (c.bm == 256 && c.bn == 256) return launch_qmm<2, 4, 8, 4, 0, 5>(p, s);
     {
         const int lk = knob(kKnobQmmLoop);                 // 0: automatic; 1: the generic loop; 2, 3: the wide loop with refills in a block / spread
         if (lk != 1) {
@@ -1316,8 +1345,8 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
         if (c.bm == 128 && c.bn == 128) return launch_qmm<2, 4, 4, 2, 3, 3>(p, s);
         return MI355_ERR_UNSUPPORTED;
     }
-    MI355_QMM_CASE(128, 320, 2, 4)
-    MI355_QMM_CASE(128, 256, 2, 4)
+    if (c.bm == 128 && c.bn == 320) return launch_qmm<2, 4, 4, 5, 0, 5>(p, s);
+    if (c.bm == 128 && c.bn == 256) return launch_qmm<2, 4, 4, 4, 0, 5>(p, s);
     MI355_QMM_CASE(128, 192, 2, 4)
     MI355_QMM_CASE(128, 128, 2, 4)
     {

@@ -420,8 +420,10 @@ __device__ __forceinline__ void request_params(char *lds, int param_base, const 
 // BIAS: 0 none, 1 bf16 (added last), 2 int32 (added to the accumulator, wrapping like it), 3 float32 (added last)
 // QP: the column scales are the low words of the packed 64-bit parameters (request_params_i8's layout) and there are no
 // per-token scales
-template <int WTN, bool F16, int BIAS, bool NT, bool QP = false>
-__device__ __forceinline__ void epilogue_rows(i32x4v (&acc)[4][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
+// I0: the first of the wavefront's 16-row blocks (the epilogues take 64 rows at a time; 256x256 tile: 6.3 us behind the loop with
+// the general one)
+template <int WTN, bool F16, int BIAS, bool NT, bool QP, int I0, int WTM>
+__device__ __forceinline__ void epilogue_rows(i32x4v (&acc)[WTM][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
 {
     constexpr int ROWB = WTN * 32 + 16;                       // padded pitch of a staged row: spreads rows over the banks
     constexpr int CHUNKS = WTN * 2;                           // 16-byte chunks per row of the wavefront tile
@@ -458,7 +460,7 @@ __device__ __forceinline__ void epilogue_rows(i32x4v (&acc)[4][WTN], char *lds, 
             float f[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                float v = BIAS == 2 ? (float)(int32_t)((uint32_t)acc[i][j][r] + __float_as_uint(bs[j][r])) : (float)acc[i][j][r];
+                float v = BIAS == 2 ? (float)(int32_t)((uint32_t)acc[I0 + i][j][r] + __float_as_uint(bs[j][r])) : (float)acc[I0 + i][j][r];
                 v = v * ps[i];
                 v = v * sc[j][r];
                 if constexpr (BIAS == 1 || BIAS == 3) v = v + bs[j][r];
@@ -491,26 +493,26 @@ __device__ __forceinline__ void epilogue_rows(i32x4v (&acc)[4][WTN], char *lds, 
 
 // EPI: the variants a kernel of the widest tile holds (0: float32 scales with no bias or a bf16 one; 1: float32 scales with
 // an int32 or float32 bias; 2: packed parameter words with no bias or an int32 one); the narrower tiles hold them all.
-template <int WTN, int EPI = 0>
-__device__ __forceinline__ void epilogue_fast(i32x4v (&acc)[4][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
+template <int WTN, int EPI = 0, int I0 = 0, int WTM>
+__device__ __forceinline__ void epilogue_fast(i32x4v (&acc)[WTM][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
 {
     // output type, kind of bias and kind of store are resolved once per wavefront
     auto go = [&](auto f16, auto bias) {
         constexpr bool H = decltype(f16)::value;
         constexpr int B = decltype(bias)::value;
-        constexpr bool LEAN = WTN >= 7;
+        constexpr bool LEAN = WTN >= 7 || WTM == 8;
         constexpr bool PLAIN = !LEAN || (EPI == 0 && B < 2) || (EPI == 1 && B >= 2);   // variants with float32 scales
         constexpr bool PACKED = !LEAN || (EPI == 2 && (B == 0 || B == 2));             // ... with packed parameter words
         if constexpr (PACKED) {
             if (LEAN || e.packed_scale) {
-                if (e.stream_out) epilogue_rows<WTN, H, B, true, true>(acc, lds, e, wave, lane);
-                else epilogue_rows<WTN, H, B, false, true>(acc, lds, e, wave, lane);
+                if (e.stream_out) epilogue_rows<WTN, H, B, true, true, I0>(acc, lds, e, wave, lane);
+                else epilogue_rows<WTN, H, B, false, true, I0>(acc, lds, e, wave, lane);
                 return;
             }
         }
         if constexpr (PLAIN) {
-            if (e.stream_out) epilogue_rows<WTN, H, B, true>(acc, lds, e, wave, lane);
-            else epilogue_rows<WTN, H, B, false>(acc, lds, e, wave, lane);
+            if (e.stream_out) epilogue_rows<WTN, H, B, true, false, I0>(acc, lds, e, wave, lane);
+            else epilogue_rows<WTN, H, B, false, false, I0>(acc, lds, e, wave, lane);
         }
     };
     using T = std::true_type;

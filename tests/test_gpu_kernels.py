@@ -391,7 +391,7 @@ def test_quant_matmul_wide_loop_tiles(capi, golden, tile, M, K, N):
     per-token scale + bf16 bias / no bias in bf16 and fp16, the LDS-parameter one for the re-quantised int8 output when the
     output rows are 16-byte aligned, and the general one for the other bias kinds, a single scale, no per-token scale, int32
     and unaligned int8 outputs) bit-identical to the generic loop and to the oracle.  (The
-    256x256 tile, which only has the generic loop, runs through the same cases against the oracle; the 128x128 and 128x192
+    256x256 tile, which only has the alternating loop, runs through the same cases against the oracle; the 128x128 and 128x192
     tiles run their variant with three whole stages, MI355_QMM_LOOP = 4, against their usual rings.)"""
     d = workloads.quant_matmul_inputs(seed=M + N + K, M=M, K=K, N=N, weight_nk=True, bias=True)
     g = torch.Generator().manual_seed(M + K)
@@ -444,6 +444,35 @@ def test_quant_matmul_wide_loop_tiles(capi, golden, tile, M, K, N):
                 capi.set_tuning("MI355_QMM_STREAM_OUT", 0)
     finally:
         for k in ("MI355_QMM_TILE", "MI355_QMM_SPLIT", "MI355_QMM_LOOP", "MI355_QMM_STREAM_OUT"):
+            capi.set_tuning(k, 0)
+
+
+@pytest.mark.parametrize("tile", [256256, 128256, 128320])
+@pytest.mark.parametrize("M,K,N,splits", [(1, 128, 16, (0,)), (129, 256, 257, (0, 2)), (300, 384, 640, (0, 3)), (777, 1040, 1000, (0, 2, 4)), (256, 2000, 321, (0, 2))])
+def test_quant_matmul_alternating_loop_tiles(capi, golden, tile, M, K, N, splits):
+    """The tiles whose wavefronts take turns at multiplying: one, two and three K steps (the prologue requests two), a K that ends
+    inside a step, ragged and tiny tiles, with and without a split of K: accumulators and outputs bit-identical to the oracle."""
+    d = workloads.quant_matmul_inputs(seed=M + N + K, M=M, K=K, N=N, weight_nk=True, bias=True)
+    x1, x2, sc, ps, bias = (d[k].cuda() for k in ("x1", "x2", "scale", "pertoken_scale", "bias"))
+    bias_i32 = torch.randint(-(1 << 20), 1 << 20, (N,), generator=torch.Generator().manual_seed(N), dtype=torch.int32)
+    qp = golden.trans_quant_param((d["scale"] * 1e-2).numpy(), np.zeros(N, np.float32))
+    acc_want = golden.int8_gemm(d["x1"].numpy(), d["x2"].numpy())
+    want, _ = golden.quant_matmul(d["x1"].numpy(), d["x2"].numpy(), d["scale"].numpy(), d["pertoken_scale"].numpy(), _bits(d["bias"]))
+    plain, _ = golden.quant_matmul(d["x1"].numpy(), d["x2"].numpy(), d["scale"].numpy(), d["pertoken_scale"].numpy())
+    want_i8 = golden.quant_matmul_requant(d["x1"].numpy(), d["x2"].numpy(), qp, bias_i32.numpy())
+    capi.set_tuning("MI355_QMM_TILE", tile)
+    try:
+        for split in splits:
+            capi.set_tuning("MI355_QMM_SPLIT", split)
+            for stream_out in (1, 2):
+                capi.set_tuning("MI355_QMM_STREAM_OUT", stream_out)
+                assert np.array_equal(capi.quant_matmul(x1, x2, None, out_dtype=torch.int32).cpu().numpy(), acc_want), split
+                assert np.array_equal(_bits(capi.quant_matmul(x1, x2, sc, ps, bias)), want), split
+                assert np.array_equal(_bits(capi.quant_matmul(x1, x2, sc, ps, None)), plain), split
+                got = capi.quant_matmul_qparam(x1, x2, capi.trans_quant_param((d["scale"] * 1e-2).cuda(), torch.zeros(N).cuda()), bias_i32.cuda())
+                assert np.array_equal(got.cpu().numpy(), want_i8), split
+    finally:
+        for k in ("MI355_QMM_TILE", "MI355_QMM_SPLIT", "MI355_QMM_STREAM_OUT"):
             capi.set_tuning(k, 0)
 
 
