@@ -120,7 +120,7 @@ __device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi)
 // Planner tuning knobs (tuning.hip): 0 = automatic.  Read with knob(); set through mi355_set_tuning() or, once at
 // load time, through the environment variable of the same name.
 // MI355_WQ_GEMM4_OFF / MI355_WQ_DECODE_OFF: 1 = the register-expanding int4 GEMM / the int4 decode kernel is not used;
-// 2 = its K-split exchange always writes through to memory.
+// 2 = its K-split exchange always writes through to memory; 3 = int8 [K, N] takes the tiles of up to 256 rows whatever the estimates say.
 // MI355_QMM_DECODE_OFF: 1 = quant_matmul with at most 64 rows takes the tiled kernel instead of the decode kernel.
 // MI355_WQ_MAX_POLLS: bound of the int4 kernels' wait for the other workgroups' partial sums (0 = 2^20 polls);
 // MI355_WQ_ONLY_CHUNK: c + 1 = only the workgroups of K chunk c do anything, -1 = only the collecting chunk (with a small MI355_WQ_MAX_POLLS this drives

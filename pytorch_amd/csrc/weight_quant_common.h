@@ -96,6 +96,20 @@ __device__ __forceinline__ u32x2 sbytes_act4(uint32_t w)
     }
 }
 
+// The images of bytes i and j of a word, in this order.
+template <int ACT>
+__device__ __forceinline__ uint32_t sbytes_act2(uint32_t w, int i, int j)
+{
+    if constexpr (ACT == 0) {
+        return pack_act2<ACT>(sbyte_f32(w, i), sbyte_f32(w, j));
+    } else {
+        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+        const f16x2 bias = {(_Float16)1152.0f, (_Float16)1152.0f};
+        const uint32_t sel = 0x04000400u | ((uint32_t)j << 16) | (uint32_t)i;
+        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, w ^ 0x80808080u, sel)) - bias);
+    }
+}
+
 template <int WBITS, int ACT>
 __device__ __forceinline__ void expand_pair(const uint32_t (&w)[8], int jb, uint32_t magic, u32x4 &b0, u32x4 &b1)
 {

@@ -8,6 +8,7 @@ namespace mi355 {
 
 struct WqGemm4Plan {
     bool ok;                 // the kernel accepts this problem
+    double us;                  // estimated time (int8 without a forced split; otherwise 0)
     int bm;                  // activation rows per workgroup tile: 64 or 128
     int tiles_m, strips;     // workgroup tiles: row blocks x strips of 256 columns (128 bytes of an int4 row, 256 of an int8 row)
     int S;                   // workgroups that share a tile's K range

@@ -566,6 +566,7 @@ WqGemm4Plan make_wq_gemm4_plan(int64_t M, int64_t N, int64_t K, int w_bits, int6
             }
         }
         if (1.05 * best_us >= even_us) S = even;
+        pl.us = S == even ? even_us : best_us;
     } else if (w_bits == 4) {
         S = even;
     }

@@ -1,5 +1,5 @@
-// npu_weight_quant_batchmatmul, int8 weight stored [N, K] with one scale per column (what LinearWeightQuant keeps), more than 32
-// activation rows: a tiled GEMM on the 16-bit MFMA.
+// npu_weight_quant_batchmatmul, int8 weight stored [N, K] with one scale per column (what LinearWeightQuant keeps), or [K, N] where the
+// estimates prefer it to weight_quant_gemm4.hip, more than 32 activation rows: a tiled GEMM on the 16-bit MFMA.
 //
 // A workgroup of eight wavefronts (4 x 2) owns 64 * WTM rows x 128 columns; a wavefront owns 16 * WTM x 64.  K is walked in stages
 // of 64.  What bounds the kernel is the LDS (192 KiB of it pass per stage of a 256-row tile, at 85 bytes per clock; the MFMAs are busy
@@ -17,6 +17,12 @@
 // times as fast on average over 120 shapes.  Two more forms, measured: raw bytes read as fragments and converted by every wavefront
 // for itself (136 KiB per stage, but four times the conversions, which take issue slots from the MFMAs): the same to 5 % slower; with
 // it tiles of 256 columns: 20 % slower.
+// [K, N] weights (template parameter KN): a wavefront copies one k octet of all 128 columns and its lanes read the bytes of two columns
+// each, row by row, so the images are written transposed; everything behind the images is the same.  The eight 2-byte reads make a
+// stage 10 to 35 % longer than that of [N, K] (four 4-byte reads of a column quad with 8-byte image writes, conflict-free by a swizzle
+// of their own, were no faster on tall tiles and 8 % slower on 128-row ones).  Before (weight_quant_gemm4.hip: 64 rows to a
+// workgroup, every weight converted once per 64 rows) and now, us: 384x4096x11008 94 -> 65, 2048x4096x4096 99 -> 82, 700x2048x8192
+// 51 -> 36, 145x10496x14560 112 -> 76, 100x14336x1040 36 -> 24, 44x4096x2816 21.5 -> 17; 0.85 of the time on average over 60 shapes.
 // Rows are 128 bytes with the 16-byte chunks XOR-swizzled by the row pair (conflict-free fragment reads); a K that is not a multiple
 // of 64 ends in a stage whose activations past K are loaded as zeros.
 //     out[m, n] = scale[n] * (sum_k x[m, k] w[n, k] + offset[n] * X[m]) + bias[n]
@@ -45,7 +51,7 @@ constexpr int kBN = 128, kStageK = 64;
 constexpr int kPitch = 128;                                    // bytes per LDS tile row: 64 k of 16 bits
 constexpr int kImageBytes = kBN * kPitch, kRawBytes = kBN * kStageK;
 
-template <int ACT, int WTM>
+template <int ACT, int WTM, bool KN>
 __global__ __launch_bounds__(512, 1) void wq_kmajor_gemm_kernel(const WqKmGemmArgs p)
 {
     constexpr int NW = 8, WGN = 2, WTN = 4;
@@ -93,26 +99,48 @@ __global__ __launch_bounds__(512, 1) void wq_kmajor_gemm_kernel(const WqKmGemmAr
         }
     };
 
-    // ---- weights: wavefront w copies the stage's 64 bytes of columns 16 w .. 16 w + 15
+    // ---- weights: wavefront w copies the stage's 64 bytes of columns 16 w .. 16 w + 15; of a [K, N] weight rows 8 w .. 8 w + 7 (the
+    // w-th k octet) of all 128 columns
     const int cols_valid = min(kBN, p.N - n0);
     const __amdgpu_buffer_rsrc_t rsrc_w =
-        make_rsrc(static_cast<const char *>(p.w) + (size_t)n0 * p.ldw, (uint32_t)(cols_valid - 1) * p.ldw + (uint32_t)p.K);
-    const uint32_t voff_w = (uint32_t)(lane >> 2) * p.ldw + (uint32_t)(lane & 3) * 16u;
+        KN ? make_rsrc(static_cast<const char *>(p.w) + n0, (uint32_t)(p.K - 1) * p.ldw + (uint32_t)cols_valid)
+           : make_rsrc(static_cast<const char *>(p.w) + (size_t)n0 * p.ldw, (uint32_t)(cols_valid - 1) * p.ldw + (uint32_t)p.K);
+    const uint32_t voff_w = !KN ? (uint32_t)(lane >> 2) * p.ldw + (uint32_t)(lane & 3) * 16u
+                            : (lane & 7) * 16 < cols_valid ? (uint32_t)(lane >> 3) * p.ldw + (uint32_t)(lane & 7) * 16u : kOutOfRange;
     auto issue_w = [&](int s) {
+        const uint32_t so = KN ? (uint32_t)((s0 + s) * kStageK + wave * 8) * p.ldw : (uint32_t)wave * 16u * p.ldw + (uint32_t)(s0 + s) * 64u;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (lds_void *)(lds + RAW_BASE + (s % 3) * kRawBytes + wave * 1024), 16,
-                                                 s < NSTG ? voff_w : kOutOfRange, (uint32_t)wave * 16u * p.ldw + (uint32_t)(s0 + s) * 64u, 0, 0);
+                                                 s < NSTG ? voff_w : kOutOfRange, so, 0, 0);
     };
-    // two runs of eight consecutive k of one column each: chunk c = t * 512 + wave * 64 + lane is k octet c % 8 of column c / 8
+    // [N, K]: two runs of eight consecutive k of one column each: chunk c = t * 512 + wave * 64 + lane is k octet c % 8 of column c / 8.
+    // [K, N]: a word per pair of rows of the octet with the bytes of columns 2 lane and 2 lane + 1 (run t is column 2 lane + t).
     u32x2 wx[2];
     auto read_raw = [&](int s) {
-        const char *src = lds + RAW_BASE + (s % 3) * kRawBytes + (wave * 64 + lane) * 8;
+        const char *src = lds + RAW_BASE + (s % 3) * kRawBytes;
+        if constexpr (KN) {
+            typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-        for (int t = 0; t < 2; t++) wx[t] = *reinterpret_cast<const u32x2 *>(src + t * 4096);
+            for (int v = 0; v < 4; v++) {
+                u16x2 rows;
+                rows.x = *reinterpret_cast<const uint16_t *>(src + wave * 1024 + (2 * v) * 128 + lane * 2);
+                rows.y = *reinterpret_cast<const uint16_t *>(src + wave * 1024 + (2 * v + 1) * 128 + lane * 2);
+                wx[v >> 1][v & 1] = __builtin_bit_cast(uint32_t, rows);
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 2; t++) wx[t] = *reinterpret_cast<const u32x2 *>(src + (wave * 64 + lane) * 8 + t * 4096);
+        }
     };
     auto expand = [&](int t, int s) {
-        const int c = t * 512 + wave * 64 + lane, n = c >> 3, o = c & 7;
-        const u32x2 lo = sbytes_act4<ACT>(wx[t][0]), hi = sbytes_act4<ACT>(wx[t][1]);
-        const u32x4 b = u32x4{lo.x, lo.y, hi.x, hi.y};
+        const int c = t * 512 + wave * 64 + lane, n = KN ? 2 * lane + t : c >> 3, o = KN ? wave : c & 7;
+        u32x4 b;
+        if constexpr (KN) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) b[v] = sbytes_act2<ACT>(wx[v >> 1][v & 1], t, 2 + t);
+        } else {
+            const u32x2 lo = sbytes_act4<ACT>(wx[t][0]), hi = sbytes_act4<ACT>(wx[t][1]);
+            b = u32x4{lo.x, lo.y, hi.x, hi.y};
+        }
         *reinterpret_cast<u32x4 *>(lds + IMAGE_BASE + (s & 1) * kImageBytes + n * kPitch + ((o ^ ((n >> 1) & 7)) * 16)) = b;
     };
 
@@ -182,7 +210,7 @@ __global__ __launch_bounds__(512, 1) void wq_kmajor_gemm_kernel(const WqKmGemmAr
             for (int i = 0; i < WTM; i++) P[i][j] = mfma_act<ACT>(bf[0][j], af[0][i], P[i][j]);
         expand(0, s + 1);                                      // its slot was last read in stage s - 1
         expand(1, s + 1);
-        constexpr int MF = WTM * WTN, RD = WTM + WTN;
+        constexpr int MF = WTM * WTN, RD = WTM + WTN, RAW = KN ? 8 : 1;   // MFMAs, fragment and raw reads of a half
         constexpr int R1 = MF >= 2 * RD ? 1 : 2;               // LDS reads per MFMA
 #pragma unroll
         for (int q = 0; q < (RD + R1 - 1) / R1; q++) {
@@ -209,7 +237,7 @@ __global__ __launch_bounds__(512, 1) void wq_kmajor_gemm_kernel(const WqKmGemmAr
 #pragma unroll
             for (int i = 0; i < WTM; i++) P[i][j] = mfma_act<ACT>(bf[1][j], af[1][i], P[i][j]);
 #pragma unroll
-        for (int q = 0; q < (RD + R1) / R1; q++) {
+        for (int q = 0; q < (RD + RAW + R1 - 1) / R1; q++) {
             __builtin_amdgcn_sched_group_barrier(0x100, R1, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
@@ -328,43 +356,47 @@ __global__ __launch_bounds__(512, 1) void wq_kmajor_gemm_kernel(const WqKmGemmAr
     }
 }
 
-template <int ACT, int WTM>
+template <int ACT, int WTM, bool KN>
 int launch_tile(WqKmGemmArgs p, hipStream_t s)
 {
     constexpr int lds_bytes = 3 * 64 * WTM * kPitch + 2 * kImageBytes + 3 * kRawBytes;
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
-    auto kern = wq_kmajor_gemm_kernel<ACT, WTM>;
+    auto kern = wq_kmajor_gemm_kernel<ACT, WTM, KN>;
     static int attr_status = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (attr_status != hipSuccess) return MI355_ERR_LAUNCH;
     hipLaunchKernelGGL(kern, dim3((unsigned)(8 * p.items_per_xcd)), dim3(512), lds_bytes, s, p);
     return check_launch();
 }
 
-template <int ACT>
+template <int ACT, bool KN>
 int launch_act(const WqKmGemmArgs &p, int wtm, hipStream_t s)
 {
-    return wtm == 1 ? launch_tile<ACT, 1>(p, s) : wtm == 2 ? launch_tile<ACT, 2>(p, s) : wtm == 3 ? launch_tile<ACT, 3>(p, s) : launch_tile<ACT, 4>(p, s);
+    return wtm == 1 ? launch_tile<ACT, 1, KN>(p, s) : wtm == 2 ? launch_tile<ACT, 2, KN>(p, s) : wtm == 3 ? launch_tile<ACT, 3, KN>(p, s) : launch_tile<ACT, 4, KN>(p, s);
 }
 
 } // namespace
 
 WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw, int64_t ldx, const void *x,
-                                      const void *w, const void *scale, const void *offset, size_t room)
+                                      const void *w, const void *scale, const void *offset, size_t room, bool n_major)
 {
     WqKmGemmPlan pl{};
+    pl.n_major = n_major;
     // the rows of a tile are addressed with 32-bit buffer offsets: rows far apart (one token of every sequence of a [128, 1024, 4096]
     // batch: a pitch of 4194304) rule out the tall tiles
     const auto offsets_fit = [&](int wtm) { return (uint64_t)(64 * wtm) * (uint64_t)ldx * 2 < (1ull << 31); };
-    pl.ok = M > 32 && M <= 0x7fffffff && (group_size == 0 || group_size == K) && K >= 128 && K % 8 == 0 && N % 8 == 0 && ldw >= K &&
-            ldw % 4 == 0 && (uint64_t)N * (uint64_t)ldw < (1ull << 32) && ldx % 8 == 0 && offsets_fit(2) &&
+    pl.ok = M > 32 && M <= 0x7fffffff && (group_size == 0 || group_size == K) && K >= 128 && K % 8 == 0 && N % 8 == 0 && ldw % 4 == 0 &&
+            (n_major ? ldw >= N && (uint64_t)K * (uint64_t)ldw < (1ull << 31) : ldw >= K && (uint64_t)N * (uint64_t)ldw < (1ull << 32)) && ldx % 8 == 0 && offsets_fit(2) &&
             (x == nullptr || aligned(x, 16)) && (w == nullptr || aligned(w, 4)) && (scale == nullptr || aligned(scale, 4)) &&
             (offset == nullptr || aligned(offset, 4)) && !knob(kKnobWqGemmOff);
     if (!pl.ok) return pl;
     // The tile and the split of K with the smallest estimated time: what a launch costs around the loop, rounds of the workgroups
     // that are resident at once (one to a CU, two of the 64-row tiles), but no less than the weights take from memory or the tiles
     // through the L2; and for a split the exchange of the sums.  Fitted to every tile and split of 120 shapes, M = 33 .. 2048, K = 1024
-    // .. 14336, N = 1024 .. 16384 spread evenly over their logarithms: the choice is 1.4 % behind the measured best on average.
-    constexpr double kBaseUs = 7.1, kStageUs[5] = {0.41, 0.675, 0.515, 0.657, 0.762};   // [0]: a 64-row tile alone on its CU
+    // .. 14336, N = 1024 .. 16384 spread evenly over their logarithms: the choice is 1.4 % behind the measured best on average.  [K, N]: the
+    // stage times of 60 such shapes on operands that come from memory.
+    constexpr double kBaseUs = 7.1;
+    constexpr double kStageUsNk[5] = {0.41, 0.675, 0.515, 0.657, 0.762}, kStageUsKn[5] = {0.49, 0.75, 0.71, 0.87, 1.05};   // [0]: a 64-row tile alone on its CU
+    const double *const kStageUs = n_major ? kStageUsKn : kStageUsNk;
     constexpr double kWeightBytesPerUs = 5.5e6, kL2BytesPerUs = 11.4e6, kExchangeUs = 2.2, kExchangeBytesPerUs = 7.5e6, kCollectorBytesPerUs = 100e3;
     const int64_t stages = (K + kStageK - 1) / kStageK;
     const int forced_bm = knob(kKnobWqgBm), forced_split = knob(kKnobWqgSplit);   // tuning aids
@@ -387,6 +419,7 @@ WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t g
             if (S > 1) us += kExchangeUs + (double)(wgs * chunk_bytes) * 2.0 / kExchangeBytesPerUs + (double)(S * chunk_bytes) / kCollectorBytesPerUs;
             if (us < best) {
                 best = us;
+                pl.us = us;
                 pl.wtm = wtm;
                 pl.S = S;
                 pl.partial_bytes = S > 1 ? (size_t)(wgs * chunk_bytes) : 0;
@@ -422,7 +455,8 @@ int launch_wq_kmajor_gemm(const WqKmGemmPlan &pl, const void *x, int act_f16, co
     p.items_per_xcd = (p.tiles_m * p.tiles_n * pl.S + 7) / 8;
     p.S = pl.S;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    return act_f16 ? launch_act<1>(p, pl.wtm, s) : launch_act<0>(p, pl.wtm, s);
+    if (pl.n_major) return act_f16 ? launch_act<1, true>(p, pl.wtm, s) : launch_act<0, true>(p, pl.wtm, s);
+    return act_f16 ? launch_act<1, false>(p, pl.wtm, s) : launch_act<0, false>(p, pl.wtm, s);
 }
 
 } // namespace mi355

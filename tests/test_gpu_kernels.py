@@ -775,6 +775,38 @@ def test_w8a16_kmajor_tiled_kernel(capi, golden, M, K, N, f16, offset):
             capi.set_tuning(k, 0)
 
 
+@pytest.mark.parametrize("M,K,N,f16,offset", [(33, 128, 8, True, True), (65, 448, 136, True, False), (129, 1040, 264, False, True),
+                                             (193, 2112, 128, True, True), (256, 1000, 392, False, False), (257, 640, 1000, False, True)])
+def test_w8a16_n_major_tall_tiles(capi, golden, M, K, N, f16, offset):
+    """int8 weight stored [K, N] on the tiles of up to 256 rows: every height unsplit and with K split, ragged rows and columns (a
+    last 16-byte piece of a weight row that is half beyond N), a partial last stage.  The activations are a view of a wider matrix whose
+    columns past K hold NaN; the weight rows are pitched."""
+    d = workloads.w8a16_inputs(seed=M + K, M=M, K=K, N=N)
+    dt = torch.float16 if f16 else torch.bfloat16
+    d = {k: (v.to(dt) if v.is_floating_point() else v) for k, v in d.items()}
+    xw = torch.full((M, K + 64), float("nan"), dtype=dt, device="cuda")
+    xw[:, :K] = d["x"].cuda()
+    ww = torch.full((K, (N + 15) // 16 * 16 + 16), 77, dtype=torch.int8, device="cuda")
+    ww[:, :N] = d["weight"].cuda()
+    of = d["antiquant_offset"] if offset else None
+    _, want = golden.weight_quant_matmul(_bits(d["x"]), d["weight"].numpy(), _bits(d["antiquant_scale"]), None if of is None else _bits(of),
+                                         dtype="fp16" if f16 else "bf16")
+    try:
+        capi.set_tuning("MI355_WQ_GEMM4_OFF", 3)
+        for bm in (64, 128, 192, 256):
+            capi.set_tuning("MI355_WQG_BM", bm)
+            for split in (1, 2, 3):
+                if split > (K + 63) // 64:
+                    continue
+                capi.set_tuning("MI355_WQG_SPLIT", split)
+                for _ in range(2):                             # the second launch meets the counters the first one left
+                    out = capi.weight_quant_matmul(xw[:, :K], ww[:, :N], d["antiquant_scale"].cuda(), None if of is None else of.cuda())
+                    bf16_gate(out, torch.from_numpy(want))
+    finally:
+        for k in ("MI355_WQ_GEMM4_OFF", "MI355_WQG_BM", "MI355_WQG_SPLIT"):
+            capi.set_tuning(k, 0)
+
+
 def test_w8a16_kmajor_and_no_offset(capi, golden):
     d = workloads.w8a16_inputs(seed=3, M=8, K=1024, N=192, weight_nk=True)
     out = capi.weight_quant_matmul(d["x"].cuda(), d["weight"].cuda(), d["antiquant_scale"].cuda(),
