@@ -790,6 +790,13 @@ bool repack_applies(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t
     return M >= kRepackRows && N % 8 == 0 && K % 128 == 0 &&
            make_wq_gemm4_plan(M, N, K, 4, group_size, repack_pitch_words(N), ldx, x, nullptr, nullptr, nullptr).ok;
 }
+// int8 [K, N] above 32 rows: the tiles of up to 256 rows where their estimate is below the one of 64-row tiles.  Over 60 shapes of
+// 33 .. 2048 rows the rule takes 39 of them, none slower than before: 384x4096x11008 94 -> 65 us, 59x1280x2400 15.7 -> 11.2; it leaves
+// 1024x4096x4096 (52, here 58) and 461x2688x4672 (32, here 37), where 64-row tiles fill one round.
+bool takes_tall_tiles(const WqKmGemmPlan &kn, const WqGemm4Plan &g8)
+{
+    return kn.ok && (kn.us < 0.99 * g8.us || knob(kKnobWqGemm4Off) == 3);
+}
 int preferred_n_major_kernel(int64_t M, int64_t N, int64_t K, int w_bits, int64_t group_size, int64_t ldw_k, int64_t ldx)
 {
     if (w_bits == 4 && make_wq_decode_plan(M, N, K, 4, group_size, ldw_k, ldx, nullptr, nullptr, nullptr, nullptr).ok) return kPreferDecode;
@@ -815,6 +822,7 @@ extern "C" size_t mi355_weight_quant_matmul_workspace(int64_t M, int64_t N, int6
     // make a launch prefer is planned within the workspace that this query asks for.
     auto pad = [](int64_t v, int64_t to) { return (v + to - 1) / to * to; };
     size_t need = 0;
+    bool kn_asked = false;
     for (int padded = 0; padded < 2; padded++) {
         const int64_t ldx = padded ? pad(K, 64) : K;                                  // activation pitch, elements
         const int64_t ldw_n_major = padded ? pad(w_bits == 4 ? N / 8 : N, w_bits == 4 ? 32 : 128) : (w_bits == 4 ? N / 8 : N);
@@ -826,6 +834,13 @@ extern "C" size_t mi355_weight_quant_matmul_workspace(int64_t M, int64_t N, int6
         }
         const WqKmGemmPlan kmg = w_bits == 8 ? make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_k_major, ldx, nullptr, nullptr, nullptr, nullptr) : WqKmGemmPlan{};
         if (kmg.ok && kmg.counter_bytes + kmg.partial_bytes > need) need = kmg.counter_bytes + kmg.partial_bytes;
+        if (w_bits == 8 && preferred == kPreferGemm4 && !kn_asked) {
+            // int8 [K, N] on the same tiles, by the launch's rule; strides do not change the plan, so one pitch is enough
+            const WqKmGemmPlan kn = make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n_major, ldx, nullptr, nullptr, nullptr, nullptr, ~(size_t)0, true);
+            const WqGemm4Plan g8 = make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_n_major, ldx, nullptr, nullptr, nullptr, nullptr);
+            if (takes_tall_tiles(kn, g8) && kn.counter_bytes + kn.partial_bytes > need) need = kn.counter_bytes + kn.partial_bytes;
+            kn_asked = kn.ok;
+        }
         for (int layout = 1; layout <= (w_bits == 8 ? 2 : 1); layout++) {
             if (layout == 1 ? w_bits == 4 && preferred != kPreferGemm : kmg.ok) continue;
             const WqGemmPlan gp = make_wq_gemm_plan(M, N, K, w_bits, group_size, layout, layout == 2 ? ldw_k_major : ldw_n_major, ldx,
@@ -1083,12 +1098,15 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
                 return make_wq_gemm4_plan(M, N, K, 8, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
             });
             if (st != MI355_OK) return st;
-            // Tiles of up to 256 rows, within the workspace that is there, where their estimate is below the one of 64-row tiles.  Over 60
-            // shapes of 33 .. 2048 rows the rule takes 39 of them, none slower than before: 384x4096x11008 94 -> 65 us, 59x1280x2400 15.7 ->
-            // 11.2; it leaves 1024x4096x4096 (52, here 58) and 461x2688x4672 (32, here 37), where 64-row tiles fill one round.
-            const WqKmGemmPlan kn = make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16,
-                                                             aligned(workspace, 16) ? room : 0, true);
-            if (kn.ok && (kn.us < 0.99 * g8.us || knob(kKnobWqGemm4Off) == 3))
+            // planned as the workspace query planned it, and within the room only where that is too little: the split, and with it the
+            // order of the float32 sums, must not depend on how far earlier calls have grown the caller's workspace
+            // (within what the query asked for other layouts: 1128x10368x3200 127 us, 1470x5120x1024 39; with its own split 100 and 35)
+            auto plan_kn = [&](size_t within) {
+                return make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_k, ldx, x_bf16, w, scale_bf16, offset_bf16, within, true);
+            };
+            WqKmGemmPlan kn = plan_kn(~(size_t)0);
+            if (kn.S > 1 && (kn.counter_bytes + kn.partial_bytes > room || !aligned(workspace, 16))) kn = plan_kn(aligned(workspace, 16) ? room : 0);
+            if (takes_tall_tiles(kn, g8))
                 return launch_wq_kmajor_gemm(kn, x_bf16, f16 ? 1 : 0, w, scale_bf16, offset_bf16, bias, out_bf16, M, N, K, ldx, ldw_k, ldo,
                                              workspace, stream);
             return launch_wq_gemm4(g8, x_bf16, f16 ? 1 : 0, w, 8, scale_bf16, offset_bf16, bias, out_bf16, M, N, K, group_size, ldx, ldw_k,

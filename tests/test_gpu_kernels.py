@@ -807,6 +807,19 @@ def test_w8a16_n_major_tall_tiles(capi, golden, M, K, N, f16, offset):
             capi.set_tuning(k, 0)
 
 
+@pytest.mark.parametrize("M,K,N", [(643, 3328, 1152), (1470, 5120, 1024), (414, 4224, 5376)])
+def test_w8a16_n_major_workspace(capi, monkeypatch, M, K, N):
+    """int8 weight stored [K, N]: the workspace query covers the split the launch prefers, so a larger workspace (what earlier calls
+    have left) gives the same bits."""
+    d = workloads.w8a16_inputs(seed=M, M=M, K=K, N=N)
+    args = d["x"].cuda(), d["weight"].cuda(), d["antiquant_scale"].cuda(), d["antiquant_offset"].cuda()
+    outs = []
+    for more in (0, 128 << 20):
+        monkeypatch.setattr(capi, "_wq_workspace", lambda device, need: torch.zeros(need + more, dtype=torch.int8, device=device))
+        outs.append(capi.weight_quant_matmul(*args))
+    assert torch.equal(*outs)
+
+
 def test_w8a16_kmajor_and_no_offset(capi, golden):
     d = workloads.w8a16_inputs(seed=3, M=8, K=1024, N=192, weight_nk=True)
     out = capi.weight_quant_matmul(d["x"].cuda(), d["weight"].cuda(), d["antiquant_scale"].cuda(),
