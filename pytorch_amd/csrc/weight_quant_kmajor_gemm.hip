@@ -305,12 +305,24 @@ __global__ __launch_bounds__(512, 1) void wq_kmajor_gemm_kernel(const WqKmGemmAr
         }
         __syncthreads();
         if (!is_last) return;
-        // every chunk is read back, the own one too: the order of the sum does not depend on the order of arrival
+        // The chunks are added in their order, whatever the order of arrival.  Tiles of 128 rows and more take the own one from registers:
+        // the last arrival reads up to 128 KiB per chunk with the chip idle around it (us before -> after, sums identical: 1024x11264x1664
+        // [N, K] 57.8 -> 56.1, four chunks; [K, N] 414x4224x5376 41.8 -> 39.6, three).  64-row tiles read it back: 1 % slower
+        // otherwise (135x3968x2176 17.6 -> 17.7, 100x14336x1040 23.2 -> 23.5).  Several chunks requested at once, the unwanted out of
+        // range, cost more than they hide (384x4096x4096 29.3 -> 30.4).
+        f32x4 sum[WTM][WTN];
 #pragma unroll
         for (int i = 0; i < WTM; i++)
 #pragma unroll
-            for (int j = 0; j < WTN; j++) P[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < WTN; j++) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int ch = 0; ch < p.S; ch++) {
+            if (WTM > 1 && ch == chunk) {
+#pragma unroll
+                for (int i = 0; i < WTM; i++)
+#pragma unroll
+                    for (int j = 0; j < WTN; j++) sum[i][j] = sum[i][j] + P[i][j];
+                continue;
+            }
             f32x4 v[WTM][WTN];
 #pragma unroll
             for (int i = 0; i < WTM; i++)
@@ -321,8 +333,12 @@ __global__ __launch_bounds__(512, 1) void wq_kmajor_gemm_kernel(const WqKmGemmAr
 #pragma unroll
             for (int i = 0; i < WTM; i++)
 #pragma unroll
-                for (int j = 0; j < WTN; j++) P[i][j] = P[i][j] + v[i][j];
+                for (int j = 0; j < WTN; j++) sum[i][j] = sum[i][j] + v[i][j];
         }
+#pragma unroll
+        for (int i = 0; i < WTM; i++)
+#pragma unroll
+            for (int j = 0; j < WTN; j++) P[i][j] = sum[i][j];
         if (threadIdx.x == 0) __hip_atomic_store(p.counter + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 
