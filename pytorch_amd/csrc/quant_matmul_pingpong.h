@@ -15,8 +15,9 @@
 // What bounds it: power.  At 4096x4096x4096 the loop runs at 2191 clocks a step where the MFMAs alone are 2048, but with operands as
 // quantisation leaves them the card holds 1.6 GHz there (2.25 GHz with zeros); v_mfma_i32_32x32x32_i8 in the same loop needs fewer
 // clocks (2134) and is slower (1.43 GHz, 62.5 us instead of 57).  Microseconds before (refills and fragment reads interleaved with the
-// MFMAs by scheduling groups) and now: 4096x4096x4096 62.0 -> 59.4, 2048x14336x4096 split two ways 114.3 -> 111.2 (256x256);
-// 777x11008x4096 split two ways 54.8 -> 45.6 (128x256).  On 256x192 and 256x224 it is level with quant_matmul_wide.h.
+// MFMAs by scheduling groups) and now: 4096x4096x4096 62.0 -> 59.4, 2048x14336x4096 split two ways 114.3 -> 111.2 (256x256),
+// and with the epilogue that has its parameters in LDS 53.0 and 102; 777x11008x4096 split two ways 54.8 -> 45.3 (128x256, with that
+// epilogue).  On 256x192 and 256x224 it is level with quant_matmul_wide.h.
 #pragma once
 #include "common.h"
 #include <type_traits>
