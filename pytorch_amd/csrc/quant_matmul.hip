@@ -209,7 +209,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     // the wide loop's epilogue for the common case takes its parameters from LDS (quant_matmul_wide.h)
     // (the widest wavefront tile holds few variants of it at a time: every further one costs the K loop registers it does not
     // have - 2048x4096x28672 went from 203 to 219 us with all of them in one kernel.  EPI 0: no bias or a bf16 one; 1: an
-    // int32 or float32 bias; 2: packed parameter words with no bias or an int32 one.)
+    // int32 or float32 bias; 2: packed parameter words with no bias or an int32 one, and on the 256x256 tile the int8 output.)
     constexpr bool LEAN = WTN >= 7 || WTM == 8;
     const bool lean_bias = EPI == 0 ? p.bias_kind == MI355_BIAS_NONE || p.bias_kind == MI355_BIAS_BF16
                                     : EPI == 1 && (p.bias_kind == MI355_BIAS_INT32 || p.bias_kind == MI355_BIAS_FP32);
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     const bool fast_epilogue_qp = LDSP && (!LEAN || lean_qp) && !p.out_i32 && !p.out_i8 && p.qparam && !p.pertoken && p.scale_len == p.N && (p.ldc & 7) == 0 &&
                                   aligned_dev(p.out, 16) && aligned_dev(p.qparam, 16) && (!p.bias || aligned_dev(p.bias, 16));
     // ... and so does the one for the re-quantised int8 output with per-channel parameter words
-    const bool fast_epilogue_i8 = LDSP && WTM == 4 && p.out_i8 && p.qparam && p.scale_len == p.N &&
+    const bool fast_epilogue_i8 = LDSP && (WTM == 4 || EPI == 2) && p.out_i8 && p.qparam && p.scale_len == p.N &&
                                   (p.bias_kind == MI355_BIAS_NONE || p.bias_kind == MI355_BIAS_INT32) && (p.ldc & 15) == 0 &&
                                   aligned_dev(p.out, 16) && aligned_dev(p.qparam, 16) && (!p.bias || aligned_dev(p.bias, 16));
 
@@ -574,7 +574,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
     }
 
     if constexpr (LDSP) {
-        // the epilogues take 64 rows of a wavefront at a time (256x256 tile: 6.3 us behind the loop with the general one)
+        // the epilogues take 64 rows of a wavefront at a time (256x256 tile: the general one is 2.0 to 2.4 us longer per round of tiles)
         if (fast_epilogue_i8) {
             wide::EpilogueArgs e;
             e.param_base = PARAM_BASE;
@@ -589,7 +589,11 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void qmm_kernel(const QmmArgs p)
             e.stream_out = p.stream_out;
             e.wm = wm * (WTM / 4);                            // in blocks of 64 rows
             e.wn = wn;
-            if constexpr (WTM == 4) wide::epilogue_fast_i8<WTN>(acc, lds, e, wave, lane);
+            if constexpr (WTM == 4 || EPI == 2) wide::epilogue_fast_i8<WTN>(acc, lds, e, wave, lane);
+            if constexpr (WTM == 8 && EPI == 2) {
+                e.wm++;
+                wide::epilogue_fast_i8<WTN, 4>(acc, lds, e, wave, lane);
+            }
             return;
         }
         if (fast_epilogue || fast_epilogue_qp) {
@@ -1320,16 +1324,18 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
 #endif
 #define MI355_QMM_CASE(bm_, bn_, wgm_, wgn_)  \
     if (c.bm == bm_ && c.bn == bn_) return launch_qmm<wgm_, wgn_, bm_ / (16 * wgm_), bn_ / (16 * wgn_)>(p, s);
-    if (c.bm == 256 && c.bn == 256) return launch_qmm<2, 4, 8, 4, 0, 5>(p, s);
+    // the instantiation of the 256x256 and 256x224 tiles whose LDS-parameter epilogue serves this call's kind of bias and scale
+    // (256x256 with the general epilogue and with its own, us: 4096x128x4096 13.9 and 11.8, 1972x1024x21888 on three rounds 66 and 57.5)
+    const bool to16 = !p.out_i32 && !p.out_i8;
+    const int epi = to16 && !p.qparam && (p.bias_kind == MI355_BIAS_INT32 || p.bias_kind == MI355_BIAS_FP32) ? 1
+                  : to16 && p.qparam && !p.pertoken && (p.bias_kind == MI355_BIAS_NONE || p.bias_kind == MI355_BIAS_INT32) ? 2 : 0;
+    if (c.bm == 256 && c.bn == 256)
+        return epi == 1 ? launch_qmm<2, 4, 8, 4, 0, 5, 1>(p, s) : epi == 2 || p.out_i8 ? launch_qmm<2, 4, 8, 4, 0, 5, 2>(p, s) : launch_qmm<2, 4, 8, 4, 0, 5>(p, s);
     {
         const int lk = knob(kKnobQmmLoop);                 // 0: automatic; 1: the generic loop; 2, 3: the wide loop with refills in a block / spread
         if (lk != 1) {
             if (c.bm == 256 && c.bn == 224) {
                 if (lk == 2) return launch_qmm<4, 2, 4, 7, 0, 1>(p, s);
-                // the instantiation whose LDS-parameter epilogue serves this call's kind of bias and scale
-                const bool to16 = !p.out_i32 && !p.out_i8;
-                const int epi = to16 && !p.qparam && (p.bias_kind == MI355_BIAS_INT32 || p.bias_kind == MI355_BIAS_FP32) ? 1
-                              : to16 && p.qparam && !p.pertoken && (p.bias_kind == MI355_BIAS_NONE || p.bias_kind == MI355_BIAS_INT32) ? 2 : 0;
                 if (p.K % BK != 0)
                     return epi == 1 ? launch_qmm<4, 2, 4, 7, 0, 4, 1>(p, s) : epi == 2 ? launch_qmm<4, 2, 4, 7, 0, 4, 2>(p, s) : launch_qmm<4, 2, 4, 7, 0, 4>(p, s);
                 return epi == 1 ? launch_qmm<4, 2, 4, 7, 0, 2, 1>(p, s) : epi == 2 ? launch_qmm<4, 2, 4, 7, 0, 2, 2>(p, s) : launch_qmm<4, 2, 4, 7, 0, 2>(p, s);

@@ -420,8 +420,7 @@ __device__ __forceinline__ void request_params(char *lds, int param_base, const 
 // BIAS: 0 none, 1 bf16 (added last), 2 int32 (added to the accumulator, wrapping like it), 3 float32 (added last)
 // QP: the column scales are the low words of the packed 64-bit parameters (request_params_i8's layout) and there are no
 // per-token scales
-// I0: the first of the wavefront's 16-row blocks (the epilogues take 64 rows at a time; 256x256 tile: 6.3 us behind the loop with
-// the general one)
+// I0: the first of the wavefront's 16-row blocks (the epilogues take 64 rows at a time)
 template <int WTN, bool F16, int BIAS, bool NT, bool QP, int I0, int WTM>
 __device__ __forceinline__ void epilogue_rows(i32x4v (&acc)[WTM][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
 {
@@ -491,7 +490,7 @@ __device__ __forceinline__ void epilogue_rows(i32x4v (&acc)[WTM][WTN], char *lds
     }
 }
 
-// EPI: the variants a kernel of the widest tile holds (0: float32 scales with no bias or a bf16 one; 1: float32 scales with
+// EPI: the variants a kernel of the widest tiles holds (0: float32 scales with no bias or a bf16 one; 1: float32 scales with
 // an int32 or float32 bias; 2: packed parameter words with no bias or an int32 one); the narrower tiles hold them all.
 template <int WTN, int EPI = 0, int I0 = 0, int WTM>
 __device__ __forceinline__ void epilogue_fast(i32x4v (&acc)[WTM][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
@@ -548,8 +547,8 @@ __device__ __forceinline__ void request_params_i8(char *lds, int param_base, con
     }
 }
 
-template <int WTN, bool BIAS, bool NT>
-__device__ __forceinline__ void epilogue_rows_i8(i32x4v (&acc)[4][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
+template <int WTN, bool BIAS, bool NT, int I0, int WTM>
+__device__ __forceinline__ void epilogue_rows_i8(i32x4v (&acc)[WTM][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
 {
     constexpr int ROWQ = WTN * 16 + 16;                       // padded pitch of a staged row of the wavefront tile
     constexpr int CHQ = WTN;                                  // 16-byte chunks per row
@@ -576,7 +575,7 @@ __device__ __forceinline__ void epilogue_rows_i8(i32x4v (&acc)[4][WTN], char *ld
             uint32_t w = 0;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                float v = (float)(int32_t)((uint32_t)acc[i][j][r] + (uint32_t)bi[r]);      // wraps like the accumulator
+                float v = (float)(int32_t)((uint32_t)acc[I0 + i][j][r] + (uint32_t)bi[r]); // wraps like the accumulator
                 v = v * sc[r];
                 v = v + of[r];
                 v = fminf(fmaxf(rintf(v), -128.0f), 127.0f);
@@ -604,15 +603,15 @@ __device__ __forceinline__ void epilogue_rows_i8(i32x4v (&acc)[4][WTN], char *ld
     }
 }
 
-template <int WTN>
-__device__ __forceinline__ void epilogue_fast_i8(i32x4v (&acc)[4][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
+template <int WTN, int I0 = 0, int WTM>
+__device__ __forceinline__ void epilogue_fast_i8(i32x4v (&acc)[WTM][WTN], char *lds, const EpilogueArgs &e, int wave, int lane)
 {
     if (e.has_bias) {
-        if (e.stream_out) epilogue_rows_i8<WTN, true, true>(acc, lds, e, wave, lane);
-        else epilogue_rows_i8<WTN, true, false>(acc, lds, e, wave, lane);
+        if (e.stream_out) epilogue_rows_i8<WTN, true, true, I0>(acc, lds, e, wave, lane);
+        else epilogue_rows_i8<WTN, true, false, I0>(acc, lds, e, wave, lane);
     } else {
-        if (e.stream_out) epilogue_rows_i8<WTN, false, true>(acc, lds, e, wave, lane);
-        else epilogue_rows_i8<WTN, false, false>(acc, lds, e, wave, lane);
+        if (e.stream_out) epilogue_rows_i8<WTN, false, true, I0>(acc, lds, e, wave, lane);
+        else epilogue_rows_i8<WTN, false, false, I0>(acc, lds, e, wave, lane);
     }
 }
 
