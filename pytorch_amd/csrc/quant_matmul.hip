@@ -1049,6 +1049,7 @@ struct QmmPlan {
 constexpr size_t kMaxPartialBytes = (size_t)128 << 20;
 constexpr uint64_t kStreamOutMaxBytes = (uint64_t)32 << 20;     // the L2s of the eight XCDs together
 constexpr double kBaseUs = 4.0, kL2BytesPerUs = 13.1e6, kExchangeUs = 2.9, kExchangeBytesPerUs = 6.0e6, kCollectorBytesPerUs = 163e3;
+constexpr double kOffLines = 1.18;
 constexpr double kAloneOnCu = 0.78, kStreamAloneOnCu = 0.70;    // 64-row tiles alone on their CU run the streaming loop or deep rings
 
 // (returns the estimate)
@@ -1091,6 +1092,11 @@ double choose_tile_and_split(int64_t M, int64_t N, int64_t K, bool may_split, si
             if (c.slots == 512 && rounds == 1 && wgs > 256) loop_us *= 512.0 / (double)wgs;
             // ... and with at most 256 every workgroup has a CU to itself
             if (c.slots == 512 && wgs <= 256) loop_us *= c.bm == 64 ? kStreamAloneOnCu : kAloneOnCu;
+            // Rows that do not start on cache lines: every 128-byte piece is two of them.  On a long K the two tiles with the most operand bytes per
+            // MFMA of those that have a CU to themselves feel it most, unsplit (870x13360x7456: 128x256 133 us, 256x256 split two ways 109).  Over 477
+            // shapes of such rows the choice is 1.9 % behind the measured best with this term, 3.2 % without; three of them are slower with it, by 6 % at
+            // most.  On all tiles, from any K, or as more bytes through the L2 it slows more shapes than it helps.
+            if (K % BK != 0 && K > 4096 && s_eff == 1 && c.bm == 128 && c.bn >= 256) loop_us *= kOffLines;
             double cost = kBaseUs + loop_us;
             const double l2 = kBaseUs + (double)tiles * (c.bm + c.bn) * (double)K / kL2BytesPerUs;
             if (l2 > cost) cost = l2;
@@ -1216,9 +1222,12 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
         if (bare.decode) pl = bare;
     }
     if (tiled && pl.workspace() > 0 && (!ws || workspace_bytes < pl.workspace() || !aligned(ws, 16))) {
-        // a K of whole steps needs its workspace; any other K also runs without one, on the generic kernel
+        // a K of whole steps needs its workspace; any other K also runs without one: unsplit, or where rows have to be copied on the
+        // generic kernel (870x13360x7456: 0.13 ms and tens of ms)
         if (K % BK == 0) return !ws || workspace_bytes < pl.workspace() ? MI355_ERR_WORKSPACE : MI355_ERR_ALIGNMENT;
-        tiled = false;
+        const QmmPlan bare = make_qmm_plan(M, N, K, ldb_k, ldb_n, zero_area, scratch_cap, false);
+        if (bare.workspace() == 0) pl = bare;
+        else tiled = false;
     }
     if (tiled && ldb_k != 1) {
         // contiguous [K,N]: transpose once into the workspace

@@ -559,6 +559,26 @@ def test_quant_matmul_256x256_epilogues_cost_the_same(capi):
     assert max(best.values()) < 1.08 * best["bf16"], best
 
 
+def test_quant_matmul_ragged_k_without_a_workspace(capi):
+    """870x13360x7456 splits K, but a caller who brings no workspace is served by unsplit tiles (0.1 ms) and not by the generic kernel (tens
+    of ms): 2 ms tell the two apart."""
+    M, K, N = 870, 13360, 7456
+    d = workloads.quant_matmul_inputs(seed=1, M=M, K=K, N=N, weight_nk=True)
+    x1, x2, sc, ps = (d[k].cuda() for k in ("x1", "x2", "scale", "pertoken_scale"))
+    assert capi.lib().mi355_quant_matmul_workspace(M, N, K, 1, K) > 0
+    want = capi.quant_matmul(x1, x2, sc, ps)
+    none = torch.empty(0, dtype=torch.int8, device="cuda")
+    times = []
+    for _ in range(5):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        got = capi.quant_matmul(x1, x2, sc, ps, workspace=none)
+        end.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(end))
+    assert torch.equal(got, want) and min(times) < 2.0, times
+
+
 def test_quant_matmul_wide_loop_strided_operands(capi, golden):
     """Row pitches larger than the rows (views into wider buffers) and an output view whose rows are not 16-byte aligned
     (the general epilogue): the wide loop addresses rows through the pitches only."""
