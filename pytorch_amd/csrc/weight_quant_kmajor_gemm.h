@@ -22,6 +22,12 @@ __attribute__((visibility("hidden"))) WqKmGemmPlan make_wq_kmajor_gemm_plan(int6
                                                                             const void *scale, const void *offset,
                                                                             size_t room = ~(size_t)0, bool n_major = false);
 
+// Whether the kernel takes such a problem.  Strides that it takes change the plan only where they rule out tall tiles, and its request then
+// never grows (200,000 shapes, activation rows 2^22 and more apart).
+__attribute__((visibility("hidden"))) bool wq_kmajor_gemm_accepts(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw, int64_t ldx,
+                                                                  const void *x, const void *w, const void *scale, const void *offset,
+                                                                  bool n_major = false);
+
 // Launches the kernel; `workspace` holds counter_bytes + partial_bytes when plan.S > 1.
 __attribute__((visibility("hidden"))) int launch_wq_kmajor_gemm(const WqKmGemmPlan &plan, const void *x, int act_f16, const void *w,
                                                                 const void *scale, const void *offset, const void *bias, void *out, int64_t M,

@@ -392,18 +392,25 @@ int launch_act(const WqKmGemmArgs &p, int wtm, hipStream_t s)
 
 } // namespace
 
+// the rows of a tile are addressed with 32-bit buffer offsets: rows far apart (one token of every sequence of a [128, 1024, 4096]
+// batch: a pitch of 4194304) rule out the tall tiles
+static bool offsets_fit(int wtm, int64_t ldx) { return (uint64_t)(64 * wtm) * (uint64_t)ldx * 2 < (1ull << 31); }
+
+bool wq_kmajor_gemm_accepts(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw, int64_t ldx, const void *x, const void *w,
+                            const void *scale, const void *offset, bool n_major)
+{
+    return M > 32 && M <= 0x7fffffff && (group_size == 0 || group_size == K) && K >= 128 && K % 8 == 0 && N % 8 == 0 && ldw % 4 == 0 &&
+           (n_major ? ldw >= N && (uint64_t)K * (uint64_t)ldw < (1ull << 31) : ldw >= K && (uint64_t)N * (uint64_t)ldw < (1ull << 32)) && ldx % 8 == 0 &&
+           offsets_fit(2, ldx) && (x == nullptr || aligned(x, 16)) && (w == nullptr || aligned(w, 4)) && (scale == nullptr || aligned(scale, 4)) &&
+           (offset == nullptr || aligned(offset, 4)) && !knob(kKnobWqGemmOff);
+}
+
 WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw, int64_t ldx, const void *x,
                                       const void *w, const void *scale, const void *offset, size_t room, bool n_major)
 {
     WqKmGemmPlan pl{};
     pl.n_major = n_major;
-    // the rows of a tile are addressed with 32-bit buffer offsets: rows far apart (one token of every sequence of a [128, 1024, 4096]
-    // batch: a pitch of 4194304) rule out the tall tiles
-    const auto offsets_fit = [&](int wtm) { return (uint64_t)(64 * wtm) * (uint64_t)ldx * 2 < (1ull << 31); };
-    pl.ok = M > 32 && M <= 0x7fffffff && (group_size == 0 || group_size == K) && K >= 128 && K % 8 == 0 && N % 8 == 0 && ldw % 4 == 0 &&
-            (n_major ? ldw >= N && (uint64_t)K * (uint64_t)ldw < (1ull << 31) : ldw >= K && (uint64_t)N * (uint64_t)ldw < (1ull << 32)) && ldx % 8 == 0 && offsets_fit(2) &&
-            (x == nullptr || aligned(x, 16)) && (w == nullptr || aligned(w, 4)) && (scale == nullptr || aligned(scale, 4)) &&
-            (offset == nullptr || aligned(offset, 4)) && !knob(kKnobWqGemmOff);
+    pl.ok = wq_kmajor_gemm_accepts(M, N, K, group_size, ldw, ldx, x, w, scale, offset, n_major);
     if (!pl.ok) return pl;
     // The tile and the split of K with the smallest estimated time: what a launch costs around the loop, rounds of the workgroups
     // that are resident at once (one to a CU, two of the 64-row tiles), but no less than the weights take from memory or the tiles
@@ -420,12 +427,13 @@ WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t g
     double best = 1e300;
     for (int wtm = 1; wtm <= 4; wtm++) {
         if (forced_bm > 0 && forced_bm % 64 == 0 && forced_bm <= 256 && forced_bm != 64 * wtm) continue;
-        if (!offsets_fit(wtm)) continue;
+        if (!offsets_fit(wtm, ldx)) continue;
         const int64_t tiles = ((M + 64 * wtm - 1) / (64 * wtm)) * ((N + kBN - 1) / kBN);
         if (tiles > 0x7fffffff / 16) continue;
         for (int S = 1; S <= 16; S++) {
             const int64_t slots = wtm == 1 ? 2 * kNumCU : kNumCU, wgs = tiles * S;
-            if (forced ? S != forced_split : S > 1 && (wgs > slots || stages / S < 4)) continue;
+            if (forced && S != forced_split) continue;
+            if (!forced && S > 1 && (wgs > slots || stages / S < 4)) break;
             const int64_t chunk_bytes = 64 * wtm * kBN * 4;
             if (S > 1 && ((uint64_t)tiles * 4 > kWorkspaceCounterBytes || (uint64_t)(wgs * chunk_bytes) > ((uint64_t)128 << 20) ||
                           kWorkspaceZeroBytes + (uint64_t)(wgs * chunk_bytes) > room)) continue;

@@ -621,3 +621,25 @@ def test_quant_matmul_rows_off_the_cache_lines(M, K, N, tile, split):
     tiles = -(-M // tile[0]) * -(-N // tile[1])
     need = _capi.ZERO_AREA_BYTES + tiles * split * tile[0] * tile[1] * 4 if split > 1 else 0
     assert _capi.lib().mi355_quant_matmul_workspace(M, N, K, 1, K) == need
+
+
+def test_weight_quant_workspace_query_plans_once():
+    """The query runs in front of every call and plans a kernel once, not once for dense and once for padded rows: above 32 rows it takes 2.3 to
+    2.5 times as long as at 16 rows (3.6 to 4.0 times when every kernel is planned twice).  The call that returns at once is the binding's share."""
+    import time
+    from pytorch_amd import _capi
+    query = _capi.lib().mi355_weight_quant_matmul_workspace
+    calls = {"none": (0, 1024, 1024, 8, 0), "few rows": (16, 4096, 4096, 8, 0), "tiled": (48, 1024, 1024, 8, 0)}
+    ratios = []
+    for _ in range(8):                                         # a busy machine disturbs some attempts
+        best = dict.fromkeys(calls, float("inf"))
+        for _ in range(30):
+            for name, args in calls.items():
+                start = time.perf_counter()
+                for _ in range(500):
+                    query(*args)
+                best[name] = min(best[name], time.perf_counter() - start)
+        ratios.append((best["tiled"] - best["none"]) / (best["few rows"] - best["none"]))
+        if ratios[-1] < 3.1:
+            return
+    raise AssertionError(ratios)
