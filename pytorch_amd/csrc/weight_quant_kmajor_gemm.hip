@@ -416,7 +416,8 @@ WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t g
     // that are resident at once (one to a CU, two of the 64-row tiles), but no less than the weights take from memory or the tiles
     // through the L2; and for a split the exchange of the sums.  Fitted to every tile and split of 120 shapes, M = 33 .. 2048, K = 1024
     // .. 14336, N = 1024 .. 16384 spread evenly over their logarithms: the choice is 1.4 % behind the measured best on average.  [K, N]: the
-    // stage times of 60 such shapes on operands that come from memory.
+    // stage times of 60 such shapes on operands that come from memory.  The collecting workgroup reads every chunk, of tiles of 128 rows and more
+    // all but its own: over 94 further shapes of [N, K] and 125 of [K, N] the choice is 0.8 and 1.3 % behind (1.1 and 1.9 with the own one counted).
     constexpr double kBaseUs = 7.1;
     constexpr double kStageUsNk[5] = {0.41, 0.675, 0.515, 0.657, 0.762}, kStageUsKn[5] = {0.49, 0.75, 0.71, 0.87, 1.05};   // [0]: a 64-row tile alone on its CU
     const double *const kStageUs = n_major ? kStageUsKn : kStageUsNk;
@@ -440,7 +441,7 @@ WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t g
             double us = (double)((wgs + slots - 1) / slots * ((stages + S - 1) / S)) * kStageUs[wtm == 1 && wgs <= kNumCU ? 0 : wtm];
             const double mem = (double)K * (double)N / kWeightBytesPerUs, l2 = (double)tiles * (128 * wtm + kBN) * (double)K / kL2BytesPerUs;
             us = kBaseUs + (us > mem ? us > l2 ? us : l2 : mem > l2 ? mem : l2);
-            if (S > 1) us += kExchangeUs + (double)(wgs * chunk_bytes) * 2.0 / kExchangeBytesPerUs + (double)(S * chunk_bytes) / kCollectorBytesPerUs;
+            if (S > 1) us += kExchangeUs + (double)(wgs * chunk_bytes) * 2.0 / kExchangeBytesPerUs + (double)((wtm > 1 ? S - 1 : S) * chunk_bytes) / kCollectorBytesPerUs;
             if (us < best) {
                 best = us;
                 pl.us = us;

@@ -643,3 +643,13 @@ def test_weight_quant_workspace_query_plans_once():
         if ratios[-1] < 3.1:
             return
     raise AssertionError(ratios)
+
+
+@pytest.mark.parametrize("M,K,N,rows,split", [(1491, 3840, 1808, 192, 2), (471, 3328, 4320, 128, 3)])
+def test_weight_quant_split_counts_the_chunks_that_are_read(M, K, N, rows, split):
+    """int8 tiles of 128 rows and more: the collecting workgroup reads the chunks of the others.  With its own one counted as well these
+    shapes were left to unsplit tiles ([N, K] 1491x3840x1808: 43 us, split two ways 37) or to the kernel of 64-row tiles ([K, N]
+    471x3328x4320: 38 and 34)."""
+    from pytorch_amd import _capi
+    workgroups = -(-M // rows) * -(-N // 128) * split
+    assert _capi.lib().mi355_weight_quant_matmul_workspace(M, N, K, 8, 0) == _capi.ZERO_AREA_BYTES + workgroups * rows * 128 * 4
