@@ -2,9 +2,9 @@
 // fragments from LDS and requests refills.  Tiles 256x256 (2 x 4 wavefronts of 128 x 64), 128x256 and 128x320 (2 x 4 of 64 x 64 / 80).
 //
 // A K step of 128 bytes is two parts.  The operand of which a wavefront needs fewer rows is read whole in the first part, the other one
-// half per part, so that a part is 20 to 32 MFMAs on fragments that fit beside the accumulators (64 registers; no spills, where
-// double-buffered fragments made the 256x256 tile spill 33).  A part is two intervals between barriers: fragments and refills, then
-// MFMAs.  Wavefronts w and w + 4 share a SIMD; 4 .. 7 run one interval behind 0 .. 3, so one of the two is always in its MFMAs.
+// half per part, so that a part is 16 to 32 MFMAs on one set of fragments beside the accumulators (64 registers; the loop has no scratch
+// access.  The kernels of the 256x256 tile spill 35 to 42 registers, one store in front of the loop and the rest in the general epilogue, which
+// takes what the epilogues with their parameters in LDS do not).  A part is two intervals between barriers: fragments and refills, then MFMAs.  Wavefronts w and w + 4 share a SIMD; 4 .. 7 run one interval behind 0 .. 3, so one of the two is always in its MFMAs.
 //
 // Slots.  Whoever reads a slot is done (lgkmcnt 0) before the barrier that ends the interval, and the wavefronts one interval behind
 // before the next one; a slot is refilled two intervals after the leading wavefronts read it, i.e. never before the others are done.
@@ -13,11 +13,11 @@
 // number of loads that may be outstanding at a wait is a constant.
 //
 // What bounds it: power.  At 4096x4096x4096 the loop runs at 2191 clocks a step where the MFMAs alone are 2048, but with operands as
-// quantisation leaves them the card holds 1.6 GHz there (2.25 GHz with zeros); v_mfma_i32_32x32x32_i8 in the same loop needs fewer
-// clocks (2134) and is slower (1.43 GHz, 62.5 us instead of 57).  Microseconds before (refills and fragment reads interleaved with the
-// MFMAs by scheduling groups) and now: 4096x4096x4096 62.0 -> 59.4, 2048x14336x4096 split two ways 114.3 -> 111.2 (256x256),
-// and with the epilogue that has its parameters in LDS 53.0 and 102; 777x11008x4096 split two ways 54.8 -> 45.3 (128x256, with that
-// epilogue).  On 256x192 and 256x224 it is level with quant_matmul_wide.h.
+// quantisation leaves them the card holds 1.65 GHz there and 2.2 with zeros, for the same cycles (55.6 and 42.4 us back to back);
+// v_mfma_i32_32x32x32_i8 in the same loop needs fewer clocks (2134) and is 10 % slower (1.43 GHz).  Microseconds before (refills and
+// fragment reads interleaved with the MFMAs by scheduling groups, general epilogue), with this loop and that epilogue, and with the one that has its
+// parameters in LDS, on one box: 4096x4096x4096 57.3, 55.5, 52.9; 2048x14336x4096 split two ways 110.9, 105.6, 102.7 (256x256).
+// 777x11008x4096 split two ways 54.8 -> 45.3 (128x256, with that epilogue).  On 256x192 and 256x224 it is level with quant_matmul_wide.h.
 #pragma once
 #include "common.h"
 #include <type_traits>

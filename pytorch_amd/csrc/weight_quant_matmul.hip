@@ -790,8 +790,8 @@ bool repack_applies(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t
     return M >= kRepackRows && N % 8 == 0 && K % 128 == 0 &&
            make_wq_gemm4_plan(M, N, K, 4, group_size, repack_pitch_words(N), ldx, x, nullptr, nullptr, nullptr).ok;
 }
-// int8 [K, N] above 32 rows: the tiles of up to 256 rows where their estimate is below the one of 64-row tiles.  Over 60 shapes of
-// 33 .. 2048 rows the rule takes 39 of them, none slower than before: 384x4096x11008 94 -> 65 us, 59x1280x2400 15.7 -> 11.2; it leaves
+// int8 [K, N] above 32 rows: the tiles of up to 256 rows where their estimate is below the one of 64-row tiles.  Over 90 shapes of
+// 33 .. 2048 rows the rule takes 55, none slower than before and 0.87 of the time on average over the 90: 384x4096x11008 94 -> 65 us, 59x1280x2400 15.7 -> 11.2; it leaves
 // 1024x4096x4096 (52, here 58) and 461x2688x4672 (32, here 37), where 64-row tiles fill one round.
 bool takes_tall_tiles(const WqKmGemmPlan &kn, const WqGemm4Plan &g8)
 {
