@@ -1226,7 +1226,7 @@ int run_quant_matmul(const int8_t *a, const int8_t *b, const float *pertoken_sca
         // generic kernel (870x13360x7456: 0.13 ms and tens of ms)
         if (K % BK == 0) return !ws || workspace_bytes < pl.workspace() ? MI355_ERR_WORKSPACE : MI355_ERR_ALIGNMENT;
         const QmmPlan bare = make_qmm_plan(M, N, K, ldb_k, ldb_n, zero_area, scratch_cap, false);
-        if (bare.workspace() == 0) pl = bare;
+        if (bare.workspace() == 0 || (ws && workspace_bytes >= bare.workspace() && aligned(ws, 16))) pl = bare;
         else tiled = false;
     }
     if (tiled && ldb_k != 1) {

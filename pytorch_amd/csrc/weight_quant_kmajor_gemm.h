@@ -16,11 +16,12 @@ struct WqKmGemmPlan {
 };
 
 // `n_major`: the weight is [K, N].  `ldw`: bytes between its columns, of a [K, N] weight between its rows.  Null pointers (the workspace query) count as aligned.  `room`: the workspace that a split of K
-// may use.
+// may use.  `own_chunk_counts`: the estimate of a split as if the collecting workgroup read its own chunk back.
 __attribute__((visibility("hidden"))) WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw,
                                                                             int64_t ldx, const void *x, const void *w,
                                                                             const void *scale, const void *offset,
-                                                                            size_t room = ~(size_t)0, bool n_major = false);
+                                                                            size_t room = ~(size_t)0, bool n_major = false,
+                                                                            bool own_chunk_counts = false);
 
 // Whether the kernel takes such a problem.  Strides that it takes change the plan only where they rule out tall tiles, and its request then
 // never grows (200,000 shapes, activation rows 2^22 and more apart).

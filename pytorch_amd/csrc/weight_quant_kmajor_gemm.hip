@@ -406,7 +406,8 @@ bool wq_kmajor_gemm_accepts(int64_t M, int64_t N, int64_t K, int64_t group_size,
 }
 
 WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t ldw, int64_t ldx, const void *x,
-                                      const void *w, const void *scale, const void *offset, size_t room, bool n_major)
+                                      const void *w, const void *scale, const void *offset, size_t room, bool n_major,
+                                      bool own_chunk_counts)
 {
     WqKmGemmPlan pl{};
     pl.n_major = n_major;
@@ -441,7 +442,7 @@ WqKmGemmPlan make_wq_kmajor_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t g
             double us = (double)((wgs + slots - 1) / slots * ((stages + S - 1) / S)) * kStageUs[wtm == 1 && wgs <= kNumCU ? 0 : wtm];
             const double mem = (double)K * (double)N / kWeightBytesPerUs, l2 = (double)tiles * (128 * wtm + kBN) * (double)K / kL2BytesPerUs;
             us = kBaseUs + (us > mem ? us > l2 ? us : l2 : mem > l2 ? mem : l2);
-            if (S > 1) us += kExchangeUs + (double)(wgs * chunk_bytes) * 2.0 / kExchangeBytesPerUs + (double)((wtm > 1 ? S - 1 : S) * chunk_bytes) / kCollectorBytesPerUs;
+            if (S > 1) us += kExchangeUs + (double)(wgs * chunk_bytes) * 2.0 / kExchangeBytesPerUs + (double)((wtm > 1 && !own_chunk_counts ? S - 1 : S) * chunk_bytes) / kCollectorBytesPerUs;
             if (us < best) {
                 best = us;
                 pl.us = us;

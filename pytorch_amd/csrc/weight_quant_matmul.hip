@@ -1022,9 +1022,16 @@ extern "C" int mi355_weight_quant_matmul(const void *x_bf16, int act_dtype, cons
         }
         WqKmGemmPlan kg = make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16);
         if (kg.ok && out_ok) {
-            const int st = fit_workspace(kg, kg.counter_bytes + kg.partial_bytes, [&]() {
-                return make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16, room);
-            });
+            const auto plan_kg = [&](size_t within, bool own_chunk_counts) {
+                return make_wq_kmajor_gemm_plan(M, N, K, group_size, ldw_n, ldx, x_bf16, w, scale_bf16, offset_bf16, within, false, own_chunk_counts);
+            };
+            const size_t usable = aligned(workspace, 16) ? room : 0;
+            if (kg.S > 1 && usable < kg.counter_bytes + kg.partial_bytes) {
+                // a split that pays only because its own chunk is not read back is no reason to refuse a caller
+                const WqKmGemmPlan strict = plan_kg(~(size_t)0, true);
+                if (usable >= strict.counter_bytes + strict.partial_bytes) kg = plan_kg(usable, false);
+            }
+            const int st = fit_workspace(kg, kg.counter_bytes + kg.partial_bytes, [&]() { return plan_kg(room, false); });
             if (st != MI355_OK) return st;
         }
         if (kg.ok && out_ok)

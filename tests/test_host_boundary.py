@@ -653,3 +653,18 @@ def test_weight_quant_split_counts_the_chunks_that_are_read(M, K, N, rows, split
     from pytorch_amd import _capi
     workgroups = -(-M // rows) * -(-N // 128) * split
     assert _capi.lib().mi355_weight_quant_matmul_workspace(M, N, K, 8, 0) == _capi.ZERO_AREA_BYTES + workgroups * rows * 128 * 4
+
+
+@pytest.mark.parametrize("M,K,N,workspace_bytes", [(1491, 3840, 1808, 0), (1095, 3456, 2400, 0), (1438, 4096, 1536, 35667968), (200, 4096, 1024, None)])
+def test_weight_quant_kmajor_tiles_without_their_split(M, K, N, workspace_bytes):
+    """int8 [N, K]: a split that pays only since the collecting workgroup keeps its own chunk in registers is given up by callers without the
+    workspace for it (or with a misaligned one), or with the one of the split that they ran before; one that pays in any case is still refused."""
+    from pytorch_amd import _capi
+    if workspace_bytes is None:
+        assert _weight_quant_status(M, N, K, 8, 0, K, 1, K, 0) == _WORKSPACE_ERROR
+    else:
+        assert _weight_quant_status(M, N, K, 8, 0, K, 1, K, workspace_bytes) == _LAUNCH_ERROR
+    assert _weight_quant_status(M, N, K, 8, 0, K, 1, K) == _LAUNCH_ERROR
+    p = [i << 32 for i in range(1, 8)]
+    misaligned = _capi.lib().mi355_weight_quant_matmul(p[0], 0, p[1], 8, p[2], p[3], p[4], p[5], M, N, K, 0, 0, 1, K, 1, K, N, p[6] + 8, 1 << 30, None)
+    assert misaligned == (_LAUNCH_ERROR if workspace_bytes == 0 else _ALIGNMENT_ERROR)
