@@ -525,10 +525,11 @@ def test_quant_matmul_alternating_loop_epilogues(capi, golden, tile, M, K, N, sp
             capi.set_tuning(k, 0)
 
 
-def test_quant_matmul_256x256_epilogues_cost_the_same(capi):
+def test_quant_matmul_256x256_epilogues_cost_alike(capi):
     """The 256x256 tile has an epilogue with its parameters in LDS for every kind of bias and scale.  4096x128x4096, one K step, is little
-    else than the epilogue: 10.4 us in a recorded graph with it and 12.7 to 13.8 with the general one, 22 to 32 % more; kinds that all have it
-    differ by 2 %, so 8 % tells the two apart.  (Everything else about these outputs is the test above.)"""
+    else than the epilogue: 10.2 us in a recorded graph for bf16.  The other 16-bit kinds take 0.99 to 1.02 of that and 1.22 to 1.26 with the
+    general epilogue; int8, whose rows leave the LDS after a whole half of the tile and not after 16 rows, 1.08 to 1.10 and 1.31 to 1.33 (nine
+    runs each).  The bounds lie half way.  (Everything else about these outputs is the test above.)"""
     M, K, N = 4096, 128, 4096
     d = workloads.quant_matmul_inputs(seed=1, M=M, K=K, N=N, weight_nk=True, bias=True)
     x1, x2, sc, ps = (d[k].cuda() for k in ("x1", "x2", "scale", "pertoken_scale"))
@@ -558,7 +559,8 @@ def test_quant_matmul_256x256_epilogues_cost_the_same(capi):
             torch.cuda.synchronize()
             if rep:
                 best[name] = min(best[name], start.elapsed_time(end))
-    assert max(best.values()) < 1.08 * best["bf16"], best
+    for name in calls:
+        assert best[name] < (1.20 if name == "int8" else 1.11) * best["bf16"], (name, best)
 
 
 def test_quant_matmul_ragged_k_without_a_workspace(capi):
